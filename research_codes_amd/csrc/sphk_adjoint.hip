@@ -151,10 +151,24 @@ __global__ __launch_bounds__(kWave) void gravity_vjp_kernel(
 // i-side derivative of its pair terms and the j-side derivative of its
 // neighbours' pair terms: one register accumulator per lane, no atomics,
 // and a fixed summation order (bitwise reproducible).
+//
+// Both are derivatives of one scalar, the pair's terms in P's and in Q's
+// outputs weighted by their cotangents, with respect to P's inputs.  The
+// factors the two orders share (distance, F_P + F_Q, v_sig, 1/(rho_P +
+// rho_Q), ...) are symmetric or change sign, so the scalar is
+//   L = -5 C1 [ (F_P + F_Q) (-P_t (A.d)/2 + r B/2 + 2 rhi du D) + E (G.d)/2 ]
+// with A = m_Q abar_P - m_P abar_Q (G the same of the accg cotangents), B and
+// D the mass-weighted du/dt and diffu cotangents, and is reversed once per
+// pair.  Bound by FP64 issue: an IEEE FP64 square root measures 86 cycles per
+// wave and a division 59 against 4 for an FMA, so 1/r, 1/(rho_P + rho_Q) and
+// the signal-speed root come from Newton-refined v_rsq / v_rcp.  2x10^5
+// particles, 3.5x10^7 entries: 0.97 ms with two one-sided reverses per pair
+// and IEEE roots and divisions, 0.56 ms so.  205 VGPRs, 2 waves per SIMD;
+// held to 168 (3 waves) it spills and takes 2.8 ms, and tiles of 32 or 48
+// records measure 0.58 and 0.57 ms.
 // ---------------------------------------------------------------------------
 struct HP {           // one particle's hydro inputs (hinv^5 derived)
     double x, y, z, vx, vy, vz, h, h5, p, pc, b, d, c, al, au, u, et, m;
-    int32_t id;
 };
 struct HCot {         // cotangents of that particle's functor outputs
     double ax, ay, az, ud, df, gx, gy, gz;
@@ -166,7 +180,7 @@ __device__ __forceinline__ HP load_hp(const sphk_hydro_src &s, int k)
     const double h = s.hinv[k];
     const double h2 = h * h;
     return HP{s.x[k], s.y[k], s.z[k], s.vx[k], s.vy[k], s.vz[k], h, h2 * h2 * h, s.pres[k], s.presc[k],
-              s.bswt[k], s.dens[k], s.vsnd[k], s.alph[k], s.alphu[k], s.thrm[k], s.eta[k], s.m[k], s.id[k]};
+              s.bswt[k], s.dens[k], s.vsnd[k], s.alph[k], s.alphu[k], s.thrm[k], s.eta[k], s.m[k]};
 }
 
 __device__ __forceinline__ HCot load_cot(const sphk_hydro_out &c, int k)
@@ -174,155 +188,118 @@ __device__ __forceinline__ HCot load_cot(const sphk_hydro_out &c, int k)
     return HCot{c.ax[k], c.ay[k], c.az[k], c.udot[k], c.diffu[k], c.gx[k], c.gy[k], c.gz[k]};
 }
 
-// Reverse of the pair term of particle a (the functor's i) with b (its j),
-// hdr_hydro.hpp:352-399 in the closed form of the forward kernel, weighted
-// by a's output cotangents ca.  ASIDE: add the derivative with respect to
-// a's inputs to g, else with respect to b's.
-template <bool ASIDE>
-__device__ __forceinline__ void hydro_pair_vjp(const HP &a, const HP &b, const HCot &ca, double (&g)[kHG])
+// Reverse of the pair (P, Q), hdr_hydro.hpp:352-399 in the closed form of the
+// forward kernel: adds to g the derivative, with respect to P's inputs, of
+// P's outputs weighted by cp plus Q's outputs weighted by cq.
+__device__ __forceinline__ void hydro_pair_vjp(const HP &P, const HP &Q, const HCot &cp, const HCot &cq,
+                                               double (&g)[kHG])
 {
-    if (a.id == b.id) return;
-    constexpr double k5 = -5. * kCeff1;
-    const double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
-    const double dvx = a.vx - b.vx, dvy = a.vy - b.vy, dvz = a.vz - b.vz;
+    constexpr double K = -5. * kCeff1;
+    const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
     const double r2 = dx * dx + dy * dy + dz * dz;
-    const double ri = 1. / __builtin_sqrt(r2);
+    const double ri = rsqrt_f64(r2);
     const double r = r2 * ri;
-    const double qa = r * a.h, qb = r * b.h;
-    const double ta = qa < 1. ? 1. - qa : 0., tb = qb < 1. ? 1. - qb : 0.;
-    if (ta == 0. && tb == 0.) return;   // beyond both supports: value and derivatives vanish
-    const double Fa = a.h5 * (ta * ta * ta), Fb = b.h5 * (tb * tb * tb);
-    const double mk = k5 * b.m;
-    const double kri = mk * (Fa + Fb);
-    const double ka = kri * r;
-    const double rv = dx * dvx + dy * dvy + dz * dvz;
-    const double w = rv * ri;
+    const double qp = r * P.h, qq = r * Q.h;
+    const double tp = qp < 1. ? 1. - qp : 0., tq = qq < 1. ? 1. - qq : 0.;
+    if (tp == 0. && tq == 0.) return;   // beyond both supports: value and derivatives vanish
+    const double tp2 = tp * tp, tq2 = tq * tq;
+    const double Fp = P.h5 * (tp2 * tp), Fq = Q.h5 * (tq2 * tq);
+    const double KF = K * (Fp + Fq);
+    const double dvx = P.vx - Q.vx, dvy = P.vy - Q.vy, dvz = P.vz - Q.vz;
+    const double w = (dx * dvx + dy * dvy + dz * dvz) * ri;
     const double w0 = w < 0. ? w : 0.;
-    const double vs = a.c + b.c - 3. * w0;
-    const double rhi = 1. / (a.d + b.d);
-    const double bs = a.b + b.b, as = a.al + b.al;
-    const double av0 = bs * as * vs * w0;
-    const double Pt = a.pc + b.pc - 0.5 * av0 * rhi;
-    const double tpair = Pt * kri;
-    const double dP = a.p - b.p;
+    const double vs = P.c + Q.c - 3. * w0;
+    const double rhi = rcp_f64(P.d + Q.d);
+    const double bs = P.b + Q.b, as = P.al + Q.al, aus = P.au + Q.au;
+    const double bsas = bs * as;
+    const double vsw = vs * w0;
+    const double av0 = bsas * vsw;
+    const double Pt = P.pc + Q.pc - 0.5 * av0 * rhi;
+    const double dP = P.p - Q.p;
     const double vsu2 = __builtin_fabs(dP) * rhi * 2.;
-    const double vsu = vsu2 > 0. ? __builtin_sqrt(vsu2) : 0.;
-    const double du = a.u - b.u;
-    const double aus = a.au + b.au;
-    const double Y = 0.25 * av0 * w0 - aus * vsu * du;
-    const double X = a.pc * w - rhi * Y;
-    const double E = a.et * Fa + b.et * Fb;
-    const double dg = mk * E;
-    // outputs of a: ax = -0.5 sum tpair d, udot = 0.5 sum ka X,
-    // diffu = 2 sum rhi du kri, g = 0.5 sum dg d
-    const double Ad = ca.ax * dx + ca.ay * dy + ca.az * dz;
-    const double Gd = ca.gx * dx + ca.gy * dy + ca.gz * dz;
-    double d_b[3] = {-0.5 * tpair * ca.ax + 0.5 * dg * ca.gx, -0.5 * tpair * ca.ay + 0.5 * dg * ca.gy,
-                     -0.5 * tpair * ca.az + 0.5 * dg * ca.gz};
-    const double tp_b = -0.5 * Ad;
-    const double ka_b = 0.5 * ca.ud * X;
-    const double X_b = 0.5 * ca.ud * ka;
-    double kri_b = 2. * ca.df * rhi * du;
-    double rhi_b = 2. * ca.df * du * kri;
-    double du_b = 2. * ca.df * rhi * kri;
-    const double dg_b = 0.5 * Gd;
-    // X = a.pc w - rhi Y
-    double apc_b = X_b * w;
-    double w_b = X_b * a.pc;
-    rhi_b -= X_b * Y;
-    const double Y_b = -X_b * rhi;
-    // Y = av0 w0 / 4 - aus vsu du
-    double av0_b = 0.25 * w0 * Y_b;
-    double w0_b = 0.25 * av0 * Y_b;
-    const double aus_b = -vsu * du * Y_b;
-    const double vsu_b = -aus * du * Y_b;
-    du_b -= aus * vsu * Y_b;
-    // tpair = Pt kri, Pt = a.pc + b.pc - av0 rhi / 2
-    const double Pt_b = tp_b * kri;
-    kri_b += tp_b * Pt;
-    apc_b += Pt_b;
-    const double bpc_b = Pt_b;
-    av0_b -= 0.5 * rhi * Pt_b;
-    rhi_b -= 0.5 * av0 * Pt_b;
-    // ka = kri r
-    kri_b += ka_b * r;
-    double r_b = ka_b * kri;
-    // dg = mk (a.et Fa + b.et Fb), kri = mk (Fa + Fb)
-    const double E_b = dg_b * mk;
-    const double aet_b = E_b * Fa, bet_b = E_b * Fb;
-    const double Fa_b = E_b * a.et + kri_b * mk;
-    const double Fb_b = E_b * b.et + kri_b * mk;
-    // av0 = bs as vs w0
-    const double bs_b = av0_b * as * vs * w0;
-    const double as_b = av0_b * bs * vs * w0;
-    const double vs_b = av0_b * bs * as * w0;
-    w0_b += av0_b * bs * as * vs;
-    // vs = a.c + b.c - 3 w0; w0 = min(w, 0)
-    w0_b -= 3. * vs_b;
+    const double vsui = vsu2 > 0. ? rsqrt_f64(vsu2) : 0.;   // 1 / vsu
+    const double vsu = vsu2 * vsui;
+    const double du = P.u - Q.u;
+    // the cotangents of the two orders of the pair, combined
+    const double Ax = Q.m * cp.ax - P.m * cq.ax, Ay = Q.m * cp.ay - P.m * cq.ay, Az = Q.m * cp.az - P.m * cq.az;
+    const double Gx = Q.m * cp.gx - P.m * cq.gx, Gy = Q.m * cp.gy - P.m * cq.gy, Gz = Q.m * cp.gz - P.m * cq.gz;
+    const double D = Q.m * cp.df - P.m * cq.df;
+    const double up = Q.m * cp.ud, uq = P.m * cq.ud;
+    const double Us = up + uq, Ud = up - uq;
+    const double Ad = Ax * dx + Ay * dy + Az * dz;
+    const double hGd = 0.5 * (Gx * dx + Gy * dy + Gz * dz);
+    const double vdu = vsu * du * Ud;
+    const double Pw = up * P.pc + uq * Q.pc;
+    const double T = 0.25 * av0 * w0 * Us - aus * vdu;
+    const double B = w * Pw - rhi * T;
+    const double M1 = -0.5 * Pt * Ad + 0.5 * r * B + 2. * rhi * du * D;
+    // F_P, F_Q and eta
+    const double KG = K * hGd;
+    const double Fs_b = K * M1;
+    const double Fp_b = Fs_b + KG * P.et, Fq_b = Fs_b + KG * Q.et;
+    const double E = P.et * Fp + Q.et * Fq;
+    const double Gd_b = 0.5 * K * E, Ad_b = -0.5 * KF * Pt;
+    double dbx = Ad_b * Ax + Gd_b * Gx, dby = Ad_b * Ay + Gd_b * Gy, dbz = Ad_b * Az + Gd_b * Gz;
+    // P_t, B and the conduction term
+    const double Pt_b = -0.5 * KF * Ad;
+    double r_b = 0.5 * KF * B;
+    const double B_b = 0.5 * KF * r;
+    double rhi_b = 2. * KF * du * D - B_b * T - 0.5 * av0 * Pt_b;
+    double du_b = 2. * KF * rhi * D;
+    const double T_b = -B_b * rhi;
+    double w_b = B_b * Pw;
+    const double pc_b = B_b * w * up + Pt_b;
+    const double av0_b = 0.25 * w0 * Us * T_b - 0.5 * rhi * Pt_b;
+    double w0_b = 0.25 * av0 * Us * T_b;
+    const double aus_b = -vdu * T_b;
+    const double vsu_b = -aus * du * Ud * T_b;
+    du_b -= aus * vsu * Ud * T_b;
+    // av0 = bs as vs w0, vs = c_P + c_Q - 3 w0, w0 = min(w, 0)
+    const double avw = av0_b * vsw;
+    const double bs_b = as * avw, as_b = bs * avw;
+    const double abb = av0_b * bsas;
+    const double vs_b = abb * w0;
+    w0_b += abb * vs - 3. * vs_b;
     if (w < 0.) w_b += w0_b;
-    // vsu = sqrt(|dP| rhi 2)
-    const double vsu2_b = vsu2 > 0. ? vsu_b * 0.5 / vsu : 0.;
-    const double dP_b = vsu2_b * 2. * rhi * (dP > 0. ? 1. : (dP < 0. ? -1. : 0.));
-    rhi_b += vsu2_b * 2. * __builtin_fabs(dP);
-    // rhi = 1 / (a.d + b.d)
-    const double dd_b = -rhi_b * rhi * rhi;
-    // w = rv ri, rv = d . dv
+    // vsu = sqrt(2 |dP| rhi), rhi = 1 / (rho_P + rho_Q)
+    const double vsu2_b = vsu_b * vsui;   // twice the derivative: the factors 2 and 1/2 cancel below
+    const double p_b = vsu2_b * rhi * (dP > 0. ? 1. : (dP < 0. ? -1. : 0.));
+    rhi_b += vsu2_b * __builtin_fabs(dP);
+    const double d_b = -rhi_b * rhi * rhi;
+    // w = (d . dv) / r
     const double rv_b = w_b * ri;
-    double ri_b = w_b * rv;
-    double dv_b[3] = {rv_b * dx, rv_b * dy, rv_b * dz};
-    d_b[0] += rv_b * dvx;
-    d_b[1] += rv_b * dvy;
-    d_b[2] += rv_b * dvz;
-    // F = h^5 t^3, t = 1 - r h (inside the support)
-    const double ta_b = Fa_b * 3. * a.h5 * ta * ta, tb_b = Fb_b * 3. * b.h5 * tb * tb;
-    double ah_b = Fa_b * 5. * (a.h * a.h) * (a.h * a.h) * (ta * ta * ta) - ta_b * r;
-    double bh_b = Fb_b * 5. * (b.h * b.h) * (b.h * b.h) * (tb * tb * tb) - tb_b * r;
-    r_b -= ta_b * a.h + tb_b * b.h;
-    // ri = 1 / r, r = |d|
-    r_b -= ri_b * ri * ri;
-    d_b[0] += r_b * ri * dx;
-    d_b[1] += r_b * ri * dy;
-    d_b[2] += r_b * ri * dz;
-    if (ASIDE) {
-        g[0] += d_b[0];
-        g[1] += d_b[1];
-        g[2] += d_b[2];
-        g[3] += dv_b[0];
-        g[4] += dv_b[1];
-        g[5] += dv_b[2];
-        g[6] += ah_b;
-        g[7] += dP_b;
-        g[8] += apc_b;
-        g[9] += bs_b;
-        g[10] += dd_b;
-        g[11] += vs_b;
-        g[12] += as_b;
-        g[13] += aus_b;
-        g[14] += du_b;
-        g[15] += aet_b;
-    } else {
-        g[0] -= d_b[0];
-        g[1] -= d_b[1];
-        g[2] -= d_b[2];
-        g[3] -= dv_b[0];
-        g[4] -= dv_b[1];
-        g[5] -= dv_b[2];
-        g[6] += bh_b;
-        g[7] -= dP_b;
-        g[8] += bpc_b;
-        g[9] += bs_b;
-        g[10] += dd_b;
-        g[11] += vs_b;
-        g[12] += as_b;
-        g[13] += aus_b;
-        g[14] -= du_b;
-        g[15] += bet_b;
-    }
+    dbx += rv_b * dvx;
+    dby += rv_b * dvy;
+    dbz += rv_b * dvz;
+    r_b -= rv_b * w;
+    // F = h^5 t^3, t = 1 - r h inside the support
+    const double tp_b = Fp_b * 3. * P.h5 * tp2, tq_b = Fq_b * 3. * Q.h5 * tq2;
+    const double ph2 = P.h * P.h;
+    const double h_b = Fp_b * 5. * (ph2 * ph2) * (tp2 * tp) - tp_b * r;
+    r_b -= tp_b * P.h + tq_b * Q.h;
+    const double f = r_b * ri;
+    g[0] += dbx + f * dx;
+    g[1] += dby + f * dy;
+    g[2] += dbz + f * dz;
+    g[3] += rv_b * dx;
+    g[4] += rv_b * dy;
+    g[5] += rv_b * dz;
+    g[6] += h_b;
+    g[7] += p_b;
+    g[8] += pc_b;
+    g[9] += bs_b;
+    g[10] += d_b;
+    g[11] += vs_b;
+    g[12] += as_b;
+    g[13] += aus_b;
+    g[14] += du_b;
+    g[15] += KG * Fp;
 }
 
-struct HRecV {        // a staged j-record: inputs and its output cotangents
+struct HRecV {        // a staged j-record: inputs, its output cotangents, id
     HP p;
     HCot c;
+    int32_t id;
 };
 
 __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int32_t *__restrict__ i_off,
@@ -344,6 +321,7 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
         const int i = c0 + il;
         const HP P = load_hp(src, i);
         const HCot cp = load_cot(cot, i);
+        const int32_t id = src.id[i];
         double g[kHG];
 #pragma unroll
         for (int q = 0; q < kHG; q++) g[q] = 0.;
@@ -352,16 +330,12 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
             __syncthreads();
             if (lane < nt) {
                 const int j = j_idx ? j_idx[t0 + lane] : t0 + lane;
-                sp[lane] = HRecV{load_hp(src, j), load_cot(cot, j)};
-            } else {   // inert: far away, massless, no cotangent
-                sp[lane] = HRecV{HP{1e15, 1e15, 1e15, 0., 0., 0., 1., 1., 0., 0., 0., 1., 0., 0., 0., 0., 0., 0., -1},
-                                 HCot{0., 0., 0., 0., 0., 0., 0., 0.}};
+                sp[lane] = HRecV{load_hp(src, j), load_cot(cot, j), src.id[j]};
             }
             __syncthreads();
             for (int k = slice; k < nt; k += S) {
                 const HRecV &Q = sp[k];
-                hydro_pair_vjp<true>(P, Q.p, cp, g);
-                hydro_pair_vjp<false>(Q.p, P, Q.c, g);
+                if (Q.id != id) hydro_pair_vjp(P, Q.p, cp, Q.c, g);
             }
         }
         // per i: the S slices' partials in slice order, then one plain add
