@@ -46,6 +46,16 @@ int sphk_gravity_vjp_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const 
                          const double *ebar, double *gx, double *gy, double *gz, double *nx, double *ny,
                          double *nz, void *stream);
 
+/* The same with the three components of a cotangent side by side: g3[N][3]
+ * for the particles, n3[n_node][3] for the nodes (may be NULL when there is
+ * no SPJ list).  The components of one record then leave in one memory
+ * request: faster, as the atomics bound the kernel. */
+int sphk_gravity_vjp_packed_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                                const int32_t *j_idx, sphk_grav_src pj, const int32_t *s_off,
+                                const int32_t *s_idx, sphk_grav_src ps, sphk_grav_src pi, double e2,
+                                const double *abx, const double *aby, const double *abz, const double *pbar,
+                                const double *ebar, double *g3, double *n3, void *stream);
+
 /* Cotangents of the density functor's outputs, and of its differentiable
  * inputs (positions, velocities, the starting smoothing length ksr). */
 typedef struct {

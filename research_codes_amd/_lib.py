@@ -154,6 +154,8 @@ SIGNATURES.update({
     # sphk_adjoint.h
     "sphk_gravity_vjp_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, GravSrc, _P, _P, GravSrc, GravSrc, C.c_double]
                              + [_P] * 11 + [_P]),
+    "sphk_gravity_vjp_packed_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, GravSrc, _P, _P, GravSrc, GravSrc, C.c_double]
+                                    + [_P] * 7 + [_P]),
     "sphk_dtree_spread_dev": (C.c_int, [_P] + [_P] * 7),
     "sphk_hydro_vjp_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, HydroSrc, HydroOut, HydroGrad, _P]),
     "sphk_density_vjp_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, DensSrc, DensCot, DensGrad, _P]),

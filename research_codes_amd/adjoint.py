@@ -2,7 +2,7 @@
 
 Forward: the gravity functor (sphk_gravity_dev, uniform softening) on lists
 from the device tree.  Backward: the hand-written vector-Jacobian product
-(sphk_gravity_vjp_dev, include/sphk_adjoint.h) followed by the tree spread of
+(sphk_gravity_vjp_packed_dev, include/sphk_adjoint.h) followed by the tree spread of
 the node cotangents to the particles (sphk_dtree_spread_dev).  The tree and
 lists are held fixed between forward and backward, as a tree code's
 derivative is (piecewise constant in the positions).
@@ -74,17 +74,18 @@ class TreeGravity:
     def _backward(self, st, x, y, z, gax, gay, gaz, gpot, geta):
         w, mom, t = st.walks, st.mom, st.tree
         n = x.numel()
-        g = [torch.zeros(n, dtype=torch.float64, device=x.device) for _ in range(3)]
-        nb = [torch.zeros(t.n_node, dtype=torch.float64, device=x.device) for _ in range(3)]
+        g3 = torch.zeros(n, 3, dtype=torch.float64, device=x.device)
+        n3 = torch.zeros(t.n_node, 3, dtype=torch.float64, device=x.device)
         src = L.GravSrc(m=st.ms.data_ptr(), x=x.data_ptr(), y=y.data_ptr(), z=z.data_ptr(),
                         eps2=st.e2.data_ptr())
         ps = L.GravSrc(m=mom["m"].data_ptr(), x=mom["x"].data_ptr(), y=mom["y"].data_ptr(),
                        z=mom["z"].data_ptr(), eps2=mom["eps2"].data_ptr())
         cot = [c.contiguous() for c in (gax, gay, gaz, gpot, geta)]
-        check(lib().sphk_gravity_vjp_dev(self.ctx.handle, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                         w.j_idx.data_ptr(), src, w.s_off.data_ptr(), w.s_idx.data_ptr(), ps,
-                                         src, self.e2, *(c.data_ptr() for c in cot), *(a.data_ptr() for a in g),
-                                         *(a.data_ptr() for a in nb), _stream()), "sphk_gravity_vjp_dev")
+        check(lib().sphk_gravity_vjp_packed_dev(self.ctx.handle, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
+                                                w.j_idx.data_ptr(), src, w.s_off.data_ptr(), w.s_idx.data_ptr(),
+                                                ps, src, self.e2, *(c.data_ptr() for c in cot), g3.data_ptr(),
+                                                n3.data_ptr(), _stream()), "sphk_gravity_vjp_packed_dev")
+        g, nb = g3.t().contiguous(), n3.t().contiguous()
         check(lib().sphk_dtree_spread_dev(t._h, st.ms.data_ptr(), *(a.data_ptr() for a in nb),
                                           *(a.data_ptr() for a in g)), "sphk_dtree_spread_dev")
         return g

@@ -2,23 +2,19 @@
 // FP64: gravity (uniform softening, the reverse of gravity_pair_uniform),
 // hydro and density.
 //
-// Layout as the forward kernels: one wave per walk, S = floor(64/ni)
-// j-slices, 64-record LDS tiles.  The i-side cotangent of a lane stays in
-// registers and is combined across slices through LDS at the end of the
-// walk.  The j-side: gravity sweeps each tile a second time with one record
-// per lane; density collects it per tile in LDS (atomic adds); hydro needs
-// none (its symmetric lists hold both pair orders).  Either way it leaves
-// with one HBM atomic add per record and component.
+// One wave per walk.  Hydro and density: layout as the forward kernels, S =
+// floor(64/ni) j-slices, 64-record LDS tiles; the i-side cotangent of a lane
+// stays in registers and is combined across slices through LDS at the end of
+// the walk.  Gravity: one record per lane, the i-particles in LDS.  The
+// j-side: a lane's own in gravity, collected per tile in LDS (atomic adds) in
+// density, none in hydro (its symmetric lists hold both pair orders); it
+// leaves with one HBM atomic add per record and component.
 #include "sphk_adjoint.h"
 #include "sphk_device.hpp"
 #include "sphk_internal.hpp"
 
 namespace sphk {
 namespace {
-
-struct VRec {
-    double x, y, z, m;
-};
 
 __device__ __forceinline__ int xcd_walk_adj(int b, int n_walk)
 {
@@ -30,76 +26,111 @@ __device__ __forceinline__ int xcd_walk_adj(int b, int n_walk)
     return ((k / kC) * kX + x) * kC + k % kC;
 }
 
-// One i-particle's position and output cotangents, as the j-side sweep reads
-// them from LDS.
-struct VI {
+// Walk of workgroup b when each of the 8 XCDs takes one contiguous range.
+__device__ __forceinline__ int xcd_walk_range(int b, int n_walk)
+{
+    constexpr int kX = 8;
+    const int per = n_walk / kX;
+    return b < per * kX ? (b % kX) * per + b / kX : b;
+}
+
+// Gravity VJP: one record per lane.  A walk's i-particles are taken kVjpI at
+// a time; their positions and cotangents sit in LDS, read as broadcasts, and
+// each lane keeps its share of their position cotangents in registers (three
+// FP64 sums per i) over the whole list, so a pair is evaluated once for both
+// sides and the i-sides are combined across the wave once per chunk.  A lane
+// loads its next record before the j-side of the current one leaves with one
+// global FP64 atomic per component: memory operations complete in order, and
+// the next record must not wait behind the atomics.
+//
+// The atomics bound the kernel (2x10^5 particles, 2.5x10^7 records: 0.5 ms of
+// 1.2 without them), by requests, not by values: PACKED sends the three
+// components of a record from neighbouring lanes into one [n][3] array, and
+// each XCD takes one contiguous range of walks, so that fewer lines move
+// between the XCDs' caches (chunks of 8 to 1024 walks dealt in turn: 1.31 to
+// 1.39 ms, one range each 1.19).  More chunks of i-particles mean more
+// atomics: kVjpI = 8 / 12 / 16 take 2.4 / 1.9 / 1.6 ms unpacked, and 16 is
+// what leaves 3 waves per SIMD (160 VGPRs).  Before, every pair was evaluated
+// twice (a sweep per side, 64-record LDS tiles): 1.7 ms.
+constexpr int kVjpI = 16;
+
+struct alignas(16) VI {
     double x, y, z, ax, ay, az, pb, eb;
 };
 
-// Cotangent of record r's position from the pair (i, r): the reverse of the
-// uniform-softening pair term, m_r (T abar - pbar w^3 d + 3 ebar w^5 d) with
-// T = w^3 I - 3 w^5 d d^T and d = x_i - x_r; the i-side gets its negative.
-__device__ __forceinline__ void vjp_pair(const VI &I, const VRec &r, double e2, double &cx, double &cy,
-                                         double &cz)
+struct VRec {
+    double x, y, z, m;
+    int32_t j;
+};
+
+__device__ __forceinline__ VRec vjp_load(const sphk_grav_src &src, const int32_t *__restrict__ idx, int k, int ke)
 {
-    const double dx = I.x - r.x, dy = I.y - r.y, dz = I.z - r.z;
-    const double s = dx * dx + dy * dy + dz * dz + e2;
-    const double w = rsqrt_f64(s);
-    const double w3 = w * w * w;
-    const double w5 = w3 * w * w;
-    const double dot = dx * I.ax + dy * I.ay + dz * I.az;
-    // T abar = w3 abar - 3 w5 d (d . abar); then subtract pbar w3 d
-    // and add 3 ebar w5 d (the eta sum's gradient is -3 m w5 d)
-    const double f = 3. * w5 * (dot - I.eb) + I.pb * w3;
-    cx = r.m * (w3 * I.ax - f * dx);
-    cy = r.m * (w3 * I.ay - f * dy);
-    cz = r.m * (w3 * I.az - f * dz);
+    VRec r{1e15, 1e15, 1e15, 0., -1};   // past the end: far away and massless
+    if (k < ke) {
+        r.j = idx ? idx[k] : k;
+        r.x = src.x[r.j];
+        r.y = src.y[r.j];
+        r.z = src.z[r.j];
+        r.m = src.m[r.j];
+    }
+    return r;
 }
 
-// One list of a walk chunk, tile by tile, in two sweeps over the staged
-// records: the i-side (lane = (i, slice), register accumulators) and the
-// j-side (lane = record, looping over the chunk's i-particles in LDS, one
-// global atomic per record and component).  Every pair is evaluated twice;
-// summing the j-side in LDS instead needs atomics that the n_i lanes of a
-// slice issue to the same record at once.
-__device__ void vjp_list(int lane, int S, int slice, int ni, int kb, int ke, const int32_t *__restrict__ idx,
-                         const sphk_grav_src &src, const VI &I, const VI *sI, double e2, VRec *sp, int32_t *sj,
-                         double (&gi)[3], double *outx, double *outy, double *outz)
+// One list of a walk chunk (n i-particles in sI).  The cotangent of record
+// r's position from the pair (i, r) is the reverse of the uniform-softening
+// pair term, m_r (T abar - pbar w^3 d + 3 ebar w^5 d) with T = w^3 I - 3 w^5
+// d d^T and d = x_i - x_r; the i-side gets its negative.
+template <bool PACKED>
+__device__ __forceinline__ void vjp_list(int lane, int n, int kb, int ke, const int32_t *__restrict__ idx,
+                                         const sphk_grav_src &src, const VI *sI, double *sv, int32_t *sj, double e2,
+                                         double (&gi)[kVjpI][3], double *outx, double *outy, double *outz)
 {
-    for (int t0 = kb; t0 < ke; t0 += kTile) {
-        const int nt = min(kTile, ke - t0);
-        __syncthreads();
-        if (lane < nt) {
-            const int j = idx ? idx[t0 + lane] : t0 + lane;
-            sp[lane] = VRec{src.x[j], src.y[j], src.z[j], src.m[j]};
-            sj[lane] = j;
-        }
-        __syncthreads();
-        for (int k = slice; k < nt; k += S) {
-            double cx, cy, cz;
-            vjp_pair(I, sp[k], e2, cx, cy, cz);
-            gi[0] -= cx;
-            gi[1] -= cy;
-            gi[2] -= cz;
-        }
-        if (lane < nt) {
-            const VRec r = sp[lane];
-            double jx = 0., jy = 0., jz = 0.;
-            for (int q = 0; q < ni; q++) {
-                double cx, cy, cz;
-                vjp_pair(sI[q], r, e2, cx, cy, cz);
+    VRec nx = vjp_load(src, idx, kb + lane, ke);
+    for (int t0 = kb; t0 < ke; t0 += kWave) {
+        const VRec r = nx;
+        nx = vjp_load(src, idx, t0 + kWave + lane, ke);
+        double jx = 0., jy = 0., jz = 0.;
+        asm volatile("" ::: "memory");   // read sI per tile: hoisted, it would take every register
+#pragma unroll
+        for (int q = 0; q < kVjpI; q++) {
+            if (q < n) {
+                const VI I = sI[q];
+                const double dx = I.x - r.x, dy = I.y - r.y, dz = I.z - r.z;
+                const double w = rsqrt_f64(__builtin_fma(dz, dz, __builtin_fma(dy, dy, __builtin_fma(dx, dx, e2))));
+                const double w2 = w * w;
+                const double mw3 = r.m * (w2 * w);
+                const double dot = __builtin_fma(dx, I.ax, __builtin_fma(dy, I.ay, __builtin_fma(dz, I.az, -I.eb)));
+                const double f = mw3 * __builtin_fma(3. * w2, dot, I.pb);
+                const double cx = mw3 * I.ax - f * dx, cy = mw3 * I.ay - f * dy, cz = mw3 * I.az - f * dz;
                 jx += cx;
                 jy += cy;
                 jz += cz;
+                gi[q][0] -= cx;
+                gi[q][1] -= cy;
+                gi[q][2] -= cz;
             }
-            const int j = sj[lane];
-            atomicAdd(&outx[j], jx);
-            atomicAdd(&outy[j], jy);
-            atomicAdd(&outz[j], jz);
+        }
+        if (PACKED) {
+            __syncthreads();   // values of the previous tile sent
+            sj[lane] = r.j;
+            sv[3 * lane] = jx;
+            sv[3 * lane + 1] = jy;
+            sv[3 * lane + 2] = jz;
+            __syncthreads();
+            for (int t = 0; t < 3; t++) {
+                const int v = t * kWave + lane, q = v / 3;
+                const int j = sj[q];
+                if (j >= 0) atomicAdd(&outx[3 * (size_t)j + (v - 3 * q)], sv[v]);
+            }
+        } else if (r.j >= 0) {
+            atomicAdd(&outx[r.j], jx);
+            atomicAdd(&outy[r.j], jy);
+            atomicAdd(&outz[r.j], jz);
         }
     }
 }
 
+template <bool PACKED>
 __global__ __launch_bounds__(kWave) void gravity_vjp_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_grav_src pj, const int32_t *__restrict__ s_off,
@@ -108,36 +139,41 @@ __global__ __launch_bounds__(kWave) void gravity_vjp_kernel(
     const double *__restrict__ pbar, const double *__restrict__ ebar, double *gx, double *gy, double *gz,
     double *nx, double *ny, double *nz)
 {
-    __shared__ VRec sp[kTile];
-    __shared__ VI sI[kWave];
-    __shared__ int32_t sj[kTile];
-    __shared__ double red[3 * kWave];
+    __shared__ VI sI[kVjpI];
+    __shared__ double sv[PACKED ? 3 * kWave : 1];
+    __shared__ int32_t sj[PACKED ? kWave : 1];
     if ((int)blockIdx.x >= n_walk) return;
-    const int w = xcd_walk_adj(blockIdx.x, n_walk);
+    const int w = xcd_walk_range(blockIdx.x, n_walk);
     const int lane = threadIdx.x;
     const int ib = i_off[w], ie = i_off[w + 1];
-    for (int c0 = ib; c0 < ie; c0 += kWave) {
-        const int ni = min(kWave, ie - c0);
-        const int S = kWave / ni, il = lane % ni;
-        const int slice = lane / ni < S ? lane / ni : kTile;   // idle lanes sweep nothing
-        const int i = c0 + il;
-        const VI I{pi.x[i], pi.y[i], pi.z[i], abx[i], aby[i], abz[i], pbar[i], ebar ? ebar[i] : 0.};
+    for (int c0 = ib; c0 < ie; c0 += kVjpI) {
+        const int n = __builtin_amdgcn_readfirstlane(min(kVjpI, ie - c0));
         __syncthreads();   // sI of the previous chunk no longer read
-        if (lane < ni) sI[lane] = I;
-        double gi[3] = {0., 0., 0.};
-        vjp_list(lane, S, slice, ni, j_off[w], j_off[w + 1], j_idx, pj, I, sI, e2, sp, sj, gi, gx, gy, gz);
+        if (lane < n) {
+            const int i = c0 + lane;
+            sI[lane] = VI{pi.x[i], pi.y[i], pi.z[i], abx[i], aby[i], abz[i], pbar[i], ebar ? ebar[i] : 0.};
+        }
+        __syncthreads();
+        double gi[kVjpI][3];
+#pragma unroll
+        for (int q = 0; q < kVjpI; q++) gi[q][0] = gi[q][1] = gi[q][2] = 0.;
+        vjp_list<PACKED>(lane, n, j_off[w], j_off[w + 1], j_idx, pj, sI, sv, sj, e2, gi, gx, gy, gz);
         if (s_off)
-            vjp_list(lane, S, slice, ni, s_off[w], s_off[w + 1], s_idx, ps, I, sI, e2, sp, sj, gi, nx, ny, nz);
-        __syncthreads();
-        for (int q = 0; q < 3; q++) red[q * kWave + lane] = gi[q];
-        __syncthreads();
-        if (lane < ni) {
-            double s[3] = {0., 0., 0.};
-            for (int t = 0; t < S; t++)
-                for (int q = 0; q < 3; q++) s[q] += red[q * kWave + lane + ni * t];
-            atomicAdd(&gx[i], s[0]);
-            atomicAdd(&gy[i], s[1]);
-            atomicAdd(&gz[i], s[2]);
+            vjp_list<PACKED>(lane, n, s_off[w], s_off[w + 1], s_idx, ps, sI, sv, sj, e2, gi, nx, ny, nz);
+        // the wave's sums of each i, in a fixed order
+#pragma unroll
+        for (int q = 0; q < kVjpI; q++) {
+            if (q < n) {
+                double s[3] = {gi[q][0], gi[q][1], gi[q][2]};
+                for (int d = 1; d < kWave; d <<= 1)
+                    for (int c = 0; c < 3; c++) s[c] += __shfl_xor(s[c], d, kWave);
+                if (lane == 0) {
+                    const size_t i = (size_t)(c0 + q);
+                    atomicAdd(&gx[PACKED ? 3 * i : i], s[0]);
+                    atomicAdd(&(PACKED ? gx + 1 : gy)[PACKED ? 3 * i : i], s[1]);
+                    atomicAdd(&(PACKED ? gx + 2 : gz)[PACKED ? 3 * i : i], s[2]);
+                }
+            }
         }
     }
 }
@@ -679,6 +715,40 @@ extern "C" int sphk_hydro_vjp_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_of
     return SPHK_OK;
 }
 
+namespace {
+// Checks and launch of both gravity VJP entries; packed: gx and nx are [.][3]
+// arrays and the other four outputs are not used.
+int gravity_vjp(bool packed, sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                const int32_t *j_idx, const sphk_grav_src &pj, const int32_t *s_off, const int32_t *s_idx,
+                const sphk_grav_src &ps, const sphk_grav_src &pi, double e2, const double *abx, const double *aby,
+                const double *abz, const double *pbar, const double *ebar, double *gx, double *gy, double *gz,
+                double *nx, double *ny, double *nz, void *stream)
+{
+    using sphk::set_error;
+    if (!ctx) return set_error(SPHK_E_ARG, "gravity_vjp: null context");
+    if (n_walk < 0 || (n_walk > 0 && (!i_off || !j_off))) return set_error(SPHK_E_ARG, "gravity_vjp: bad walks");
+    if (n_walk == 0) return SPHK_OK;
+    if (!pi.x || !pi.y || !pi.z || !pj.m || !pj.x || !pj.y || !pj.z || !abx || !aby || !abz || !pbar || !gx ||
+        (!packed && (!gy || !gz)))
+        return set_error(SPHK_E_ARG, "gravity_vjp: null pointer");
+    if (s_off && (!ps.m || !ps.x || !ps.y || !ps.z || !nx || (!packed && (!ny || !nz))))
+        return set_error(SPHK_E_ARG, "gravity_vjp: null SPJ pointer");
+    if (!(e2 > 0.)) return set_error(SPHK_E_ARG, "gravity_vjp: softening must be positive");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (packed)
+        hipLaunchKernelGGL(sphk::gravity_vjp_kernel<true>, dim3(n_walk), dim3(sphk::kWave), 0, st, n_walk, i_off,
+                           j_off, j_idx, pj, s_off, s_idx, ps, pi, e2, abx, aby, abz, pbar, ebar, gx, gy, gz, nx, ny,
+                           nz);
+    else
+        hipLaunchKernelGGL(sphk::gravity_vjp_kernel<false>, dim3(n_walk), dim3(sphk::kWave), 0, st, n_walk, i_off,
+                           j_off, j_idx, pj, s_off, s_idx, ps, pi, e2, abx, aby, abz, pbar, ebar, gx, gy, gz, nx, ny,
+                           nz);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(SPHK_E_DEVICE, "gravity_vjp: %s", hipGetErrorString(e));
+    return SPHK_OK;
+}
+}  // namespace
+
 extern "C" int sphk_gravity_vjp_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
                                     const int32_t *j_idx, sphk_grav_src pj, const int32_t *s_off,
                                     const int32_t *s_idx, sphk_grav_src ps, sphk_grav_src pi, double e2,
@@ -686,20 +756,17 @@ extern "C" int sphk_gravity_vjp_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_
                                     const double *pbar, const double *ebar, double *gx, double *gy,
                                     double *gz, double *nx, double *ny, double *nz, void *stream)
 {
-    using sphk::set_error;
-    if (!ctx) return set_error(SPHK_E_ARG, "gravity_vjp: null context");
-    if (n_walk < 0 || (n_walk > 0 && (!i_off || !j_off))) return set_error(SPHK_E_ARG, "gravity_vjp: bad walks");
-    if (n_walk == 0) return SPHK_OK;
-    if (!pi.x || !pi.y || !pi.z || !pj.m || !pj.x || !pj.y || !pj.z || !abx || !aby || !abz || !pbar || !gx ||
-        !gy || !gz)
-        return set_error(SPHK_E_ARG, "gravity_vjp: null pointer");
-    if (s_off && (!ps.m || !ps.x || !ps.y || !ps.z || !nx || !ny || !nz))
-        return set_error(SPHK_E_ARG, "gravity_vjp: null SPJ pointer");
-    if (!(e2 > 0.)) return set_error(SPHK_E_ARG, "gravity_vjp: softening must be positive");
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(sphk::gravity_vjp_kernel, dim3(n_walk), dim3(sphk::kWave), 0, st, n_walk, i_off, j_off,
-                       j_idx, pj, s_off, s_idx, ps, pi, e2, abx, aby, abz, pbar, ebar, gx, gy, gz, nx, ny, nz);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return set_error(SPHK_E_DEVICE, "gravity_vjp: %s", hipGetErrorString(e));
-    return SPHK_OK;
+    return gravity_vjp(false, ctx, n_walk, i_off, j_off, j_idx, pj, s_off, s_idx, ps, pi, e2, abx, aby, abz, pbar,
+                       ebar, gx, gy, gz, nx, ny, nz, stream);
+}
+
+extern "C" int sphk_gravity_vjp_packed_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                                           const int32_t *j_idx, sphk_grav_src pj, const int32_t *s_off,
+                                           const int32_t *s_idx, sphk_grav_src ps, sphk_grav_src pi, double e2,
+                                           const double *abx, const double *aby, const double *abz,
+                                           const double *pbar, const double *ebar, double *g3, double *n3,
+                                           void *stream)
+{
+    return gravity_vjp(true, ctx, n_walk, i_off, j_off, j_idx, pj, s_off, s_idx, ps, pi, e2, abx, aby, abz, pbar,
+                       ebar, g3, nullptr, nullptr, n3, nullptr, nullptr, stream);
 }

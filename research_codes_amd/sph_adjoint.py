@@ -217,19 +217,20 @@ class _FrozenGravityFn(torch.autograd.Function):
         op = ctx.op
         x, y, z, X, Y, Z = ctx.saved_tensors
         w = op.walks
-        g = [torch.zeros_like(x) for _ in range(3)]
-        nb = [torch.zeros_like(X) for _ in range(3)]
+        g3, n3 = x.new_zeros(x.numel(), 3), X.new_zeros(X.numel(), 3)
         src = L.GravSrc(m=op.m.data_ptr(), x=x.data_ptr(), y=y.data_ptr(), z=z.data_ptr(),
                         eps2=op.e2p.data_ptr())
         ps = L.GravSrc(m=op.M.data_ptr(), x=X.data_ptr(), y=Y.data_ptr(), z=Z.data_ptr(),
                        eps2=op.e2n.data_ptr())
         z0 = torch.zeros_like(x)
         cot = [(z0 if c is None else c).contiguous() for c in (gax, gay, gaz, gpot)]
-        L.check(L.lib().sphk_gravity_vjp_dev(op.ctx.handle, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                             w.j_idx.data_ptr(), src, w.s_off.data_ptr(), w.s_idx.data_ptr(),
-                                             ps, src, op.e2, *(c.data_ptr() for c in cot), None,
-                                             *(a.data_ptr() for a in g), *(a.data_ptr() for a in nb),
-                                             torch.cuda.current_stream().cuda_stream), "sphk_gravity_vjp_dev")
+        L.check(L.lib().sphk_gravity_vjp_packed_dev(op.ctx.handle, w.n_walk, w.i_off.data_ptr(),
+                                                    w.j_off.data_ptr(), w.j_idx.data_ptr(), src,
+                                                    w.s_off.data_ptr(), w.s_idx.data_ptr(), ps, src, op.e2,
+                                                    *(c.data_ptr() for c in cot), None, g3.data_ptr(), n3.data_ptr(),
+                                                    torch.cuda.current_stream().cuda_stream),
+                "sphk_gravity_vjp_packed_dev")
+        g, nb = g3.t().contiguous(), n3.t().contiguous()
         return (*g, *nb, None)
 
 

@@ -1,0 +1,87 @@
+"""The vector-Jacobian products at the edges of their layouts: walks of one
+particle, of the register chunk's size and around it, of more than a wave;
+empty lists, single records, lists that end a tile exactly or one past it.
+
+Reference: the same sums over the same lists in torch FP64 on the CPU.
+Tolerance: a gradient component is a sum of at most a few hundred terms of
+one order of magnitude, each formed in a few tens of FP64 operations:
+1e-12 of the largest component is three orders above the rounding of that."""
+import numpy as np
+import pytest
+import torch
+
+from research_codes_amd import _lib as L
+from research_codes_amd.device import Context
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with Context(0) as c:
+        yield c
+
+
+def _walks(sizes, lengths, n_rec, rng):
+    i_off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    idx = np.concatenate([rng.permutation(n_rec)[:k] for k in lengths] + [np.zeros(0, int)]).astype(np.int32)
+    return i_off, off, idx
+
+
+def _pairs(i_off, off, idx):
+    i = np.concatenate([np.repeat(np.arange(i_off[w], i_off[w + 1]), off[w + 1] - off[w])
+                        for w in range(len(i_off) - 1)])
+    j = np.concatenate([np.tile(idx[off[w]:off[w + 1]], i_off[w + 1] - i_off[w]) for w in range(len(i_off) - 1)])
+    return torch.from_numpy(i).long(), torch.from_numpy(j).long()
+
+
+def _gravity_ref(x, pairs, rec, m, e2, cot):
+    """Gradients of sum(cot . (a, pot, eta)) by particle position and by record position."""
+    xi = x.clone().requires_grad_(True)
+    xr = rec.clone().requires_grad_(True)
+    i, j = pairs
+    d = xi[i] - xr[j]
+    w = ((d * d).sum(1) + e2) ** -0.5
+    mj = m[j]
+    loss = -((mj * w ** 3)[:, None] * d * cot[i, :3]).sum() - (mj * w * cot[i, 3]).sum() + (mj * w ** 3 * cot[i, 4]).sum()
+    return torch.autograd.grad(loss, [xi, xr])
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("nodes", [False, True])
+def test_gravity_vjp_edges(ctx, packed, nodes):
+    rng = np.random.default_rng(5)
+    sizes = [1, 15, 16, 17, 32, 33, 64, 70, 2]
+    n, nn, e2 = sum(sizes), 150, 0.01
+    jl = _walks(sizes, [0, 1, 63, 64, 65, 128, 130, 7, 200], n, rng)
+    sl = _walks(sizes, [64, 0, 1, 65, 63, 150, 128, 2, 0], nn, rng)
+    t = lambda *s: torch.from_numpy(rng.standard_normal(s))   # noqa: E731
+    x, X, cot = t(n, 3), 3.0 * t(nn, 3), t(n, 5)
+    m, M = torch.from_numpy(rng.uniform(0.5, 1.5, n)), torch.from_numpy(rng.uniform(0.5, 1.5, nn))
+    gi, gr = _gravity_ref(x, _pairs(*jl), x, m, e2, cot)
+    want, want_n = gi + gr, torch.zeros(nn, 3, dtype=torch.float64)
+    if nodes:
+        gi, want_n = _gravity_ref(x, _pairs(jl[0], *sl[1:]), X, M, e2, cot)
+        want = want + gi
+    dev = lambda a: a.contiguous().cuda() if isinstance(a, torch.Tensor) else torch.from_numpy(a).cuda()   # noqa: E731
+    keep = [dev(a) for a in (*jl, sl[1], sl[2], m, *x.T, M, *X.T, *cot.T)]
+    io, jo, ji, so, si = keep[:5]
+    src = L.GravSrc(**{k: a.data_ptr() for k, a in zip(("m", "x", "y", "z"), keep[5:9])})
+    ps = L.GravSrc(**{k: a.data_ptr() for k, a in zip(("m", "x", "y", "z"), keep[9:13])})
+    cots = [a.data_ptr() for a in keep[13:]]
+    lists = (ctx.handle, len(sizes), io.data_ptr(), jo.data_ptr(), ji.data_ptr(), src,
+             so.data_ptr() if nodes else None, si.data_ptr() if nodes else None, ps, src, e2, *cots)
+    st = torch.cuda.current_stream().cuda_stream
+    if packed:
+        g, gn = torch.ones(n, 3, dtype=torch.float64, device="cuda"), torch.ones(nn, 3, dtype=torch.float64, device="cuda")
+        L.check(L.lib().sphk_gravity_vjp_packed_dev(*lists, g.data_ptr(), gn.data_ptr(), st), "vjp")
+    else:
+        g, gn = torch.ones(3, n, dtype=torch.float64, device="cuda"), torch.ones(3, nn, dtype=torch.float64, device="cuda")
+        L.check(L.lib().sphk_gravity_vjp_dev(*lists, *(r.data_ptr() for r in (*g, *gn)), st), "vjp")
+        g, gn = g.T, gn.T
+    # accumulated onto what was there
+    assert float((g.cpu() - 1.0 - want).abs().max()) <= TOL * max(1.0, float(want.abs().max()))
+    assert float((gn.cpu() - 1.0 - want_n).abs().max()) <= TOL * max(1.0, float(want_n.abs().max()))
