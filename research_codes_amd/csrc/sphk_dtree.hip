@@ -4,14 +4,16 @@
 // policies; this one keeps everything in HBM:
 //   1. Morton keys over the bounding cube (block reduction, one key per
 //      thread); sphk_morton_order_dev sorts (key, index) with a radix sort.
-//   2. The octree is built breadth-first, one kernel pair per level: count
-//      the non-empty child octants of every frontier node (binary searches
-//      in the sorted keys), exclusive scan, write the children.  Children of
-//      one level are numbered in parent order and octant order, as the
-//      host's breadth-first loop numbers them.
-//   3. Node boxes and monopoles bottom-up, one kernel per level, each node
-//      summing its particles (leaf) or children in index order with FP
-//      contraction off, so the FP64 sums round as on the host.
+//   2. The octree's nodes, of all levels at once, from the sorted keys alone:
+//      which cells begin at a particle follows from its key, its neighbour's
+//      and those n_leaf places off (see span_kernel); nodes are counted per
+//      block and level, scanned, and written to their places.  A level's
+//      nodes are in key order, that is parent and octant order, as the host's
+//      breadth-first loop numbers them.
+//   3. Node boxes and monopoles bottom-up, one kernel per level (the top
+//      levels in one), each node summing its particles (leaf) or children in
+//      index order with FP contraction off, so the FP64 sums round as on the
+//      host.
 //   4. Groups: a node is a walk if it holds <= n_group particles (or is a
 //      leaf) and its parent holds more; walks are ordered by first particle.
 //   5. Lists: the host's depth-first traversal of each walk, 8 lanes per
@@ -104,16 +106,24 @@ __device__ __forceinline__ uint64_t spread3(uint64_t v)
 }
 
 // ---- bounding cube and keys ------------------------------------------------
+// COPY: the positions go to cx, cy, cz on the way.
+template <bool COPY>
 __global__ __launch_bounds__(kBlock) void bbox_partial_kernel(int n, const double *__restrict__ x,
                                                               const double *__restrict__ y,
                                                               const double *__restrict__ z,
-                                                              double *__restrict__ part)
+                                                              double *__restrict__ part, double *__restrict__ cx,
+                                                              double *__restrict__ cy, double *__restrict__ cz)
 {
     __shared__ double s[6][kBlock];
     const double inf = __builtin_inf();
     double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         const double p[3] = {x[i], y[i], z[i]};
+        if (COPY) {
+            cx[i] = p[0];
+            cy[i] = p[1];
+            cz[i] = p[2];
+        }
         for (int d = 0; d < 3; d++) {
             lo[d] = fmin(lo[d], p[d]);
             hi[d] = fmax(hi[d], p[d]);
@@ -201,22 +211,25 @@ __global__ __launch_bounds__(kBlock) void keys_kernel(int n, const double *__res
     if (idx) idx[i] = i;
 }
 
-__global__ __launch_bounds__(kBlock) void unsorted_kernel(int n, const uint64_t *__restrict__ key,
-                                                          int *__restrict__ flag)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= 1 && i < n && key[i] < key[i - 1]) atomicOr(flag, 1);
-}
-
-// Sets up the frame and keys of n particles (queued on st).
+// Sets up the frame and keys of n particles (queued on st); with copies, the
+// positions are copied to copies[0..2] first and the keys made from those.
 int make_keys(int n, const double *x, const double *y, const double *z, hipStream_t st, DArr<double> &part,
-              DArr<double> &frame, DArr<uint64_t> &key, int32_t *idx)
+              DArr<double> &frame, DArr<uint64_t> &key, int32_t *idx, double *const *copies = nullptr)
 {
     const int nb = std::min(1024, (n + kBlock - 1) / kBlock);
     SPHK_TRY(part.reserve(6 * (size_t)nb, false, st));
     SPHK_TRY(frame.reserve(4, false, st));
     SPHK_TRY(key.reserve(n, false, st));
-    hipLaunchKernelGGL(bbox_partial_kernel, dim3(nb), dim3(kBlock), 0, st, n, x, y, z, part.p);
+    if (copies) {
+        hipLaunchKernelGGL(bbox_partial_kernel<true>, dim3(nb), dim3(kBlock), 0, st, n, x, y, z, part.p, copies[0],
+                           copies[1], copies[2]);
+        x = copies[0];
+        y = copies[1];
+        z = copies[2];
+    } else {
+        hipLaunchKernelGGL(bbox_partial_kernel<false>, dim3(nb), dim3(kBlock), 0, st, n, x, y, z, part.p, nullptr,
+                           nullptr, nullptr);
+    }
     hipLaunchKernelGGL(bbox_final_kernel, dim3(1), dim3(kBlock), 0, st, nb, part.p, frame.p);
     hipLaunchKernelGGL(keys_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, n, x, y, z,
                        frame.p, key.p, idx);
@@ -230,72 +243,178 @@ struct NodeArrays {
     double *len;
 };
 
-// First index in [b, e) whose octant digit exceeds o (keys sorted).
-__device__ __forceinline__ int32_t octant_end(const uint64_t *__restrict__ key, int32_t b, int32_t e, int shift,
-                                              int o)
+// A node is a cell (level L: equal first L key digits) that is the root or
+// whose parent cell holds more than n_leaf particles; it begins at its first
+// particle.  So the nodes that begin at particle i are those of the levels
+//   c + 1 .. min(l + 1, kMaxLevel),
+// c the digits key[i] shares with key[i - 1] (-1 for i = 0) and l the deepest
+// level at which i's cell holds more than n_leaf particles: the most digits
+// shared by the ends of any n_leaf + 1 consecutive particles with i among
+// them (-1 if there are none).  All levels are built at once from these
+// spans: a count kernel, scan kernels and a write kernel per level, each with
+// a host read of the level's size, made a rebuild latency-bound (57 launches
+// and 10 reads at 10^6 particles; rebuild and the three lists 6.5 -> 5.7 ms,
+// a KDK step of 2x10^5 particles 5.2 -> 4.2 ms without them).
+constexpr int kLevels = kMaxLevel + 1;
+constexpr int kSpanTile = 1024;   // particles per block of the span, node and group kernels
+constexpr int kSpanHalo = 512;    // n_leaf up to this: window ends compared once per block, in LDS
+
+__device__ __forceinline__ int shared_digits(uint64_t a, uint64_t b)
 {
-    while (b < e) {
-        const int32_t mid = b + ((e - b) >> 1);
-        if ((int)((key[mid] >> shift) & 7) <= o)
-            b = mid + 1;
+    return a == b ? kMaxLevel : (__clzll(a ^ b) - 1) / 3;
+}
+
+struct Span {
+    int8_t lo, hi;
+};
+
+// Spans of all particles, the number of nodes that begin in each block per
+// level (hist, level-major), and *unsorted set if the keys are not in order.
+__global__ __launch_bounds__(kSpanTile) void span_kernel(int n, const uint64_t *__restrict__ key, int n_leaf,
+                                                         Span *__restrict__ span, int32_t *__restrict__ hist,
+                                                         int32_t *__restrict__ head, int *__restrict__ unsorted)
+{
+    __shared__ int8_t ends[kSpanTile + kSpanHalo];   // digits shared by the ends of window a
+    __shared__ int cnt[kLevels];
+    const int t = threadIdx.x, i0 = blockIdx.x * kSpanTile, i = i0 + t;
+    auto window = [&](int a) { return a >= 0 && a + n_leaf < n ? shared_digits(key[a], key[a + n_leaf]) : -1; };
+    if (t < kLevels) cnt[t] = 0;
+    if (n_leaf <= kSpanHalo)
+        for (int q = t; q < kSpanTile + n_leaf; q += kSpanTile) ends[q] = (int8_t)window(i0 - n_leaf + q);
+    __syncthreads();
+    int lo = kLevels, hi = -1;
+    if (i < n) {
+        int l = -1;
+        if (n_leaf <= kSpanHalo)
+            for (int q = 0; q <= n_leaf; q++) l = max(l, (int)ends[t + q]);
+        else
+            for (int q = 0; q <= n_leaf; q++) l = max(l, window(i - q));
+        if (i > 0 && key[i] < key[i - 1]) atomicOr(unsorted, 1);
+        lo = i == 0 ? 0 : shared_digits(key[i - 1], key[i]) + 1;
+        hi = min(l + 1, kMaxLevel);
+        span[i] = Span{(int8_t)lo, (int8_t)hi};
+        head[i] = -1;
+    }
+    for (int L = 0; L < kLevels; L++) {
+        const uint64_t b = __ballot(lo <= L && L <= hi);
+        if ((t & 63) == 0 && b) atomicAdd(&cnt[L], __popcll(b));
+    }
+    __syncthreads();
+    if (t < kLevels) hist[t * gridDim.x + blockIdx.x] = cnt[t];
+}
+
+// Exclusive scan of m counts in place by one block; total[0] the sum, and
+// first[L] the value at L * stride (the starts of the levels) for L < nl.
+constexpr int kScanThreads = 1024;
+
+__global__ __launch_bounds__(kScanThreads) void block_scan_kernel(int m, int32_t *__restrict__ a, int nl, int stride,
+                                                                  int64_t *__restrict__ first,
+                                                                  int64_t *__restrict__ total)
+{
+    __shared__ int64_t wsum[kScanThreads / 64];
+    const int t = threadIdx.x, lane = t & 63;
+    const int per = (m + kScanThreads - 1) / kScanThreads;
+    const int b = min(m, t * per), e = min(m, b + per);
+    int64_t sum = 0;
+    for (int k = b; k < e; k++) sum += a[k];
+    int64_t incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t u = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += u;
+    }
+    if (lane == 63) wsum[t / 64] = incl;
+    __syncthreads();
+    int64_t at = incl - sum;
+    for (int w = 0; w < t / 64; w++) at += wsum[w];
+    for (int k = b; k < e; k++) {
+        const int c = a[k];
+        if (nl && k % stride == 0) first[k / stride] = at;
+        a[k] = (int32_t)at;
+        at += c;
+    }
+    if (t == kScanThreads - 1) *total = at;   // the last threads may own nothing: at is the sum
+}
+
+// First index past i whose key differs from key[i] in the first L digits
+// (keys sorted): doubling steps, then bisection.
+__device__ __forceinline__ int32_t cell_end(const uint64_t *__restrict__ key, int n, int i, int L)
+{
+    if (L == 0) return n;
+    const int shift = 3 * (kMaxLevel - L);
+    const uint64_t p = key[i] >> shift;
+    int64_t step = 1;
+    while (i + step < n && (key[i + step] >> shift) == p) step *= 2;
+    int32_t b = (int32_t)(i + step / 2), e = (int32_t)(i + step < n ? i + step : n);   // key[b] inside, e outside
+    while (e - b > 1) {
+        const int32_t mid = b + (e - b) / 2;
+        if ((key[mid] >> shift) == p)
+            b = mid;
         else
             e = mid;
     }
-    return b;
+    return e;
 }
 
-template <bool WRITE>
-__global__ __launch_bounds__(kBlock) void split_kernel(int fa, int nf, const uint64_t *__restrict__ key,
-                                                       NodeArrays nd, int n_leaf, int64_t *__restrict__ cnt,
-                                                       const int64_t *__restrict__ off, int base)
+// The nodes that begin at each particle, at the places the scanned counts
+// give.  A node's parent is the last node of the level above that begins at
+// or before it; a parent counts its children (nchild zero before).
+__global__ __launch_bounds__(kSpanTile) void node_kernel(int n, const uint64_t *__restrict__ key,
+                                                         const Span *__restrict__ span,
+                                                         const int32_t *__restrict__ hist, NodeArrays nd,
+                                                         const double *__restrict__ frame)
 {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nf) return;
-    const int a = fa + k;
-    const int32_t nb = nd.begin[a], ne = nd.end[a], lv = nd.level[a];
-    if (ne - nb <= n_leaf || lv >= kMaxLevel) {
-        if (!WRITE) cnt[k] = 0;
-        return;
+    __shared__ int base[kSpanTile / 64][kLevels];
+    const int t = threadIdx.x, lane = t & 63, wave = t / 64, i = blockIdx.x * kSpanTile + t;
+    const Span sp = i < n ? span[i] : Span{(int8_t)kLevels, (int8_t)-1};
+    for (int L = 0; L < kLevels; L++) {
+        const uint64_t b = __ballot(sp.lo <= L && L <= sp.hi);
+        if (lane == 0) base[wave][L] = __popcll(b);
     }
-    const int shift = 3 * (20 - lv);
-    int32_t b = nb;
-    int nch = 0;
-    const int first = WRITE ? base + (int)off[k] : 0;
-    for (int o = 0; o < 8 && b < ne; o++) {
-        const int32_t e = octant_end(key, b, ne, shift, o);
-        if (e > b) {
-            if (WRITE) {
-                const int c = first + nch;
-                nd.begin[c] = b;
-                nd.end[c] = e;
-                nd.child[c] = -1;
-                nd.nchild[c] = 0;
-                nd.level[c] = lv + 1;
-                nd.parent[c] = a;
-                nd.len[c] = nd.len[a] * 0.5;
-            }
-            nch++;
+    __syncthreads();
+    if (t < kLevels) {
+        int at = hist[t * gridDim.x + blockIdx.x];
+        for (int w = 0; w < kSpanTile / 64; w++) {
+            const int c = base[w][t];
+            base[w][t] = at;
+            at += c;
         }
-        b = e;
     }
-    if (WRITE) {
-        nd.child[a] = first;
-        nd.nchild[a] = nch;
-    } else {
-        cnt[k] = nch;
+    __syncthreads();
+    int above = -1;   // the node of level L - 1 that holds i
+    double len = frame[3];
+    for (int L = 0; L < kLevels; L++, len *= 0.5) {
+        const bool in = sp.lo <= L && L <= sp.hi;
+        const uint64_t b = __ballot(in);
+        const int a = base[wave][L] + __popcll(b & ((1ull << lane) - 1));
+        if (in) {
+            nd.begin[a] = i;
+            nd.end[a] = cell_end(key, n, i, L);
+            nd.level[a] = L;
+            nd.parent[a] = above;
+            nd.len[a] = len;
+            if (L == sp.hi) nd.child[a] = -1;            // a leaf: its first particle heads no deeper node
+            if (L > sp.lo) nd.child[above] = a;          // begins where its parent does
+            if (L > 0) atomicAdd(&nd.nchild[above], 1);
+        }
+        above = in ? a : a - 1;
     }
 }
 
-__global__ void root_kernel(int n, NodeArrays nd, const double *__restrict__ frame)
-{
-    nd.begin[0] = 0;
-    nd.end[0] = n;
-    nd.child[0] = -1;
-    nd.nchild[0] = 0;
-    nd.level[0] = 0;
-    nd.parent[0] = -1;
-    nd.len[0] = frame[3];
-}
+// Node records for the list walks: the fields one visit reads, packed in
+// one 64-byte record per node (one memory segment per visit instead of one
+// per field array).  Values are copies of the node arrays, so the walks'
+// comparisons and their results are unchanged.
+struct alignas(64) BoxRec {     // gather and symmetry walks
+    double lo[3], hi[3];        // tight box
+    int32_t child, nchild, begin, end;
+};
+struct alignas(64) MacRec {     // long walk
+    double mx, my, mz, mm, len;
+    int32_t child, nchild, begin, end;
+};
+struct alignas(64) OboxRec {    // symmetry walk: box of the nodes' particle spheres
+    double lo[3], hi[3];
+};
 
 // ---- boxes and monopoles, one level at a time (bottom-up) ------------------
 struct Moments {
@@ -305,17 +424,12 @@ struct Moments {
     size_t cap;
 };
 
-__global__ __launch_bounds__(kBlock) void moments_kernel(int a0, int na, NodeArrays nd, Moments mo,
-                                                         const double *__restrict__ x,
-                                                         const double *__restrict__ y,
-                                                         const double *__restrict__ z,
-                                                         const double *__restrict__ m,
-                                                         const double *__restrict__ eps2)
+__device__ __forceinline__ void node_moments(int a, const NodeArrays &nd, const Moments &mo, BoxRec *__restrict__ br,
+                                             MacRec *__restrict__ mr, const double *__restrict__ x,
+                                             const double *__restrict__ y, const double *__restrict__ z,
+                                             const double *__restrict__ m, const double *__restrict__ eps2)
 {
 #pragma clang fp contract(off)
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= na) return;
-    const int a = a0 + k;
     const size_t C = mo.cap;
     const double inf = __builtin_inf();
     double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
@@ -356,30 +470,61 @@ __global__ __launch_bounds__(kBlock) void moments_kernel(int a0, int na, NodeArr
     mo.sy[a] = Y;
     mo.sz[a] = Z;
     mo.se[a] = E;
+    double c[3], e = 0.;
     if (M > 0.) {
-        mo.mx[a] = X / M;
-        mo.my[a] = Y / M;
-        mo.mz[a] = Z / M;
-        mo.me[a] = E / M;
+        c[0] = X / M;
+        c[1] = Y / M;
+        c[2] = Z / M;
+        e = E / M;
     } else {
-        mo.mx[a] = 0.5 * (lo[0] + hi[0]);
-        mo.my[a] = 0.5 * (lo[1] + hi[1]);
-        mo.mz[a] = 0.5 * (lo[2] + hi[2]);
-        mo.me[a] = 0.;
+        for (int d = 0; d < 3; d++) c[d] = 0.5 * (lo[d] + hi[d]);
+    }
+    mo.mx[a] = c[0];
+    mo.my[a] = c[1];
+    mo.mz[a] = c[2];
+    mo.me[a] = e;
+    // the records the list walks read
+    const int child = nd.child[a], nch = nd.nchild[a], begin = nd.begin[a], end = nd.end[a];
+    br[a] = BoxRec{{lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}, child, nch, begin, end};
+    mr[a] = MacRec{c[0], c[1], c[2], M, nd.len[a], child, nch, begin, end};
+}
+
+__global__ __launch_bounds__(kBlock) void moments_kernel(int a0, int na, NodeArrays nd, Moments mo,
+                                                         BoxRec *__restrict__ br, MacRec *__restrict__ mr,
+                                                         const double *__restrict__ x, const double *__restrict__ y,
+                                                         const double *__restrict__ z, const double *__restrict__ m,
+                                                         const double *__restrict__ eps2)
+{
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < na) node_moments(a0 + k, nd, mo, br, mr, x, y, z, m, eps2);
+}
+
+// The top levels (starts in ls, `levels` of them) in one block, deepest first:
+// a launch per level costs more than their few nodes.
+struct TopLevels {
+    int levels;
+    int ls[kMaxLevel + 2];
+};
+constexpr int kTopThreads = 1024;
+constexpr int kTopNodes = 4096;   // levels are top while no level is wider than this
+
+__global__ __launch_bounds__(kTopThreads) void moments_top_kernel(TopLevels tl, NodeArrays nd, Moments mo,
+                                                                  BoxRec *br, MacRec *mr, const double *x,
+                                                                  const double *y, const double *z, const double *m,
+                                                                  const double *eps2)
+{
+    for (int L = tl.levels - 1; L >= 0; L--) {
+        for (int a = tl.ls[L] + threadIdx.x; a < tl.ls[L + 1]; a += kTopThreads)
+            node_moments(a, nd, mo, br, mr, x, y, z, m, eps2);
+        __syncthreads();   // children's sums written before the parents read them
     }
 }
 
 // Box of x_j +- h_j per node (symmetry lists), bottom-up.
-__global__ __launch_bounds__(kBlock) void obox_kernel(int a0, int na, NodeArrays nd, double *__restrict__ olo,
-                                                      double *__restrict__ ohi, size_t C,
-                                                      const double *__restrict__ x,
-                                                      const double *__restrict__ y,
-                                                      const double *__restrict__ z,
-                                                      const double *__restrict__ h)
+__device__ __forceinline__ void node_obox(int a, const NodeArrays &nd, OboxRec *orr, const double *__restrict__ x,
+                                          const double *__restrict__ y, const double *__restrict__ z,
+                                          const double *__restrict__ h)
 {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= na) return;
-    const int a = a0 + k;
     const double inf = __builtin_inf();
     double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     if (nd.child[a] < 0) {
@@ -391,15 +536,32 @@ __global__ __launch_bounds__(kBlock) void obox_kernel(int a0, int na, NodeArrays
             }
         }
     } else {
-        for (int c = nd.child[a]; c < nd.child[a] + nd.nchild[a]; c++)
+        for (int c = nd.child[a]; c < nd.child[a] + nd.nchild[a]; c++) {
+            const OboxRec o = orr[c];
             for (int d = 0; d < 3; d++) {
-                lo[d] = fmin(lo[d], olo[d * C + c]);
-                hi[d] = fmax(hi[d], ohi[d * C + c]);
+                lo[d] = fmin(lo[d], o.lo[d]);
+                hi[d] = fmax(hi[d], o.hi[d]);
             }
+        }
     }
-    for (int d = 0; d < 3; d++) {
-        olo[d * C + a] = lo[d];
-        ohi[d * C + a] = hi[d];
+    orr[a] = OboxRec{{lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}};
+}
+
+__global__ __launch_bounds__(kBlock) void obox_kernel(int a0, int na, NodeArrays nd, OboxRec *orr,
+                                                      const double *__restrict__ x, const double *__restrict__ y,
+                                                      const double *__restrict__ z, const double *__restrict__ h)
+{
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < na) node_obox(a0 + k, nd, orr, x, y, z, h);
+}
+
+__global__ __launch_bounds__(kTopThreads) void obox_top_kernel(TopLevels tl, NodeArrays nd, OboxRec *orr,
+                                                               const double *x, const double *y, const double *z,
+                                                               const double *h)
+{
+    for (int L = tl.levels - 1; L >= 0; L--) {
+        for (int a = tl.ls[L] + threadIdx.x; a < tl.ls[L + 1]; a += kTopThreads) node_obox(a, nd, orr, x, y, z, h);
+        __syncthreads();
     }
 }
 
@@ -421,77 +583,42 @@ __global__ __launch_bounds__(kBlock) void group_mark_kernel(int nn, NodeArrays n
     if (small && opened) head[nd.begin[a]] = a;
 }
 
-__global__ __launch_bounds__(kBlock) void head_flag_kernel(int n, const int32_t *__restrict__ head,
-                                                           int64_t *__restrict__ flag)
+// Groups that begin in each block of particles.
+__global__ __launch_bounds__(kSpanTile) void group_count_kernel(int n, const int32_t *__restrict__ head,
+                                                                int32_t *__restrict__ cnt)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) flag[i] = head[i] >= 0 ? 1 : 0;
+    __shared__ int c;
+    const int i = blockIdx.x * kSpanTile + threadIdx.x;
+    if (threadIdx.x == 0) c = 0;
+    __syncthreads();
+    const uint64_t b = __ballot(i < n && head[i] >= 0);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&c, __popcll(b));
+    __syncthreads();
+    if (threadIdx.x == 0) cnt[blockIdx.x] = c;
 }
 
-__global__ __launch_bounds__(kBlock) void group_write_kernel(int n, const int32_t *__restrict__ head,
-                                                             const int64_t *__restrict__ pos,
-                                                             int32_t *__restrict__ group,
-                                                             int32_t *__restrict__ i_off, int ng)
+__global__ __launch_bounds__(kSpanTile) void group_write_kernel(int n, const int32_t *__restrict__ head,
+                                                                const int32_t *__restrict__ pos,
+                                                                const int64_t *__restrict__ total,
+                                                                int32_t *__restrict__ group,
+                                                                int32_t *__restrict__ i_off)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    if (head[i] >= 0) {
-        group[pos[i]] = head[i];
-        i_off[pos[i]] = i;
+    __shared__ int wc[kSpanTile / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t / 64, i = blockIdx.x * kSpanTile + t;
+    const int a = i < n ? head[i] : -1;
+    const uint64_t b = __ballot(a >= 0);
+    if (lane == 0) wc[wave] = __popcll(b);
+    __syncthreads();
+    int at = pos[blockIdx.x] + __popcll(b & ((1ull << lane) - 1));
+    for (int w = 0; w < wave; w++) at += wc[w];
+    if (a >= 0) {
+        group[at] = a;
+        i_off[at] = i;
     }
-    if (i == 0) i_off[ng] = n;
+    if (i == 0) i_off[*total] = n;
 }
 
 // ---- lists -------------------------------------------------------------------
-// Node records for the list walks: the fields one visit reads, packed in
-// one 64-byte record per node (one memory segment per visit instead of one
-// per field array).  Values are copies of the node arrays, so the walks'
-// comparisons and their results are unchanged.
-struct alignas(64) BoxRec {     // gather and symmetry walks
-    double lo[3], hi[3];        // tight box
-    int32_t child, nchild, begin, end;
-};
-struct alignas(64) MacRec {     // long walk
-    double mx, my, mz, mm, len;
-    int32_t child, nchild, begin, end;
-};
-struct alignas(64) OboxRec {    // symmetry walk: box of the nodes' particle spheres
-    double lo[3], hi[3];
-};
-
-__global__ __launch_bounds__(kBlock) void pack_nodes_kernel(int nn, NodeArrays nd, Moments mo,
-                                                            BoxRec *__restrict__ br, MacRec *__restrict__ mr)
-{
-    const int a = blockIdx.x * kBlock + threadIdx.x;
-    if (a >= nn) return;
-    const size_t C = mo.cap;
-    BoxRec b;
-    for (int d = 0; d < 3; d++) {
-        b.lo[d] = mo.lo[d * C + a];
-        b.hi[d] = mo.hi[d * C + a];
-    }
-    b.child = nd.child[a];
-    b.nchild = nd.nchild[a];
-    b.begin = nd.begin[a];
-    b.end = nd.end[a];
-    br[a] = b;
-    mr[a] = MacRec{mo.mx[a], mo.my[a], mo.mz[a], mo.mm[a], nd.len[a], b.child, b.nchild, b.begin, b.end};
-}
-
-__global__ __launch_bounds__(kBlock) void pack_obox_kernel(int nn, const double *__restrict__ olo,
-                                                           const double *__restrict__ ohi, size_t C,
-                                                           OboxRec *__restrict__ orr)
-{
-    const int a = blockIdx.x * kBlock + threadIdx.x;
-    if (a >= nn) return;
-    OboxRec o;
-    for (int d = 0; d < 3; d++) {
-        o.lo[d] = olo[d * C + a];
-        o.hi[d] = ohi[d * C + a];
-    }
-    orr[a] = o;
-}
-
 struct TreeView {
     NodeArrays nd;
     Moments mo;
@@ -912,8 +1039,10 @@ struct sphk_dtree {
     DArr<int32_t> begin, end, child, nchild, level, parent;
     std::vector<int> level_start;   // node index of the first node of each level
     int n_node = 0;
-    DArr<double> box_lo, box_hi, mm, mx, my, mz, me, sx, sy, sz, se, olo, ohi;
-    DArr<int32_t> head, group, i_off, mscr;
+    DArr<double> box_lo, box_hi, mm, mx, my, mz, me, sx, sy, sz, se;
+    DArr<int32_t> head, group, i_off, mscr, hist;
+    DArr<Span> span;
+    DArr<int64_t> levels;   // starts of the levels and the node count; the group count; the unsorted flag
     int n_walk = 0;
     DArr<double> wbox;
     DArr<BoxRec> brec;
@@ -939,11 +1068,13 @@ struct sphk_dtree {
     void release()
     {
         for (auto *a : {&x, &y, &z, &part, &frame, &len, &box_lo, &box_hi, &mm, &mx, &my, &mz, &me, &sx, &sy,
-                        &sz, &se, &olo, &ohi})
+                        &sz, &se})
             a->release();
         key.release();
-        for (auto *a : {&begin, &end, &child, &nchild, &level, &parent, &head, &group, &i_off, &mscr})
+        for (auto *a : {&begin, &end, &child, &nchild, &level, &parent, &head, &group, &i_off, &mscr, &hist})
             a->release();
+        span.release();
+        levels.release();
         wbox.release();
         brec.release();
         mrec.release();
@@ -965,10 +1096,16 @@ namespace {
 
 int reserve_nodes(sphk_dtree *t, size_t cap)
 {
-    if (cap <= t->begin.cap) return SPHK_OK;
     for (auto *a : {&t->begin, &t->end, &t->child, &t->nchild, &t->level, &t->parent})
-        SPHK_TRY(a->reserve(cap, true, t->st));
-    SPHK_TRY(t->len.reserve(cap, true, t->st));
+        SPHK_TRY(a->reserve(cap, false, t->st));
+    SPHK_TRY(t->len.reserve(cap, false, t->st));
+    for (auto *a : {&t->mm, &t->mx, &t->my, &t->mz, &t->me, &t->sx, &t->sy, &t->sz, &t->se})
+        SPHK_TRY(a->reserve(cap, false, t->st));
+    // the box arrays are [3][cap]
+    SPHK_TRY(t->box_lo.reserve(3 * cap, false, t->st));
+    SPHK_TRY(t->box_hi.reserve(3 * cap, false, t->st));
+    SPHK_TRY(t->brec.reserve(cap, false, t->st));
+    SPHK_TRY(t->mrec.reserve(cap, false, t->st));
     return SPHK_OK;
 }
 
@@ -1263,6 +1400,17 @@ int sphk_morton_order_dev(int n, const double *x, const double *y, const double 
 
 namespace {
 
+// The levels that moments_top_kernel and obox_top_kernel take: from the root
+// while none is wider than kTopNodes.
+TopLevels top_levels(const sphk_dtree *t)
+{
+    TopLevels tl{};
+    const int n = (int)t->level_start.size() - 1;
+    while (tl.levels < n && t->level_start[tl.levels + 1] - t->level_start[tl.levels] <= kTopNodes) tl.levels++;
+    for (int L = 0; L <= tl.levels; L++) tl.ls[L] = t->level_start[L];
+    return tl;
+}
+
 // The build proper, into t's buffers (grown as needed).  On failure t holds
 // no tree; its buffers stay allocated for a later build or sphk_dtree_free.
 int build_tree(sphk_dtree *t, int n, const double *x, const double *y, const double *z, const double *m,
@@ -1287,92 +1435,67 @@ int build_tree(sphk_dtree *t, int n, const double *x, const double *y, const dou
         return rc;
     };
     hipStream_t st = t->st;
+    const int nb = (n + kSpanTile - 1) / kSpanTile;
     // own copies of the positions (list builds read them later)
-    for (auto pr : {std::make_pair(&t->x, x), std::make_pair(&t->y, y), std::make_pair(&t->z, z)}) {
-        if (pr.first->reserve(n, false, st) != hipSuccess ||
-            hipMemcpyAsync(pr.first->p, pr.second, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess)
-            return fail(set_error(SPHK_E_DEVICE, "dtree: position copy failed"));
-    }
-    if (int rc = make_keys(n, t->x.p, t->y.p, t->z.p, st, t->part, t->frame, t->key, nullptr)) return fail(rc);
-    if (t->err.reserve(1, false, st) != hipSuccess || hipMemsetAsync(t->err.p, 0, sizeof(int), st) != hipSuccess)
+    for (auto *a : {&t->x, &t->y, &t->z})
+        if (a->reserve(n, false, st) != hipSuccess) return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
+    if (t->err.reserve(1, false, st) != hipSuccess || t->span.reserve(n, false, st) != hipSuccess ||
+        t->head.reserve(n, false, st) != hipSuccess || t->hist.reserve((size_t)kLevels * nb, false, st) != hipSuccess ||
+        t->levels.reserve(kLevels + 3, false, st) != hipSuccess)
         return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    hipLaunchKernelGGL(unsorted_kernel, dim3(grid(n)), dim3(kBlock), 0, st, n, t->key.p, t->err.p);
-    int unsorted = 0;
-    if (int rc = read1(st, t->err.p, &unsorted)) return fail(rc);
-    if (unsorted)
-        return fail(set_error(SPHK_E_ARG, "dtree: particles are not in Morton order (use sphk_morton_order_dev)"));
+    double *const copies[3] = {t->x.p, t->y.p, t->z.p};
+    if (int rc = make_keys(n, x, y, z, st, t->part, t->frame, t->key, nullptr, copies)) return fail(rc);
 
-    // root, then one level at a time
-    if (int rc = reserve_nodes(t, 2 * (size_t)n / std::max(1, n_leaf) + 16)) return fail(rc);
-    hipLaunchKernelGGL(root_kernel, dim3(1), dim3(1), 0, st, n, t->nodes(), t->frame.p);
-    t->level_start = {0, 1};
-    int fa = 0, fb = 1;
-    while (fa < fb) {
-        const int nf = fb - fa;
-        if (t->i64a.reserve(nf, false, st) != hipSuccess || t->i64c.reserve(nf, false, st) != hipSuccess ||
-            t->total.reserve(2, false, st) != hipSuccess)
-            return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-        hipLaunchKernelGGL((split_kernel<false>), dim3(grid(nf)), dim3(kBlock), 0, st, fa, nf, t->key.p,
-                           t->nodes(), n_leaf, t->i64a.p, nullptr, 0);
-        if (int rc = scan64(t, t->i64a.p, t->i64c.p, nf)) return fail(rc);
-        int64_t last[2];
-        if (hipMemcpyAsync(&last[0], t->i64c.p + nf - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipMemcpyAsync(&last[1], t->i64a.p + nf - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            return fail(set_error(SPHK_E_DEVICE, "dtree: level size read failed"));
-        const int64_t nnew = last[0] + last[1];
-        if (nnew == 0) break;
-        if (fb + nnew >= (1 << 29))   // list walks pack node indices into 29 bits
-            return fail(set_error(SPHK_E_CAPACITY, "dtree: too many nodes"));
-        if ((size_t)(fb + nnew) > t->begin.cap)
-            if (int rc = reserve_nodes(t, std::max<size_t>((size_t)(fb + nnew), t->begin.cap * 3 / 2))) return fail(rc);
-        hipLaunchKernelGGL((split_kernel<true>), dim3(grid(nf)), dim3(kBlock), 0, st, fa, nf, t->key.p, t->nodes(),
-                           n_leaf, nullptr, t->i64c.p, fb);
-        fa = fb;
-        fb = fb + (int)nnew;
-        t->level_start.push_back(fb);
-    }
-    t->n_node = fb;
-    const size_t nn = (size_t)fb;
+    // nodes per level: one host read of the level starts and the order check
+    int64_t *const lv = t->levels.p, *const n_group_dev = lv + kLevels + 1;
+    int *const unsorted = reinterpret_cast<int *>(lv + kLevels + 2);
+    hipLaunchKernelGGL(fill_kernel, dim3(1), dim3(kBlock), 0, st, 2, reinterpret_cast<int32_t *>(unsorted), 0);
+    hipLaunchKernelGGL(span_kernel, dim3(nb), dim3(kSpanTile), 0, st, n, t->key.p, std::min(n_leaf, n), t->span.p, t->hist.p,
+                       t->head.p, unsorted);
+    hipLaunchKernelGGL(block_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, kLevels * nb, t->hist.p, kLevels, nb, lv,
+                       lv + kLevels);
+    int64_t h[kLevels + 3];
+    if (hipMemcpyAsync(h, lv, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+        return fail(set_error(SPHK_E_DEVICE, "dtree: level sizes read failed"));
+    if (h[kLevels + 2] != 0)
+        return fail(set_error(SPHK_E_ARG, "dtree: particles are not in Morton order (use sphk_morton_order_dev)"));
+    if (h[kLevels] >= (1 << 29))   // list walks pack node indices into 29 bits
+        return fail(set_error(SPHK_E_CAPACITY, "dtree: too many nodes"));
+    const size_t nn = (size_t)h[kLevels];
+    t->n_node = (int)nn;
+    t->level_start.clear();
+    for (int L = 0; L <= kLevels && (L == 0 || h[L] > h[L - 1]); L++) t->level_start.push_back((int)h[L]);
+    if (nn > t->begin.cap)
+        if (int rc = reserve_nodes(t, std::max<size_t>(nn, 2 * (size_t)n / std::max(1, n_leaf) + 16))) return fail(rc);
+    hipLaunchKernelGGL(fill_kernel, dim3(grid((int)nn)), dim3(kBlock), 0, st, (int)nn, t->nchild.p, 0);
+    hipLaunchKernelGGL(node_kernel, dim3(nb), dim3(kSpanTile), 0, st, n, t->key.p, t->span.p, t->hist.p, t->nodes(),
+                       t->frame.p);
 
     // boxes and monopoles, deepest level first
-    for (auto *a : {&t->mm, &t->mx, &t->my, &t->mz, &t->me, &t->sx, &t->sy, &t->sz, &t->se})
-        if (a->reserve(nn, false, st) != hipSuccess) return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    if (t->box_lo.reserve(3 * nn, false, st) != hipSuccess || t->box_hi.reserve(3 * nn, false, st) != hipSuccess)
-        return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    // the box arrays are [3][cap]; cap = box_lo.cap / 3 must match box_hi's
-    if (t->box_lo.cap != t->box_hi.cap) return fail(set_error(SPHK_E_STATE, "dtree: box capacity mismatch"));
-    for (int L = (int)t->level_start.size() - 2; L >= 0; L--) {
+    const TopLevels top = top_levels(t);
+    for (int L = (int)t->level_start.size() - 2; L >= top.levels; L--) {
         const int a0 = t->level_start[L], na = t->level_start[L + 1] - a0;
         hipLaunchKernelGGL(moments_kernel, dim3(grid(na)), dim3(kBlock), 0, st, a0, na, t->nodes(), t->moments(),
-                           t->x.p, t->y.p, t->z.p, m, eps2);
+                           t->brec.p, t->mrec.p, t->x.p, t->y.p, t->z.p, m, eps2);
     }
+    hipLaunchKernelGGL(moments_top_kernel, dim3(1), dim3(kTopThreads), 0, st, top, t->nodes(), t->moments(), t->brec.p,
+                       t->mrec.p, t->x.p, t->y.p, t->z.p, m, eps2);
     if (hipGetLastError() != hipSuccess) return fail(set_error(SPHK_E_DEVICE, "dtree: moments launch failed"));
-    if (t->brec.reserve(nn, false, st) != hipSuccess || t->mrec.reserve(nn, false, st) != hipSuccess)
-        return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    hipLaunchKernelGGL(pack_nodes_kernel, dim3(grid((int)nn)), dim3(kBlock), 0, st, (int)nn, t->nodes(),
-                       t->moments(), t->brec.p, t->mrec.p);
 
-    // groups
-    if (t->head.reserve(n, false, st) != hipSuccess || t->i64a.reserve(n, false, st) != hipSuccess ||
-        t->i64c.reserve(n, false, st) != hipSuccess)
+    // groups (at most one per particle)
+    if (t->group.reserve(n, false, st) != hipSuccess || t->i_off.reserve((size_t)n + 1, false, st) != hipSuccess)
         return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    hipLaunchKernelGGL(fill_kernel, dim3(grid(n)), dim3(kBlock), 0, st, n, t->head.p, -1);
     hipLaunchKernelGGL(group_mark_kernel, dim3(grid((int)nn)), dim3(kBlock), 0, st, (int)nn, t->nodes(), n_group,
                        t->head.p);
-    hipLaunchKernelGGL(head_flag_kernel, dim3(grid(n)), dim3(kBlock), 0, st, n, t->head.p, t->i64a.p);
-    if (int rc = scan64(t, t->i64a.p, t->i64c.p, n)) return fail(rc);
-    int64_t last[2];
-    if (hipMemcpyAsync(&last[0], t->i64c.p + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(&last[1], t->i64a.p + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-        return fail(set_error(SPHK_E_DEVICE, "dtree: group count read failed"));
-    const int ng = (int)(last[0] + last[1]);
-    if (t->group.reserve(ng, false, st) != hipSuccess || t->i_off.reserve(ng + 1, false, st) != hipSuccess)
-        return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
-    hipLaunchKernelGGL(group_write_kernel, dim3(grid(n)), dim3(kBlock), 0, st, n, t->head.p, t->i64c.p, t->group.p,
-                       t->i_off.p, ng);
+    hipLaunchKernelGGL(group_count_kernel, dim3(nb), dim3(kSpanTile), 0, st, n, t->head.p, t->hist.p);
+    hipLaunchKernelGGL(block_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, nb, t->hist.p, 0, 1, nullptr, n_group_dev);
+    hipLaunchKernelGGL(group_write_kernel, dim3(nb), dim3(kSpanTile), 0, st, n, t->head.p, t->hist.p, n_group_dev,
+                       t->group.p, t->i_off.p);
     if (hipGetLastError() != hipSuccess) return fail(set_error(SPHK_E_DEVICE, "dtree: build failed"));
+    int64_t groups = 0;
+    if (int rc = read1(st, n_group_dev, &groups)) return fail(rc);
+    const int ng = (int)groups;
     t->n_walk = ng;
     return SPHK_OK;
 }
@@ -1438,26 +1561,16 @@ int sphk_dtree_list_symmetry(sphk_dtree *t, const double *h)
 {
     if (!t || !h) return set_error(SPHK_E_ARG, "dtree symmetry: null argument");
     if (t->n_walk <= 0) return set_error(SPHK_E_STATE, "dtree symmetry: no tree built");
-    const size_t nn = (size_t)t->n_node;
-    if (t->olo.reserve(3 * nn, false, t->st) != hipSuccess || t->ohi.reserve(3 * nn, false, t->st) != hipSuccess)
+    if (t->orec.reserve((size_t)t->n_node, false, t->st) != hipSuccess)
         return set_error(SPHK_E_DEVICE, "dtree symmetry: allocation failed");
-    // the obox arrays use the same [3][cap] stride as the tight boxes
-    const size_t C = t->box_lo.cap / 3;
-    if (t->olo.cap < 3 * C || t->ohi.cap < 3 * C) {
-        t->olo.release();
-        t->ohi.release();
-        if (t->olo.reserve(3 * C, false, t->st) != hipSuccess || t->ohi.reserve(3 * C, false, t->st) != hipSuccess)
-            return set_error(SPHK_E_DEVICE, "dtree symmetry: allocation failed");
-    }
-    for (int L = (int)t->level_start.size() - 2; L >= 0; L--) {
+    const TopLevels top = top_levels(t);
+    for (int L = (int)t->level_start.size() - 2; L >= top.levels; L--) {
         const int a0 = t->level_start[L], na = t->level_start[L + 1] - a0;
-        hipLaunchKernelGGL(obox_kernel, dim3(grid(na)), dim3(kBlock), 0, t->st, a0, na, t->nodes(), t->olo.p,
-                           t->ohi.p, C, t->x.p, t->y.p, t->z.p, h);
+        hipLaunchKernelGGL(obox_kernel, dim3(grid(na)), dim3(kBlock), 0, t->st, a0, na, t->nodes(), t->orec.p, t->x.p,
+                           t->y.p, t->z.p, h);
     }
-    if (t->orec.reserve(nn, false, t->st) != hipSuccess)
-        return set_error(SPHK_E_DEVICE, "dtree symmetry: allocation failed");
-    hipLaunchKernelGGL(pack_obox_kernel, dim3(grid((int)nn)), dim3(kBlock), 0, t->st, (int)nn, t->olo.p, t->ohi.p, C,
-                       t->orec.p);
+    hipLaunchKernelGGL(obox_top_kernel, dim3(1), dim3(kTopThreads), 0, t->st, top, t->nodes(), t->orec.p, t->x.p,
+                       t->y.p, t->z.p, h);
     SPHK_TRY(hipGetLastError());
     return build_list<1>(t, h, 0.);
 }

@@ -1,0 +1,51 @@
+"""The device tree at the edges of its construction: trees of one node, sizes
+around the blocks of 1024 particles that nodes are counted in, leaves larger
+than the window compared in LDS, and coincident particles (cells that cannot
+be split at the deepest level).  Everything must equal the host tree's."""
+import numpy as np
+import pytest
+import torch
+
+from research_codes_amd.tree import DeviceTree, HostTree, morton_order
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(kind, n, rng):
+    x = rng.random((3, n))
+    if kind == "clumped":                  # a quarter of them at three places
+        for k in range(3):
+            x[:, k * n // 12:(k + 1) * n // 12] = rng.random((3, 1))
+    if kind == "line":                     # one octant pair per level: long chains of single children
+        x = np.stack([0.5 ** (1.0 + 18.0 * rng.random(n))] * 3)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["uniform", "clumped", "line"])
+@pytest.mark.parametrize("n,n_leaf,n_group", [(1, 8, 16), (2, 1, 1), (8, 8, 16), (9, 8, 8), (1023, 8, 16), (1024, 8, 32),
+                                              (1025, 8, 64), (2049, 1, 8), (3000, 512, 600), (3000, 513, 16),
+                                              (5000, 8, 7)])
+def test_tree_equals_host(kind, n, n_leaf, n_group):
+    rng = np.random.default_rng(n + n_leaf)
+    x, y, z = _points(kind, n, rng)
+    perm = morton_order(x, y, z)
+    x, y, z = (np.ascontiguousarray(a[perm]) for a in (x, y, z))
+    m, eps2, h = rng.uniform(0.5, 1.5, n), rng.uniform(1e-5, 1e-3, n), rng.uniform(0.02, 0.3, n)
+    d = lambda a: torch.from_numpy(a).cuda()   # noqa: E731
+    ht = HostTree(x, y, z, m, eps2, n_leaf, n_group)
+    dt = DeviceTree(*map(d, (x, y, z, m, eps2)), n_leaf, n_group)
+    try:
+        for again in range(2):             # built, and built again into the same buffers
+            assert dt.n_node == ht.n_node and dt.n_walk == ht.n_walk
+            assert np.array_equal(dt.i_off.cpu().numpy(), ht.i_off)
+            for k, v in ht.moments().items():
+                assert np.array_equal(dt.moments()[k].cpu().numpy(), v), k
+            for name, hl, dl in (("gather", ht.gather(h), dt.gather(d(h))), ("symmetry", ht.symmetry(h), dt.symmetry(d(h))),
+                                 ("long", ht.long(0.5), dt.long(0.5))):
+                for a, b in zip(hl, dl):
+                    assert np.array_equal(a, b.cpu().numpy()), (name, again)
+            dt._src = None
+            dt.rebuild(*map(d, (x, y, z, m, eps2)), n_leaf, n_group)
+    finally:
+        ht.close()
+        dt.close()
