@@ -16,11 +16,13 @@
 //      host.
 //   4. Groups: a node is a walk if it holds <= n_group particles (or is a
 //      leaf) and its parent holds more; walks are ordered by first particle.
-//   5. Lists: the host's depth-first traversal of each walk, 8 lanes per
+//   5. Lists, the host's element for element, each in one pass into a room
+//      per walk.  Long list: the host's depth-first traversal, 8 lanes per
 //      walk (the children of one opened node at a time, a stack of pending
-//      entries in LDS), run twice: count, then fill at scanned offsets; the
-//      output is the host's, element for element.  The short-range lists test
-//      each reached leaf's particles for exact membership on the way.
+//      entries in LDS).  Short-range lists: one wave per walk, up to 8 nodes
+//      opened at a time, the reached leaves' particles tested for exact
+//      membership on the way.  A walk that overflows its room or stack sends
+//      the build through count and fill walks at scanned offsets.
 #include <hip/hip_runtime.h>
 
 #include <cstring>   // rocPRIM's iterator headers use memset without including it
@@ -412,8 +414,8 @@ struct alignas(64) MacRec {     // long walk
     double mx, my, mz, mm, len;
     int32_t child, nchild, begin, end;
 };
-struct alignas(64) OboxRec {    // symmetry walk: box of the nodes' particle spheres
-    double lo[3], hi[3];
+struct alignas(64) OboxRec {    // symmetry walk: box of the nodes' particle spheres, largest |h|
+    double lo[3], hi[3], h;
 };
 
 // ---- boxes and monopoles, one level at a time (bottom-up) ------------------
@@ -526,10 +528,11 @@ __device__ __forceinline__ void node_obox(int a, const NodeArrays &nd, OboxRec *
                                           const double *__restrict__ h)
 {
     const double inf = __builtin_inf();
-    double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+    double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf}, hm = 0.;
     if (nd.child[a] < 0) {
         for (int i = nd.begin[a]; i < nd.end[a]; i++) {
             const double p[3] = {x[i], y[i], z[i]};
+            hm = fmax(hm, fabs(h[i]));
             for (int d = 0; d < 3; d++) {
                 lo[d] = fmin(lo[d], p[d] - h[i]);
                 hi[d] = fmax(hi[d], p[d] + h[i]);
@@ -538,13 +541,14 @@ __device__ __forceinline__ void node_obox(int a, const NodeArrays &nd, OboxRec *
     } else {
         for (int c = nd.child[a]; c < nd.child[a] + nd.nchild[a]; c++) {
             const OboxRec o = orr[c];
+            hm = fmax(hm, o.h);
             for (int d = 0; d < 3; d++) {
                 lo[d] = fmin(lo[d], o.lo[d]);
                 hi[d] = fmax(hi[d], o.hi[d]);
             }
         }
     }
-    orr[a] = OboxRec{{lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}};
+    orr[a] = OboxRec{{lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}, hm};
 }
 
 __global__ __launch_bounds__(kBlock) void obox_kernel(int a0, int na, NodeArrays nd, OboxRec *orr,
@@ -619,6 +623,17 @@ __global__ __launch_bounds__(kSpanTile) void group_write_kernel(int n, const int
 }
 
 // ---- lists -------------------------------------------------------------------
+// Walk of workgroup b: chunks of 64 consecutive walks dealt to the 8 XCDs in
+// turn, so that an XCD's L2 serves the nodes and particles neighbours share.
+__device__ __forceinline__ int xcd_chunk(int b, int n)
+{
+    constexpr int kX = 8, kC = 64;
+    const int n_full = n / (kX * kC) * (kX * kC);
+    if (b >= n_full) return b;
+    const int x = b % kX, k = b / kX;
+    return ((k / kC) * kX + x) * kC + k % kC;
+}
+
 struct TreeView {
     NodeArrays nd;
     Moments mo;
@@ -637,7 +652,8 @@ __device__ __forceinline__ bool box_overlaps(const double (&alo)[3], const doubl
     return true;
 }
 
-// Box of the i search spheres of each walk (gather: rs, symmetry: h).
+// Box of the i search spheres of each walk (gather: rs, symmetry: h) and the
+// largest |r| (rows 0-5 and 6 of wb).
 __global__ __launch_bounds__(kBlock) void walk_box_kernel(int ng, const int32_t *__restrict__ i_off,
                                                           const double *__restrict__ x,
                                                           const double *__restrict__ y,
@@ -647,9 +663,10 @@ __global__ __launch_bounds__(kBlock) void walk_box_kernel(int ng, const int32_t 
     const int g = blockIdx.x * kBlock + threadIdx.x;
     if (g >= ng) return;
     const double inf = __builtin_inf();
-    double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+    double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf}, rm = 0.;
     for (int i = i_off[g]; i < i_off[g + 1]; i++) {
         const double p[3] = {x[i], y[i], z[i]};
+        rm = fmax(rm, fabs(r[i]));
         for (int d = 0; d < 3; d++) {
             lo[d] = fmin(lo[d], p[d] - r[i]);
             hi[d] = fmax(hi[d], p[d] + r[i]);
@@ -659,6 +676,7 @@ __global__ __launch_bounds__(kBlock) void walk_box_kernel(int ng, const int32_t 
         wb[d * ng + g] = lo[d];
         wb[(3 + d) * ng + g] = hi[d];
     }
+    wb[6 * ng + g] = rm;
 }
 
 // What the depth-first walk does at node a: skip it (pruned, or massless for
@@ -790,12 +808,13 @@ __device__ __forceinline__ bool member(const TreeView &t, const double *__restri
 // The particles of the leaves reached into jout (MODE 0 gather, 1 symmetry:
 // the candidates of the short-range lists), and for MODE 2 (long) the SPJ
 // nodes into sout.  FILL 0: the walk's counts go to cj/cs.  FILL 1: written
-// from the walk's offsets oj/os.  FILL 2: written into rooms of `room`
-// (jout) and `room_s` (sout) entries per walk, walk g's from g * room and
-// g * room_s; short lists: the count to cj and the room's offset to cs;
-// long list: the counts to cj and cs.  Bit 2 (4) of err is set if a walk
+// from the walk's offsets oj/os.  FILL 2 (long list): written into rooms of
+// `room` (jout) and `room_s` (sout) entries per walk, walk g's from g * room
+// and g * room_s, the counts to cj and cs.  Bit 2 (4) of err is set if a walk
 // does not fit its jout (sout) room: entries past it are not written and
 // its count is the room's.
+// The short-range lists come here only when near_list_kernel's stack or rooms
+// overflowed.
 // Bit 1 of err is set if a stack of STACK entries would overflow.
 template <int MODE, int FILL, int STACK>
 __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
@@ -806,6 +825,7 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
                                                        int *__restrict__ err, int64_t room = 0, int64_t room_s = 0)
 {
 #pragma clang fp contract(off)
+    static_assert(FILL != 2 || MODE == 2, "rooms are the long list's");
     __shared__ uint2 stk[kListWalks][STACK];
     const int lane = threadIdx.x, sub = lane >> 3, c = lane & 7;
     const int g = blockIdx.x * kListWalks + sub;
@@ -830,7 +850,7 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
         }
         if (FILL == 2) {
             j0 = (int64_t)g * room;
-            if (MODE == 2) s0 = (int64_t)g * room_s;
+            s0 = (int64_t)g * room_s;
         }
     }
     // emit the entries (w0, w1) of the lanes with em set, in lane order
@@ -913,12 +933,9 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
     }
     if (FILL == 2 && live && c == 0) {
         cj[g] = nj < room ? nj : room;   // what the room holds (all of it unless err bit 2)
-        if (MODE == 2)
-            cs[g] = ns < room_s ? ns : room_s;
-        else
-            cs[g] = j0;
+        cs[g] = ns < room_s ? ns : room_s;
         if (nj > room) atomicOr(err, 2);
-        if (MODE == 2 && ns > room_s) atomicOr(err, 4);
+        if (ns > room_s) atomicOr(err, 4);
     }
 }
 
@@ -986,6 +1003,207 @@ __global__ __launch_bounds__(64) void member_kernel(int ng, TreeView t, const do
     if (lane == 0) cnt[g] = count;
 }
 
+// ---- short-range lists in one pass: one wave per walk ------------------------
+// The walk of the tree and the member test of a gather (MODE 0) or symmetry
+// (MODE 1) list together.  The wave keeps the walk's pending entries in LDS in
+// preorder, the next one on top.  A step looks at the top 64 entries: leaves
+// on top are turned into candidates; otherwise up to 8 of the nodes among them
+// are opened at once, 8 lanes each, and the entries from the top to the last
+// opened one are written back with every opened node replaced by its kept
+// children.  The order stays preorder, so candidates come in the host's order;
+// 256 or more of them are tested together (positions of four per lane loaded
+// before any test) and the members written to the walk's room.
+//
+// One wave per walk because the walks differ: with 8 lanes per walk and 8
+// walks per wave the kernel waited for a few walks in the outskirts that open
+// nodes one after the other (VALU issue 16 %, 1.8 waves per SIMD).
+//
+// A node is skipped if no particle of it can be a member: its tight box must
+// meet the box of the walk's spheres (or its own spheres' box the walk's), as
+// in the host's walk, and must lie within the largest radius that matters of
+// the walk's box: the walk's largest r or, for symmetry, the node's.  The
+// distance test (half the candidates: a sphere's share of its cube) leaves
+// out only particles that the member test refuses, with 1e-9 to spare for
+// rounding, so the lists do not change.
+constexpr int kNearStack = 384;    // entries; a walk that needs more sets bit 1 of err
+constexpr int kNearCand = 512;
+constexpr int kNearBatch = 256;    // candidates tested together
+constexpr int kNearLeaves = 16;    // leaves on top that are worth taking before the next nodes are opened
+
+template <int MODE>
+__global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
+                                                       const double *__restrict__ r, int64_t *__restrict__ cnt,
+                                                       int32_t *__restrict__ out, int64_t room, int n_si,
+                                                       int *__restrict__ err)
+{
+#pragma clang fp contract(off)
+    __shared__ uint2 stk[kNearStack];
+    __shared__ int32_t cand[kNearCand];
+    __shared__ uint32_t s_first[8], s_count[8], s_place[8];
+    extern __shared__ double4 si[];
+    if ((int)blockIdx.x >= ng) return;
+    const int g = xcd_chunk(blockIdx.x, ng), lane = threadIdx.x;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const size_t C = t.mo.cap;
+    const int ib = t.i_off[g], ni = t.i_off[g + 1] - ib;
+    const int nl = ni < n_si ? ni : n_si;
+    for (int q = lane; q < nl; q += 64)
+        si[q] = make_double4(t.x[ib + q], t.y[ib + q], t.z[ib + q], r[ib + q]);
+    const int gn = t.group[g];
+    double olo[3], ohi[3], glo[3], ghi[3];
+    for (int d = 0; d < 3; d++) {
+        olo[d] = wb[d * ng + g];
+        ohi[d] = wb[(3 + d) * ng + g];
+        glo[d] = t.mo.lo[d * C + gn];
+        ghi[d] = t.mo.hi[d * C + gn];
+    }
+    const double rm = wb[6 * ng + g];
+    int32_t *const room_out = out + (int64_t)g * room;
+    int64_t count = 0;
+    int nc = 0;          // candidates waiting
+
+    // node a: its entry (0 type if skipped)
+    auto look = [&](int a) {
+        const BoxRec b = t.br[a];
+        OboxRec o{};
+        if (MODE == 1) o = t.orr[a];
+        uint2 e = make_uint2(0u, 0u);
+        const bool near = box_overlaps(olo, ohi, b.lo, b.hi) || (MODE == 1 && box_overlaps(glo, ghi, o.lo, o.hi));
+        double s = 0.;
+        for (int d = 0; d < 3; d++) {
+            const double e1 = glo[d] - b.hi[d], e2 = b.lo[d] - ghi[d];
+            const double m = e1 > e2 ? e1 : e2;
+            s += m > 0. ? m * m : 0.;
+        }
+        const double R = (MODE == 1 && o.h > rm ? o.h : rm) * (1. + 1e-9);
+        if (near && !(s > R * R)) {
+            e = b.child < 0 ? make_uint2((uint32_t)b.begin, kTyLeaf | (uint32_t)(b.end - b.begin))
+                            : make_uint2((uint32_t)b.child, kTyOpen | (uint32_t)b.nchild);
+        }
+        return e;
+    };
+    // the members among candidates, n (<= 64 * U) of them, get(k) the k-th
+    auto test = [&](auto &&get, int n) {
+        int j[kMemberU];
+        double p[kMemberU][3], hj[kMemberU];
+#pragma unroll
+        for (int u = 0; u < kMemberU; u++) {
+            const int k = 64 * u + lane;
+            j[u] = k < n ? get(k) : -1;
+            const int jj = j[u] < 0 ? ib : j[u];
+            p[u][0] = t.x[jj];
+            p[u][1] = t.y[jj];
+            p[u][2] = t.z[jj];
+            hj[u] = MODE == 1 ? r[jj] : 0.;
+        }
+#pragma unroll
+        for (int u = 0; u < kMemberU; u++) {
+            if (64 * u >= n) break;
+            const bool acc = j[u] >= 0 && member<MODE>(t, r, p[u], hj[u], ib, ni, nl, si, olo, ohi, glo, ghi);
+            const uint64_t bal = __ballot(acc);
+            const int64_t at = count + __popcll(bal & below);
+            if (acc && at < room) room_out[at] = j[u];
+            count += __popcll(bal);
+        }
+    };
+    // candidates waiting: whole batches, or (all) every one
+    auto drain = [&](bool all) {
+        __syncthreads();
+        int at = 0;
+        while (nc - at >= (all ? 1 : kNearBatch)) {
+            const int n = min(kNearBatch, nc - at);
+            test([&](int k) { return cand[at + k]; }, n);
+            at += n;
+        }
+        int32_t keep[(kNearBatch + 63) / 64];
+        const int left = nc - at;
+#pragma unroll
+        for (int u = 0; u < (kNearBatch + 63) / 64; u++)
+            keep[u] = at && 64 * u + lane < left ? cand[at + 64 * u + lane] : 0;
+        __syncthreads();
+        if (at)
+#pragma unroll
+            for (int u = 0; u < (kNearBatch + 63) / 64; u++)
+                if (64 * u + lane < left) cand[64 * u + lane] = keep[u];
+        nc = left;
+    };
+
+    int sp = 0;
+    {
+        const uint2 e = look(0);
+        if (lane == 0) stk[0] = e;
+        sp = __builtin_amdgcn_readfirstlane(e.y) != 0u ? 1 : 0;
+    }
+    bool bad = false;
+    while (sp > 0) {
+        __syncthreads();   // the entries of the last step are written
+        const int W = sp < 64 ? sp : 64;
+        const uint2 e = lane < W ? stk[sp - 1 - lane] : make_uint2(0u, 0u);
+        const uint64_t ob = __ballot((e.y & kTyMask) == kTyOpen);
+        const int P = ob ? __builtin_ctzll(ob) : W;    // leaves on top
+        if (!ob || P >= kNearLeaves) {
+            const int sz = lane < P ? (int)(e.y & kCountMask) : 0;
+            int incl = sz;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int u = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += u;
+            }
+            // the leading leaves that fit (nc < kNearBatch here)
+            const int take = __popcll(__ballot(lane < P && incl <= kNearCand - nc));
+            if (take > 0) {
+                if (lane < take)
+                    for (int q = 0; q < sz; q++) cand[nc + incl - sz + q] = (int32_t)e.x + q;
+                nc += __shfl(incl, take - 1, 64);
+                sp -= take;
+                if (nc >= kNearBatch) drain(false);
+            } else {   // one leaf of more particles than fit: from its range
+                drain(true);
+                const int b = __shfl((int)e.x, 0, 64), n = __shfl(sz, 0, 64);
+                for (int c = 0; c < n; c += kNearBatch) test([&](int k) { return b + c + k; }, min(kNearBatch, n - c));
+                sp -= 1;
+            }
+            continue;
+        }
+        // open the first (at most 8) nodes of the window
+        const int rank = __popcll(ob & below);
+        const bool sel = ((ob >> lane) & 1) && rank < 8;
+        const uint64_t sb = __ballot(sel);
+        const int n_open = __popcll(sb), last = 63 - __builtin_clzll(sb);
+        if (sel) {
+            s_first[rank] = e.x;
+            s_count[rank] = e.y & kCountMask;
+            s_place[rank] = (uint32_t)lane;
+        }
+        __syncthreads();
+        const int k = lane >> 3, c = lane & 7;
+        uint2 w = make_uint2(0u, 0u);
+        int place = 0;
+        if (k < n_open) {
+            place = (int)s_place[k];
+            if (c < (int)s_count[k]) w = look((int)s_first[k] + c);
+        }
+        const uint64_t km = __ballot(w.y != 0u);
+        const int T = last + 1 - n_open + __popcll(km), base = sp - 1 - last;
+        if (base + T > kNearStack) {
+            bad = true;
+            break;
+        }
+        // entry o of the rewritten window goes to stk[base + T - 1 - o]
+        if (lane <= last && !sel) {
+            const int before = __popcll(sb & below);   // <= 7: the last one opened lies behind
+            stk[base + T - 1 - (lane - before + __popcll(km & ((1ull << (8 * before)) - 1ull)))] = e;
+        }
+        if (w.y != 0u) stk[base + T - 1 - (place - k + __popcll(km & below))] = w;
+        sp = base + T;
+    }
+    drain(true);
+    if (lane == 0) {
+        cnt[g] = count < room ? count : room;
+        if (bad) atomicOr(err, 1);
+        if (count > room) atomicOr(err, 2);
+    }
+}
+
 // Members of each walk, from its stretch of the candidate scratch to its
 // place in the list.
 __global__ __launch_bounds__(64) void member_copy_kernel(int ng, const int64_t *__restrict__ soff,
@@ -1026,7 +1244,8 @@ __global__ void offsets_kernel(int ng, const int64_t *__restrict__ scan, const i
 
 }  // namespace
 
-constexpr int64_t kRoomStart = 2048;          // candidates (SPJ nodes) per walk
+constexpr int64_t kRoomNearStart = 1024;      // short-range list entries per walk
+constexpr int64_t kRoomStart = 2048;          // SPJ nodes per walk
 constexpr int64_t kRoomLongStart = 8192;      // long-list particles per walk
 constexpr int64_t kRoomMax = 1 << 16;
 constexpr int64_t kRoomMaxEntries = 1ll << 31;  // scratch entries (8 GiB)
@@ -1053,10 +1272,10 @@ struct sphk_dtree {
     DArr<int> err;
     DArr<char> scratch;
     DLists lists[3];
-    // per-walk rooms of the one-walk list builds (gather and symmetry
-    // candidates; long-list EPJ and SPJ entries), doubled after a build that
+    // per-walk rooms of the one-pass list builds (gather and symmetry
+    // members; long-list EPJ and SPJ entries), doubled after a build that
     // overflowed them
-    int64_t room[2] = {kRoomStart, kRoomStart};
+    int64_t room[2] = {kRoomNearStart, kRoomNearStart};
     int64_t room_long[2] = {kRoomLongStart, kRoomStart};
     DArr<int32_t> sscr;   // SPJ room of the long list
 
@@ -1183,12 +1402,13 @@ int pack_list(sphk_dtree *t, int kind, int32_t *j_idx, int32_t *s_idx)
     return SPHK_OK;
 }
 
-// Interaction lists of every walk.  Long list: the tree walk (count, scan,
-// fill) gives each walk's EPJ particles and SPJ nodes.  Short-range lists
-// (gather: r = rs, symmetry: r = H): the tree walk (count, scan, fill)
-// writes the particles of the leaves reached into the walk's stretch of a
-// scratch array, member_kernel keeps the members there, and they are copied
-// to their offsets in the list.
+// Interaction lists of every walk: one pass into rooms, and if a room or a
+// stack overflowed the counted build.  That is, for the long list, the tree
+// walk run as count, scan and fill; for the short-range lists (gather: r =
+// rs, symmetry: r = H) the tree walk (count, scan, fill) writes the particles
+// of the leaves reached into the walk's stretch of a scratch array,
+// member_kernel keeps the members there, and they are copied to their offsets
+// in the list.
 template <int MODE>
 int build_list(sphk_dtree *t, const double *r, double inv_t2)
 {
@@ -1211,7 +1431,7 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
     if (MODE == 2) SPHK_TRY(L.s_off.reserve(ng + 1, false, t->st));
     SPHK_TRY(hipMemsetAsync(t->err.p, 0, sizeof(int), t->st));
     if (MODE != 2) {
-        SPHK_TRY(t->wbox.reserve(6 * (size_t)ng, false, t->st));
+        SPHK_TRY(t->wbox.reserve(7 * (size_t)ng, false, t->st));
         hipLaunchKernelGGL(walk_box_kernel, dim3(grid(ng)), dim3(kBlock), 0, t->st, ng, t->i_off.p, t->x.p,
                            t->y.p, t->z.p, r, t->wbox.p);
     }
@@ -1220,16 +1440,14 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
     const double *wb = MODE == 2 ? nullptr : t->wbox.p;
     const dim3 lg((unsigned)((ng + kListWalks - 1) / kListWalks)), lb(64);
     if constexpr (MODE != 2) {
-        // one walk into a room per walk: no count walk, one host read.  If a
-        // walk overflows its room or the small stack, the counted build below
-        // runs instead (and later builds get twice the room).
+        // one pass into a room per walk: no count walk, one host read.  If a
+        // walk overflows its room or the stack, the counted build below runs
+        // instead (and later builds get twice the room).
         int64_t &room = t->room[MODE];
         if ((int64_t)ng * room <= kRoomMaxEntries) {
             SPHK_TRY(t->mscr.reserve((size_t)ng * (size_t)room, false, t->st));
-            hipLaunchKernelGGL((walk_list_kernel<MODE, 2, kListStackSmall>), lg, lb, 0, t->st, ng, v, wb, r, inv_t2,
-                               t->i64a.p, t->i64c.p, nullptr, nullptr, t->mscr.p, nullptr, t->err.p, room);
-            hipLaunchKernelGGL((member_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
-                               r, t->i64c.p, t->i64a.p, t->mscr.p, t->i64b.p, n_si);
+            hipLaunchKernelGGL((near_list_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
+                               r, t->i64b.p, t->mscr.p, room, n_si, t->err.p);
             SPHK_TRY(hipGetLastError());
             if (int rc = walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr)) return rc;
             int64_t tot1[2] = {0, 0};
