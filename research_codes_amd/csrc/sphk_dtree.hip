@@ -508,7 +508,7 @@ struct TopLevels {
     int ls[kMaxLevel + 2];
 };
 constexpr int kTopThreads = 1024;
-constexpr int kTopNodes = 4096;   // levels are top while no level is wider than this
+constexpr int kTopNodes = 512;   // levels are top while no level is wider than this
 
 __global__ __launch_bounds__(kTopThreads) void moments_top_kernel(TopLevels tl, NodeArrays nd, Moments mo,
                                                                   BoxRec *br, MacRec *mr, const double *x,
@@ -808,13 +808,8 @@ __device__ __forceinline__ bool member(const TreeView &t, const double *__restri
 // The particles of the leaves reached into jout (MODE 0 gather, 1 symmetry:
 // the candidates of the short-range lists), and for MODE 2 (long) the SPJ
 // nodes into sout.  FILL 0: the walk's counts go to cj/cs.  FILL 1: written
-// from the walk's offsets oj/os.  FILL 2 (long list): written into rooms of
-// `room` (jout) and `room_s` (sout) entries per walk, walk g's from g * room
-// and g * room_s, the counts to cj and cs.  Bit 2 (4) of err is set if a walk
-// does not fit its jout (sout) room: entries past it are not written and
-// its count is the room's.
-// The short-range lists come here only when near_list_kernel's stack or rooms
-// overflowed.
+// from the walk's offsets oj/os.  Runs only when the stack or a room of
+// room_list_kernel overflowed.
 // Bit 1 of err is set if a stack of STACK entries would overflow.
 template <int MODE, int FILL, int STACK>
 __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
@@ -822,10 +817,9 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
                                                        int64_t *__restrict__ cj, int64_t *__restrict__ cs,
                                                        const int64_t *__restrict__ oj, const int64_t *__restrict__ os,
                                                        int32_t *__restrict__ jout, int32_t *__restrict__ sout,
-                                                       int *__restrict__ err, int64_t room = 0, int64_t room_s = 0)
+                                                       int *__restrict__ err)
 {
 #pragma clang fp contract(off)
-    static_assert(FILL != 2 || MODE == 2, "rooms are the long list's");
     __shared__ uint2 stk[kListWalks][STACK];
     const int lane = threadIdx.x, sub = lane >> 3, c = lane & 7;
     const int g = blockIdx.x * kListWalks + sub;
@@ -848,10 +842,6 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
             j0 = oj[g];
             if (MODE == 2) s0 = os[g];
         }
-        if (FILL == 2) {
-            j0 = (int64_t)g * room;
-            s0 = (int64_t)g * room_s;
-        }
     }
     // emit the entries (w0, w1) of the lanes with em set, in lane order
     auto emit = [&](bool em, uint32_t w0, uint32_t w1) {
@@ -860,7 +850,6 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
             const bool is_s = em && ty == kTySpj;
             const unsigned sb = walk_bits(is_s, lane);
             if (FILL == 1 && is_s) sout[s0 + ns + __popc(sb & below)] = (int32_t)w0;
-        if (FILL == 2 && is_s && ns + __popc(sb & below) < room_s) sout[s0 + ns + __popc(sb & below)] = (int32_t)w0;
             ns += __popc(sb);
         }
         const bool is_l = em && ty == kTyLeaf;
@@ -869,11 +858,6 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
         if (FILL == 1 && is_l) {
             const int64_t p0 = j0 + nj + incl - sz;
             for (int q = 0; q < sz; q++) jout[p0 + q] = (int32_t)w0 + q;
-        }
-        if (FILL == 2 && is_l) {
-            const int64_t p0 = nj + incl - sz;   // within the room
-            for (int q = 0; q < sz; q++)
-                if (p0 + q < room) jout[j0 + p0 + q] = (int32_t)w0 + q;
         }
         nj += __shfl(incl, 7, 8);
     };
@@ -930,12 +914,6 @@ __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const
     if (FILL == 0 && live && c == 0) {
         cj[g] = nj;
         if (MODE == 2) cs[g] = ns;
-    }
-    if (FILL == 2 && live && c == 0) {
-        cj[g] = nj < room ? nj : room;   // what the room holds (all of it unless err bit 2)
-        cs[g] = ns < room_s ? ns : room_s;
-        if (nj > room) atomicOr(err, 2);
-        if (ns > room_s) atomicOr(err, 4);
     }
 }
 
@@ -1003,42 +981,50 @@ __global__ __launch_bounds__(64) void member_kernel(int ng, TreeView t, const do
     if (lane == 0) cnt[g] = count;
 }
 
-// ---- short-range lists in one pass: one wave per walk ------------------------
-// The walk of the tree and the member test of a gather (MODE 0) or symmetry
-// (MODE 1) list together.  The wave keeps the walk's pending entries in LDS in
-// preorder, the next one on top.  A step looks at the top 64 entries: leaves
-// on top are turned into candidates; otherwise up to 8 of the nodes among them
-// are opened at once, 8 lanes each, and the entries from the top to the last
-// opened one are written back with every opened node replaced by its kept
-// children.  The order stays preorder, so candidates come in the host's order;
-// 256 or more of them are tested together (positions of four per lane loaded
-// before any test) and the members written to the walk's room.
+// ---- lists in one pass into rooms: one wave per walk --------------------------
+// MODE 0 gather, 1 symmetry: the walk of the tree and the member test
+// together; MODE 2 the long list.  The wave keeps the walk's pending entries
+// in LDS in preorder, the next one on top.  A step looks at the top 64
+// entries: finished ones on top (leaves, SPJ nodes) are taken off; otherwise
+// up to 8 of the nodes to open among them are opened at once, 8 lanes each,
+// and the entries from the top to the last opened one are written back with
+// every opened node replaced by its kept children.  The order stays preorder,
+// so entries come off in the host's order.  Long list: SPJ nodes and the
+// leaves' particles go to the walk's two rooms.  Short-range lists: the
+// leaves' particles are candidates; 256 or more of them are tested together
+// (positions of four per lane loaded before any test) and the members written
+// to the walk's room.
 //
 // One wave per walk because the walks differ: with 8 lanes per walk and 8
-// walks per wave the kernel waited for a few walks in the outskirts that open
-// nodes one after the other (VALU issue 16 %, 1.8 waves per SIMD).
+// walks per wave the short-range lists waited for a few walks in the
+// outskirts that open nodes one after the other (VALU issue 16 %, 1.8 waves
+// per SIMD), and the long list, issue-bound, paid two emissions per 8 nodes
+// looked at.  10^6 particles, before and now: gather and symmetry with their
+// member kernels 2.0 and 1.85 ms, 0.79 and 0.80; long 1.42, 0.95.
 //
-// A node is skipped if no particle of it can be a member: its tight box must
-// meet the box of the walk's spheres (or its own spheres' box the walk's), as
-// in the host's walk, and must lie within the largest radius that matters of
-// the walk's box: the walk's largest r or, for symmetry, the node's.  The
-// distance test (half the candidates: a sphere's share of its cube) leaves
-// out only particles that the member test refuses, with 1e-9 to spare for
-// rounding, so the lists do not change.
-constexpr int kNearStack = 384;    // entries; a walk that needs more sets bit 1 of err
-constexpr int kNearCand = 512;
-constexpr int kNearBatch = 256;    // candidates tested together
-constexpr int kNearLeaves = 16;    // leaves on top that are worth taking before the next nodes are opened
+// A node of a short-range list is skipped if no particle of it can be a
+// member: its tight box must meet the box of the walk's spheres (or its own
+// spheres' box the walk's), as in the host's walk, and must lie within the
+// largest radius that matters of the walk's box: the walk's largest r or, for
+// symmetry, the node's.  The distance test (half the candidates: a sphere's
+// share of its cube) leaves out only particles that the member test refuses,
+// with 1e-9 to spare for rounding, so the lists do not change.
+constexpr int kRoomStack = 384;    // entries; a walk that needs more sets bit 1 of err
+constexpr int kRoomCand = 512;
+constexpr int kRoomBatch = 256;    // candidates tested together
+constexpr int kRoomTake = 32;      // finished entries on top that are worth taking before the next nodes are opened
 
 template <int MODE>
-__global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
-                                                       const double *__restrict__ r, int64_t *__restrict__ cnt,
-                                                       int32_t *__restrict__ out, int64_t room, int n_si,
+__global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
+                                                       const double *__restrict__ r, double inv_t2,
+                                                       int64_t *__restrict__ cnt, int32_t *__restrict__ out,
+                                                       int64_t room, int64_t *__restrict__ cnt_s,
+                                                       int32_t *__restrict__ out_s, int64_t room_s, int n_si,
                                                        int *__restrict__ err)
 {
 #pragma clang fp contract(off)
-    __shared__ uint2 stk[kNearStack];
-    __shared__ int32_t cand[kNearCand];
+    __shared__ uint2 stk[kRoomStack];
+    __shared__ int32_t cand[MODE == 2 ? 1 : kRoomCand];
     __shared__ uint32_t s_first[8], s_count[8], s_place[8];
     extern __shared__ double4 si[];
     if ((int)blockIdx.x >= ng) return;
@@ -1047,23 +1033,32 @@ __global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const
     const size_t C = t.mo.cap;
     const int ib = t.i_off[g], ni = t.i_off[g + 1] - ib;
     const int nl = ni < n_si ? ni : n_si;
-    for (int q = lane; q < nl; q += 64)
+    if (MODE != 2) for (int q = lane; q < nl; q += 64)
         si[q] = make_double4(t.x[ib + q], t.y[ib + q], t.z[ib + q], r[ib + q]);
     const int gn = t.group[g];
     double olo[3], ohi[3], glo[3], ghi[3];
     for (int d = 0; d < 3; d++) {
-        olo[d] = wb[d * ng + g];
-        ohi[d] = wb[(3 + d) * ng + g];
+        olo[d] = MODE == 2 ? 0. : wb[d * ng + g];
+        ohi[d] = MODE == 2 ? 0. : wb[(3 + d) * ng + g];
         glo[d] = t.mo.lo[d * C + gn];
         ghi[d] = t.mo.hi[d * C + gn];
     }
-    const double rm = wb[6 * ng + g];
+    const double rm = MODE == 2 ? 0. : wb[6 * ng + g];
     int32_t *const room_out = out + (int64_t)g * room;
-    int64_t count = 0;
+    int32_t *const room_spj = MODE == 2 ? out_s + (int64_t)g * room_s : nullptr;
+    int64_t count = 0, spj = 0;
     int nc = 0;          // candidates waiting
 
     // node a: its entry (0 type if skipped)
     auto look = [&](int a) {
+        if (MODE == 2) {
+            NodeLinks ln;
+            const Visit v = visit<2>(t, a, olo, ohi, glo, ghi, inv_t2, ln);
+            return v == kSpj    ? make_uint2((uint32_t)a, kTySpj)
+                   : v == kLeaf ? make_uint2((uint32_t)ln.begin, kTyLeaf | (uint32_t)(ln.end - ln.begin))
+                   : v == kOpen ? make_uint2((uint32_t)ln.child, kTyOpen | (uint32_t)ln.nchild)
+                                : make_uint2(0u, 0u);
+        }
         const BoxRec b = t.br[a];
         OboxRec o{};
         if (MODE == 1) o = t.orr[a];
@@ -1110,20 +1105,20 @@ __global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const
     auto drain = [&](bool all) {
         __syncthreads();
         int at = 0;
-        while (nc - at >= (all ? 1 : kNearBatch)) {
-            const int n = min(kNearBatch, nc - at);
+        while (nc - at >= (all ? 1 : kRoomBatch)) {
+            const int n = min(kRoomBatch, nc - at);
             test([&](int k) { return cand[at + k]; }, n);
             at += n;
         }
-        int32_t keep[(kNearBatch + 63) / 64];
+        int32_t keep[(kRoomBatch + 63) / 64];
         const int left = nc - at;
 #pragma unroll
-        for (int u = 0; u < (kNearBatch + 63) / 64; u++)
+        for (int u = 0; u < (kRoomBatch + 63) / 64; u++)
             keep[u] = at && 64 * u + lane < left ? cand[at + 64 * u + lane] : 0;
         __syncthreads();
         if (at)
 #pragma unroll
-            for (int u = 0; u < (kNearBatch + 63) / 64; u++)
+            for (int u = 0; u < (kRoomBatch + 63) / 64; u++)
                 if (64 * u + lane < left) cand[64 * u + lane] = keep[u];
         nc = left;
     };
@@ -1140,26 +1135,45 @@ __global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const
         const int W = sp < 64 ? sp : 64;
         const uint2 e = lane < W ? stk[sp - 1 - lane] : make_uint2(0u, 0u);
         const uint64_t ob = __ballot((e.y & kTyMask) == kTyOpen);
-        const int P = ob ? __builtin_ctzll(ob) : W;    // leaves on top
-        if (!ob || P >= kNearLeaves) {
-            const int sz = lane < P ? (int)(e.y & kCountMask) : 0;
+        const int P = ob ? __builtin_ctzll(ob) : W;    // finished entries on top
+        if (!ob || P >= kRoomTake) {
+            const int sz = lane < P && (e.y & kTyMask) == kTyLeaf ? (int)(e.y & kCountMask) : 0;
+            if (MODE == 2) {
+                const uint64_t sb = __ballot(lane < P && (e.y & kTyMask) == kTySpj);
+                const int64_t at = spj + __popcll(sb & below);
+                if (((sb >> lane) & 1) && at < room_s) room_spj[at] = (int32_t)e.x;
+                spj += __popcll(sb);
+                if (P < 64 ? sb == (1ull << P) - 1ull : sb == ~0ull) {   // no leaf among them
+                    sp -= P;
+                    continue;
+                }
+            }
             int incl = sz;
             for (int d = 1; d < 64; d <<= 1) {
                 const int u = __shfl_up(incl, d, 64);
                 if (lane >= d) incl += u;
             }
-            // the leading leaves that fit (nc < kNearBatch here)
-            const int take = __popcll(__ballot(lane < P && incl <= kNearCand - nc));
+            if (MODE == 2) {
+                for (int q = 0; q < sz; q++) {
+                    const int64_t at = count + incl - sz + q;
+                    if (at < room) room_out[at] = (int32_t)e.x + q;
+                }
+                count += __shfl(incl, 63, 64);
+                sp -= P;
+                continue;
+            }
+            // the leading leaves that fit (nc < kRoomBatch here)
+            const int take = __popcll(__ballot(lane < P && incl <= kRoomCand - nc));
             if (take > 0) {
                 if (lane < take)
                     for (int q = 0; q < sz; q++) cand[nc + incl - sz + q] = (int32_t)e.x + q;
                 nc += __shfl(incl, take - 1, 64);
                 sp -= take;
-                if (nc >= kNearBatch) drain(false);
+                if (nc >= kRoomBatch) drain(false);
             } else {   // one leaf of more particles than fit: from its range
                 drain(true);
                 const int b = __shfl((int)e.x, 0, 64), n = __shfl(sz, 0, 64);
-                for (int c = 0; c < n; c += kNearBatch) test([&](int k) { return b + c + k; }, min(kNearBatch, n - c));
+                for (int c = 0; c < n; c += kRoomBatch) test([&](int k) { return b + c + k; }, min(kRoomBatch, n - c));
                 sp -= 1;
             }
             continue;
@@ -1184,7 +1198,7 @@ __global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const
         }
         const uint64_t km = __ballot(w.y != 0u);
         const int T = last + 1 - n_open + __popcll(km), base = sp - 1 - last;
-        if (base + T > kNearStack) {
+        if (base + T > kRoomStack) {
             bad = true;
             break;
         }
@@ -1196,11 +1210,13 @@ __global__ __launch_bounds__(64) void near_list_kernel(int ng, TreeView t, const
         if (w.y != 0u) stk[base + T - 1 - (place - k + __popcll(km & below))] = w;
         sp = base + T;
     }
-    drain(true);
+    if (MODE != 2) drain(true);
     if (lane == 0) {
-        cnt[g] = count < room ? count : room;
+        cnt[g] = count < room ? count : room;   // what the room holds (all of it unless err bit 2)
+        if (MODE == 2) cnt_s[g] = spj < room_s ? spj : room_s;
         if (bad) atomicOr(err, 1);
         if (count > room) atomicOr(err, 2);
+        if (MODE == 2 && spj > room_s) atomicOr(err, 4);
     }
 }
 
@@ -1446,8 +1462,8 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
         int64_t &room = t->room[MODE];
         if ((int64_t)ng * room <= kRoomMaxEntries) {
             SPHK_TRY(t->mscr.reserve((size_t)ng * (size_t)room, false, t->st));
-            hipLaunchKernelGGL((near_list_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
-                               r, t->i64b.p, t->mscr.p, room, n_si, t->err.p);
+            hipLaunchKernelGGL((room_list_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
+                               r, 0., t->i64b.p, t->mscr.p, room, nullptr, nullptr, 0, n_si, t->err.p);
             SPHK_TRY(hipGetLastError());
             if (int rc = walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr)) return rc;
             int64_t tot1[2] = {0, 0};
@@ -1478,8 +1494,8 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
         if ((int64_t)ng * rj <= kRoomMaxEntries && (int64_t)ng * rsp <= kRoomMaxEntries) {
             SPHK_TRY(t->mscr.reserve((size_t)ng * (size_t)rj, false, t->st));
             SPHK_TRY(t->sscr.reserve((size_t)ng * (size_t)rsp, false, t->st));
-            hipLaunchKernelGGL((walk_list_kernel<2, 2, kListStackSmall>), lg, lb, 0, t->st, ng, v, wb, r, inv_t2,
-                               t->i64a.p, t->i64b.p, nullptr, nullptr, t->mscr.p, t->sscr.p, t->err.p, rj, rsp);
+            hipLaunchKernelGGL((room_list_kernel<2>), dim3(ng), dim3(64), 0, t->st, ng, v, wb, r, inv_t2, t->i64a.p,
+                               t->mscr.p, rj, t->i64b.p, t->sscr.p, rsp, 0, t->err.p);
             SPHK_TRY(hipGetLastError());
             if (int rc = walk_offsets(t, ng, t->i64a.p, t->i64c.p, L.j_off.p, t->i64b.p, t->i64d.p, L.s_off.p))
                 return rc;
