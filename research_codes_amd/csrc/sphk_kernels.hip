@@ -1,7 +1,8 @@
 // sphk_kernels.hip -- gfx950 kernels for the SPH interaction functors.
 //
-// Launch shape (all three kernels): one 64-lane workgroup (one wavefront)
-// per walk.  A walk's i-particles are processed in chunks of <= 64.  Inside a
+// Launch shape (all three kernels): one workgroup per walk, of one 64-lane
+// wavefront (several for the hydro and gravity functors of a launch of few
+// walks, see WaveRule).  A walk's i-particles are processed in chunks of <= 64.  Inside a
 // chunk of ni particles the wave is split into S = floor(64/ni) j-slices:
 // lane l holds i = l mod ni and slice l / ni (lanes beyond S*ni idle), so a
 // walk of 5 particles keeps 60 of 64 lanes busy.  j-entries are staged
@@ -67,7 +68,7 @@ template <bool PERSIST, typename F>
 __device__ __forceinline__ void run_walks(int n_walk, int *queue, F &&walk)
 {
     if (!PERSIST) {
-        if ((int)blockIdx.x < n_walk) walk(xcd_walk(blockIdx.x, n_walk), (int)threadIdx.x);
+        if ((int)blockIdx.x < n_walk) walk(xcd_walk(blockIdx.x, n_walk), (int)(threadIdx.x % kWave));
         return;
     }
     const int x = (int)(blockIdx.x % kXcd);
@@ -87,6 +88,44 @@ __device__ __forceinline__ void run_walks(int n_walk, int *queue, F &&walk)
             atomicExch(queue + kXcd * kQueueStride, 0);
         }
     }
+}
+
+// LDS written by a wave's lanes before, read by them after (one wave's LDS
+// operations complete in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Waves per walk of the hydro and gravity functors.  A launch of few walks
+// leaves SIMDs idle at one wave per walk, and each walk's list is a serial
+// chain of tiles; so NW waves of one workgroup take a walk's tiles in turn.
+// Every wave sums its tile in the pair type as a single wave would, and the
+// tiles' sums are folded into FP64 in list order (wave q keeps quantities q,
+// q + NW, ...): the results do not depend on NW, bit for bit, so the choice
+// may follow the size of the launch.  It costs a walk's set-up once per wave,
+// two barriers per NW tiles and LDS, so large launches take one wave.  The
+// lines lie where the two sides measured equal (us, NW = 1 / 2 / 4 / 8):
+//   gravity, FP64, softening per particle: 1007 walks 82 / 68 / 48 / 44, 2144
+//     155 / 124 / 89 / 86, 9198 385 / 349 / 309 / 354, 22946 656 / 682 / 623,
+//     51463 1463 / 1612 / 1518; mixed alike (9198: 250 / 194 / 178 / 192)
+//   gravity, mixed, uniform softening (blocks of 256 records): 1007 walks 41 /
+//     29 / 23 / 25, 4660 81 / 62 / 58 / 81, 9198 153 / 121 / 125, 22946 228 /
+//     220 / 245, 51463 479 / 513
+//   hydro, mixed: 1007 walks 31 / 26 / 22 / 24, 4660 90 / 78 / 73 (eta 1.6) and
+//     57 / 53 / 54 (1.25), 9198 89 / 97; FP64 (twice the LDS): 1007 48 / 44 /
+//     33 / 45, 3302 148 / 116 / 115, 4660 88 / 92 / 108
+struct WaveRule {
+    int w8, w4, w2;   // most walks for 8, 4 and 2 waves per walk
+};
+constexpr WaveRule kGravRule{1500, 23000, 23000}, kGravRelRule{0, 6000, 23000};
+constexpr WaveRule kHydroRule{0, 4700, 6500}, kHydroF64Rule{0, 2000, 4000};
+
+int waves_per_walk(int n_walk, const WaveRule &r)
+{
+    return n_walk <= r.w8 ? 8 : n_walk <= r.w4 ? 4 : n_walk <= r.w2 ? 2 : 1;
 }
 
 // Lane map of one i-chunk: S = floor(64/ni) slices.
@@ -880,19 +919,23 @@ __device__ __forceinline__ HRec<R> hydro_load(const sphk_hydro_src &pj, const in
 
 // FP64: at most 168 VGPRs (3 waves per SIMD, a few spills): 11 % faster than
 // 2 waves without spills.  Mixed needs 115 VGPRs (4 waves) as written.
-template <bool MIXED, bool PERSIST>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED ? (PERSIST ? 4 : 1) : 3))) void hydro_kernel(
+template <bool MIXED, bool PERSIST, int NW>
+__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(MIXED ? (PERSIST ? 4 : 1) : 3))) void hydro_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_hydro_src pi, sphk_hydro_src pj, sphk_hydro_out out, int *queue)
 {
     using R = real_t<MIXED>;
+    static_assert(!PERSIST || NW == 1, "persistent launches take one wave per walk");
     // tile records and the slice-reduction buffer share one LDS block (the
-    // reduction runs after the last tile)
+    // reduction runs after the last tile); NW > 1: the waves' sums beside it
     using PR = typename HPos<R>::rec;
     constexpr int kTileBytes = kTile * (sizeof(PR) + 3 * sizeof(R4<R>) + 2 * sizeof(R) + 4);
     constexpr int kRedBytes = 9 * kWave * sizeof(double);
-    __shared__ __attribute__((aligned(32))) char smem[kTileBytes > kRedBytes ? kTileBytes : kRedBytes];
-    PR *sp = reinterpret_cast<PR *>(smem);
+    constexpr int kWaveBytes = (kTileBytes > kRedBytes ? kTileBytes : kRedBytes);
+    __shared__ __attribute__((aligned(32))) char smem[NW * kWaveBytes];
+    __shared__ R part[NW > 1 ? NW : 1][8][NW > 1 ? kWave : 1];
+    const int wv = NW > 1 ? (int)threadIdx.x / kWave : 0;
+    PR *sp = reinterpret_cast<PR *>(smem + wv * kWaveBytes);
     R4<R> *sa = reinterpret_cast<R4<R> *>(sp + kTile);
     R4<R> *sb = sa + kTile;
     R4<R> *sc = sb + kTile;
@@ -931,58 +974,98 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED ? (
             I.et = (R)pi.eta[i];
             I.id = pi.id[i];
 
-            double acc[9] = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
+            constexpr int kOwn = (8 + NW - 1) / NW;   // sums a wave keeps
+            double acc[kOwn];
+#pragma unroll
+            for (int q = 0; q < kOwn; q++) acc[q] = 0.;
             R vsmx = R(0);
             // each lane loads its record of the tile into registers before the
             // barrier (loading the next tile's record during the sweep measured
             // 3 % slower in mixed mode, and its registers spill in FP64)
-            for (int t0 = jb; t0 < je; t0 += kTile) {
-                const int nt = min(kTile, je - t0);
-                const HRec<R> nx = hydro_load<R>(pj, j_idx, t0 + lane, je, cx, cy, cz);
-                __syncthreads();
-                sp[lane] = nx.p;
-                sa[lane] = nx.a;
-                sb[lane] = nx.b;
-                sc[lane] = nx.c;
-                se[lane] = nx.e;
-                sh[lane] = nx.h5;
-                sid[lane] = nx.id;
-                __syncthreads();
+            for (int r0 = jb; r0 < je; r0 += NW * kTile) {
+                const int t0 = r0 + wv * kTile;
                 HydroAcc<R> a{R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0), vsmx};
-                int k = M.slice;
-                for (; k + M.S < nt; k += 2 * M.S) {
-                    const int k1 = k + M.S;
-                    const PR p0 = sp[k], p1 = sp[k1];
-                    const R4<R> a0 = sa[k], a1 = sa[k1], b0 = sb[k], b1 = sb[k1], c0_ = sc[k], c1 = sc[k1];
-                    const R e0 = se[k], e1 = se[k1], f0 = sh[k], f1 = sh[k1];
-                    const int32_t d0 = sid[k], d1 = sid[k1];
-                    hydro_pair<R>(p0, a0, b0, c0_, e0, f0, d0, I, a);
-                    hydro_pair<R>(p1, a1, b1, c1, e1, f1, d1, I, a);
+                if (t0 < je) {
+                    const int nt = min(kTile, je - t0);
+                    const HRec<R> nx = hydro_load<R>(pj, j_idx, t0 + lane, je, cx, cy, cz);
+                    wave_sync();
+                    sp[lane] = nx.p;
+                    sa[lane] = nx.a;
+                    sb[lane] = nx.b;
+                    sc[lane] = nx.c;
+                    se[lane] = nx.e;
+                    sh[lane] = nx.h5;
+                    sid[lane] = nx.id;
+                    wave_sync();
+                    int k = M.slice;
+                    for (; k + M.S < nt; k += 2 * M.S) {
+                        const int k1 = k + M.S;
+                        const PR p0 = sp[k], p1 = sp[k1];
+                        const R4<R> a0 = sa[k], a1 = sa[k1], b0 = sb[k], b1 = sb[k1], c0_ = sc[k], c1 = sc[k1];
+                        const R e0 = se[k], e1 = se[k1], f0 = sh[k], f1 = sh[k1];
+                        const int32_t d0 = sid[k], d1 = sid[k1];
+                        hydro_pair<R>(p0, a0, b0, c0_, e0, f0, d0, I, a);
+                        hydro_pair<R>(p1, a1, b1, c1, e1, f1, d1, I, a);
+                    }
+                    for (; k < nt; k += M.S) hydro_pair<R>(sp[k], sa[k], sb[k], sc[k], se[k], sh[k], sid[k], I, a);
                 }
-                for (; k < nt; k += M.S) hydro_pair<R>(sp[k], sa[k], sb[k], sc[k], se[k], sh[k], sid[k], I, a);
-                acc[0] += (double)a.ax;
-                acc[1] += (double)a.ay;
-                acc[2] += (double)a.az;
-                acc[3] += (double)a.ud;
-                acc[4] += (double)a.df;
-                acc[5] += (double)a.gx;
-                acc[6] += (double)a.gy;
-                acc[7] += (double)a.gz;
                 vsmx = a.vs;
+                const R sum[8] = {a.ax, a.ay, a.az, a.ud, a.df, a.gx, a.gy, a.gz};
+                if (NW == 1) {
+#pragma unroll
+                    for (int q = 0; q < kOwn; q++) acc[q] += (double)sum[q];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 8; q++) part[wv][q][lane] = sum[q];
+                    __syncthreads();
+#pragma unroll
+                    for (int o = 0; o < kOwn; o++) {
+                        const int q = wv + o * NW;
+                        if (q < 8)
+                            for (int v = 0; v < NW && r0 + v * kTile < je; v++) acc[o] += (double)part[v][q][lane];
+                    }
+                    __syncthreads();
+                }
             }
-            acc[8] = (double)vsmx;
-            slice_reduce<9>(acc, red, M, lane, 1 << 8);
             // hdr_hydro.hpp:402-419
-            if (M.lead) {
-                out.ax[i] = acc[0] * 0.5;
-                out.ay[i] = acc[1] * 0.5;
-                out.az[i] = acc[2] * 0.5;
-                out.udot[i] = acc[3] * 0.5;
-                out.diffu[i] = acc[4] * 2.;
-                out.gx[i] = acc[5] * 0.5;
-                out.gy[i] = acc[6] * 0.5;
-                out.gz[i] = acc[7] * 0.5;
-                out.vsmx[i] = acc[8];
+            if (NW == 1) {
+                double v[9] = {acc[0], acc[1 % kOwn], acc[2 % kOwn], acc[3 % kOwn], acc[4 % kOwn], acc[5 % kOwn],
+                               acc[6 % kOwn], acc[7 % kOwn], (double)vsmx};
+                slice_reduce<9>(v, red, M, lane, 1 << 8);
+                if (M.lead) {
+                    out.ax[i] = v[0] * 0.5;
+                    out.ay[i] = v[1] * 0.5;
+                    out.az[i] = v[2] * 0.5;
+                    out.udot[i] = v[3] * 0.5;
+                    out.diffu[i] = v[4] * 2.;
+                    out.gx[i] = v[5] * 0.5;
+                    out.gy[i] = v[6] * 0.5;
+                    out.gz[i] = v[7] * 0.5;
+                    out.vsmx[i] = v[8];
+                }
+            } else {
+                double *const dst[9] = {out.ax, out.ay, out.az, out.udot, out.diffu, out.gx, out.gy, out.gz, out.vsmx};
+                part[wv][0][lane] = vsmx;   // part and the tiles are no longer read
+                __syncthreads();
+#pragma unroll
+                for (int o = 0; o < kOwn; o++)
+                    if (wv + o * NW < 8) red[(wv + o * NW) * kWave + lane] = acc[o];
+                if (wv == NW - 1) {
+                    R m = part[0][0][lane];
+                    for (int v = 1; v < NW; v++) m = m > part[v][0][lane] ? m : part[v][0][lane];
+                    red[8 * kWave + lane] = (double)m;
+                }
+                __syncthreads();
+                if (M.lead)
+                    for (int q = wv; q < 9; q += NW) {
+                        double a = red[q * kWave + M.il];
+                        for (int t = 1; t < M.S; t++) {
+                            const double b = red[q * kWave + M.il + M.ni * t];
+                            a = q == 8 ? (a > b ? a : b) : a + b;
+                        }
+                        dst[q][i] = q == 8 ? a : q == 4 ? a * 2. : a * 0.5;
+                    }
+                __syncthreads();   // LDS of this chunk no longer read
             }
         }
     };
@@ -1062,52 +1145,47 @@ __device__ __forceinline__ void gravity_pair_uniform(const GRec<MIXED> &p, doubl
     if (ETA) a.et += w;
 }
 
+// Records kb .. ke - 1 (at most kTile) of a list: the lane's sums over its slice.
 template <bool MIXED, bool UNIFORM, bool ETA>
-__device__ __forceinline__ void gravity_list(int lane, const Map &M, int kb, int ke,
-                                             const int32_t *__restrict__ idx, sphk_grav_src src,
-                                             double px, double py, double pz, double e2_i,
-                                             GRec<MIXED> *sp, double (&acc)[5])
+__device__ __forceinline__ GravAcc<real_t<MIXED>> gravity_tile(int lane, const Map &M, int kb, int ke,
+                                                               const int32_t *__restrict__ idx,
+                                                               const sphk_grav_src &src, double px, double py,
+                                                               double pz, double e2_i, GRec<MIXED> *sp)
 {
     using R = real_t<MIXED>;
     const R e2 = (R)e2_i;
-    for (int t0 = kb; t0 < ke; t0 += kTile) {
-        const int nt = min(kTile, ke - t0);
-        __syncthreads();
-        if (lane < nt) {
-            const int j = idx ? idx[t0 + lane] : t0 + lane;
-            sp[lane] = GRec<MIXED>{src.x[j], src.y[j], src.z[j], (R)src.m[j], (R)src.eps2[j]};
-        } else {
-            sp[lane] = GRec<MIXED>{kFar, kFar, kFar, R(0), R(1)};
-        }
-        __syncthreads();
-        GravAcc<R> a{R(0), R(0), R(0), R(0), R(0)};
-        int k = M.slice;
-        for (; k + 3 * M.S < nt; k += 4 * M.S) {
-            const GRec<MIXED> p0 = sp[k], p1 = sp[k + M.S], p2 = sp[k + 2 * M.S], p3 = sp[k + 3 * M.S];
-            if (UNIFORM) {
-                gravity_pair_uniform<MIXED, ETA>(p0, px, py, pz, e2, a);
-                gravity_pair_uniform<MIXED, ETA>(p1, px, py, pz, e2, a);
-                gravity_pair_uniform<MIXED, ETA>(p2, px, py, pz, e2, a);
-                gravity_pair_uniform<MIXED, ETA>(p3, px, py, pz, e2, a);
-            } else {
-                gravity_pair<MIXED, ETA>(p0, px, py, pz, e2, a);
-                gravity_pair<MIXED, ETA>(p1, px, py, pz, e2, a);
-                gravity_pair<MIXED, ETA>(p2, px, py, pz, e2, a);
-                gravity_pair<MIXED, ETA>(p3, px, py, pz, e2, a);
-            }
-        }
-        for (; k < nt; k += M.S) {
-            if (UNIFORM)
-                gravity_pair_uniform<MIXED, ETA>(sp[k], px, py, pz, e2, a);
-            else
-                gravity_pair<MIXED, ETA>(sp[k], px, py, pz, e2, a);
-        }
-        acc[0] += (double)a.ax;
-        acc[1] += (double)a.ay;
-        acc[2] += (double)a.az;
-        acc[3] += (double)a.pt;
-        acc[4] += (double)a.et;
+    const int nt = ke - kb;
+    wave_sync();
+    if (lane < nt) {
+        const int j = idx ? idx[kb + lane] : kb + lane;
+        sp[lane] = GRec<MIXED>{src.x[j], src.y[j], src.z[j], (R)src.m[j], (R)src.eps2[j]};
+    } else {
+        sp[lane] = GRec<MIXED>{kFar, kFar, kFar, R(0), R(1)};
     }
+    wave_sync();
+    GravAcc<R> a{R(0), R(0), R(0), R(0), R(0)};
+    int k = M.slice;
+    for (; k + 3 * M.S < nt; k += 4 * M.S) {
+        const GRec<MIXED> p0 = sp[k], p1 = sp[k + M.S], p2 = sp[k + 2 * M.S], p3 = sp[k + 3 * M.S];
+        if (UNIFORM) {
+            gravity_pair_uniform<MIXED, ETA>(p0, px, py, pz, e2, a);
+            gravity_pair_uniform<MIXED, ETA>(p1, px, py, pz, e2, a);
+            gravity_pair_uniform<MIXED, ETA>(p2, px, py, pz, e2, a);
+            gravity_pair_uniform<MIXED, ETA>(p3, px, py, pz, e2, a);
+        } else {
+            gravity_pair<MIXED, ETA>(p0, px, py, pz, e2, a);
+            gravity_pair<MIXED, ETA>(p1, px, py, pz, e2, a);
+            gravity_pair<MIXED, ETA>(p2, px, py, pz, e2, a);
+            gravity_pair<MIXED, ETA>(p3, px, py, pz, e2, a);
+        }
+    }
+    for (; k < nt; k += M.S) {
+        if (UNIFORM)
+            gravity_pair_uniform<MIXED, ETA>(sp[k], px, py, pz, e2, a);
+        else
+            gravity_pair<MIXED, ETA>(sp[k], px, py, pz, e2, a);
+    }
+    return a;
 }
 
 // Mixed precision with uniform softening: the j-records of a walk are staged
@@ -1138,54 +1216,65 @@ __device__ __forceinline__ void gravity_pair_rel(const float4 &p, float xi, floa
 // (at most kGravBlock / S terms) are folded into FP64 once per block.
 constexpr int kGravBlock = 4 * kTile;
 
+// Records kb .. ke - 1 (at most kGravBlock) of a list, as gravity_tile.
 template <bool ETA>
-__device__ __forceinline__ void gravity_list_rel(const Map &M, int lane, int kb, int ke,
-                                                 const int32_t *__restrict__ idx, const sphk_grav_src &src,
-                                                 double cx, double cy, double cz, float xi, float yi,
-                                                 float zi, float e2, float4 *sp, double (&acc)[5])
+__device__ __forceinline__ GravAcc<float> gravity_block_rel(const Map &M, int lane, int kb, int ke,
+                                                            const int32_t *__restrict__ idx,
+                                                            const sphk_grav_src &src, double cx, double cy, double cz,
+                                                            float xi, float yi, float zi, float e2, float4 *sp)
 {
-    const int k0 = M.slice < M.S ? M.slice : kGravBlock;   // idle lanes: empty sweeps
-    for (int b0 = kb; b0 < ke; b0 += kGravBlock) {
-        const int nb = min(kGravBlock, ke - b0);
-        __syncthreads();
-        for (int e = lane; e < nb; e += kWave) {
-            const int j = idx ? idx[b0 + e] : b0 + e;
-            sp[e] = make_float4((float)(src.x[j] - cx), (float)(src.y[j] - cy), (float)(src.z[j] - cz),
-                                (float)src.m[j]);
-        }
-        __syncthreads();
-        GravAcc<float> a{0.f, 0.f, 0.f, 0.f, 0.f};
-        int k = k0;
-        for (; k + 3 * M.S < nb; k += 4 * M.S) {
-            const float4 p0 = sp[k], p1 = sp[k + M.S], p2 = sp[k + 2 * M.S], p3 = sp[k + 3 * M.S];
-            gravity_pair_rel<ETA>(p0, xi, yi, zi, e2, a);
-            gravity_pair_rel<ETA>(p1, xi, yi, zi, e2, a);
-            gravity_pair_rel<ETA>(p2, xi, yi, zi, e2, a);
-            gravity_pair_rel<ETA>(p3, xi, yi, zi, e2, a);
-        }
-        for (; k < nb; k += M.S) gravity_pair_rel<ETA>(sp[k], xi, yi, zi, e2, a);
-        acc[0] += (double)a.ax;
-        acc[1] += (double)a.ay;
-        acc[2] += (double)a.az;
-        acc[3] += (double)a.pt;
-        acc[4] += (double)a.et;
+    const int nb = ke - kb;
+    wave_sync();
+    // all of a lane's indices, then all its records, are loaded before any is
+    // written (past the end: the last record again): 955 -> 938 us at 10^6
+    // particles against one record after the other
+    constexpr int kPer = kGravBlock / kWave;
+    int j[kPer];
+    double4 v[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const int e = min(u * kWave + lane, nb - 1);
+        j[u] = idx ? idx[kb + e] : kb + e;
     }
+#pragma unroll
+    for (int u = 0; u < kPer; u++) v[u] = make_double4(src.x[j[u]], src.y[j[u]], src.z[j[u]], src.m[j[u]]);
+#pragma unroll
+    for (int u = 0; u < kPer; u++)
+        sp[u * kWave + lane] = make_float4((float)(v[u].x - cx), (float)(v[u].y - cy), (float)(v[u].z - cz), (float)v[u].w);
+    wave_sync();
+    GravAcc<float> a{0.f, 0.f, 0.f, 0.f, 0.f};
+    int k = M.slice < M.S ? M.slice : kGravBlock;   // idle lanes: empty sweeps
+    for (; k + 3 * M.S < nb; k += 4 * M.S) {
+        const float4 p0 = sp[k], p1 = sp[k + M.S], p2 = sp[k + 2 * M.S], p3 = sp[k + 3 * M.S];
+        gravity_pair_rel<ETA>(p0, xi, yi, zi, e2, a);
+        gravity_pair_rel<ETA>(p1, xi, yi, zi, e2, a);
+        gravity_pair_rel<ETA>(p2, xi, yi, zi, e2, a);
+        gravity_pair_rel<ETA>(p3, xi, yi, zi, e2, a);
+    }
+    for (; k < nb; k += M.S) gravity_pair_rel<ETA>(sp[k], xi, yi, zi, e2, a);
+    return a;
 }
 
 // ETA false: the caller does not need the softening-gradient sum (out.eta
 // NULL, e.g. under a constant softening, where it does not enter).
-template <bool MIXED, bool UNIFORM, bool ETA, bool PERSIST>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PERSIST && MIXED ? 8 : 1))) void gravity_kernel(
+template <bool MIXED, bool UNIFORM, bool ETA, bool PERSIST, int NW>
+__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(PERSIST && MIXED ? 8 : 1))) void gravity_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_grav_src pj, const int32_t *__restrict__ s_off,
     const int32_t *__restrict__ s_idx, sphk_grav_src ps, sphk_grav_src pi, sphk_grav_out out, int *queue)
 {
-    constexpr int kTileBytes = kTile * sizeof(GRec<MIXED>);
-    constexpr int kRelBytes = (MIXED && UNIFORM) ? kGravBlock * (int)sizeof(float4) : 0;
+    using R = real_t<MIXED>;
+    static_assert(!PERSIST || NW == 1, "persistent launches take one wave per walk");
+    constexpr bool kRel = MIXED && UNIFORM;
+    constexpr int kBlk = kRel ? kGravBlock : kTile;
+    constexpr int kBlkBytes = kRel ? kGravBlock * (int)sizeof(float4) : kTile * (int)sizeof(GRec<MIXED>);
     constexpr int kRedBytes = 5 * kWave * sizeof(double);
-    constexpr int kMax1 = kTileBytes > kRedBytes ? kTileBytes : kRedBytes;
-    __shared__ __attribute__((aligned(32))) char smem[kMax1 > kRelBytes ? kMax1 : kRelBytes];
-    GRec<MIXED> *sp = reinterpret_cast<GRec<MIXED> *>(smem);
+    constexpr int kWaveBytes = NW > 1 || kBlkBytes > kRedBytes ? kBlkBytes : kRedBytes;
+    static_assert(NW == 1 || NW * kWaveBytes >= kRedBytes, "reduction buffer");
+    __shared__ __attribute__((aligned(32))) char smem[NW * kWaveBytes];
+    __shared__ R part[NW > 1 ? NW : 1][5][NW > 1 ? kWave : 1];   // the waves' block sums
+    const int wv = NW > 1 ? (int)threadIdx.x / kWave : 0;
+    char *mine = smem + wv * kWaveBytes;
     double *red = reinterpret_cast<double *>(smem);
 
     auto walk = [&](const int w, const int lane) {
@@ -1195,38 +1284,80 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PERSIST &
             const Map M(min(kWave, ie - c0), lane);
             const int i = c0 + M.il;
             const double px = pi.x[i], py = pi.y[i], pz = pi.z[i], e2 = pi.eps2[i];
-            double acc[5] = {0., 0., 0., 0., 0.};
-            if (MIXED && UNIFORM) {
-                const double cx = pi.x[ib], cy = pi.y[ib], cz = pi.z[ib];
-                const float xi = (float)(px - cx), yi = (float)(py - cy), zi = (float)(pz - cz);
-                float4 *sr = reinterpret_cast<float4 *>(smem);
-                gravity_list_rel<ETA>(M, lane, j_off[w], j_off[w + 1], j_idx, pj, cx, cy, cz, xi, yi, zi,
-                                      (float)e2, sr, acc);
-                if (s_off)
-                    gravity_list_rel<ETA>(M, lane, s_off[w], s_off[w + 1], s_idx, ps, cx, cy, cz, xi, yi, zi,
-                                          (float)e2, sr, acc);
-            } else {
-                gravity_list<MIXED, UNIFORM, ETA>(lane, M, j_off[w], j_off[w + 1], j_idx, pj, px, py, pz, e2, sp,
-                                                  acc);
-                if (s_off)
-                    gravity_list<MIXED, UNIFORM, ETA>(lane, M, s_off[w], s_off[w + 1], s_idx, ps, px, py, pz, e2,
-                                                      sp, acc);
+            double cx = 0., cy = 0., cz = 0.;
+            float xi = 0.f, yi = 0.f, zi = 0.f;
+            if (kRel) {
+                cx = pi.x[ib];
+                cy = pi.y[ib];
+                cz = pi.z[ib];
+                xi = (float)(px - cx);
+                yi = (float)(py - cy);
+                zi = (float)(pz - cz);
             }
-            slice_reduce<5>(acc, red, M, lane);
-            if (M.lead) {
-                if (UNIFORM) {
-                    // 0.5 * (-2 sum m rei3 x) etc.
-                    out.ax[i] = -acc[0];
-                    out.ay[i] = -acc[1];
-                    out.az[i] = -acc[2];
-                    out.pot[i] = -acc[3];
-                } else {
-                    out.ax[i] = acc[0] * 0.5;
-                    out.ay[i] = acc[1] * 0.5;
-                    out.az[i] = acc[2] * 0.5;
-                    out.pot[i] = acc[3] * 0.5;
+            constexpr int kOwn = (5 + NW - 1) / NW;   // sums a wave keeps
+            double acc[kOwn];
+#pragma unroll
+            for (int q = 0; q < kOwn; q++) acc[q] = 0.;
+            // the EPJ list, then the SPJ list; NW blocks at a time
+            auto list = [&](int kb, int ke, const int32_t *idx, const sphk_grav_src &src) {
+                for (int r0 = kb; r0 < ke; r0 += NW * kBlk) {
+                    const int b0 = r0 + wv * kBlk;
+                    GravAcc<R> a{R(0), R(0), R(0), R(0), R(0)};
+                    if (b0 < ke) {
+                        const int b1 = min(ke, b0 + kBlk);
+                        if constexpr (kRel)
+                            a = gravity_block_rel<ETA>(M, lane, b0, b1, idx, src, cx, cy, cz, xi, yi, zi, (float)e2,
+                                                       reinterpret_cast<float4 *>(mine));
+                        else
+                            a = gravity_tile<MIXED, UNIFORM, ETA>(lane, M, b0, b1, idx, src, px, py, pz, e2,
+                                                                  reinterpret_cast<GRec<MIXED> *>(mine));
+                    }
+                    const R sum[5] = {a.ax, a.ay, a.az, a.pt, a.et};
+                    if (NW == 1) {
+#pragma unroll
+                        for (int q = 0; q < kOwn; q++) acc[q] += (double)sum[q];
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 5; q++) part[wv][q][lane] = sum[q];
+                        __syncthreads();
+#pragma unroll
+                        for (int o = 0; o < kOwn; o++) {
+                            const int q = wv + o * NW;
+                            if (q < 5)
+                                for (int v = 0; v < NW && r0 + v * kBlk < ke; v++) acc[o] += (double)part[v][q][lane];
+                        }
+                        __syncthreads();
+                    }
                 }
-                if (ETA) out.eta[i] = acc[4];
+            };
+            list(j_off[w], j_off[w + 1], j_idx, pj);
+            if (s_off) list(s_off[w], s_off[w + 1], s_idx, ps);
+            // UNIFORM: 0.5 * (-2 sum m rei3 x) etc.
+            constexpr double kf = UNIFORM ? -1. : 0.5;
+            if (NW == 1) {
+                double v[5] = {acc[0], acc[1 % kOwn], acc[2 % kOwn], acc[3 % kOwn], acc[4 % kOwn]};
+                slice_reduce<5>(v, red, M, lane);
+                if (M.lead) {
+                    out.ax[i] = v[0] * kf;
+                    out.ay[i] = v[1] * kf;
+                    out.az[i] = v[2] * kf;
+                    out.pot[i] = v[3] * kf;
+                    if (ETA) out.eta[i] = v[4];
+                }
+            } else {
+                double *const dst[5] = {out.ax, out.ay, out.az, out.pot, out.eta};
+                __syncthreads();   // the last blocks are read
+#pragma unroll
+                for (int o = 0; o < kOwn; o++)
+                    if (wv + o * NW < 5) red[(wv + o * NW) * kWave + lane] = acc[o];
+                wave_sync();
+                if (M.lead)
+                    for (int q = wv; q < (ETA ? 5 : 4); q += NW) {
+                        double a = red[q * kWave + M.il];
+                        for (int t = 1; t < M.S; t++) a = a + red[q * kWave + M.il + M.ni * t];
+                        dst[q][i] = q == 4 ? a : a * kf;
+                    }
+                __syncthreads();   // LDS of this chunk no longer read
             }
         }
     };
@@ -1252,18 +1383,18 @@ static int persistent_grid(K kernel, int n_walk)
     return g < need ? g : need;
 }
 
-// One launch: ordinary (grid = n_walk) or, with a queue, persistent.
-#define SPHK_LAUNCH(KERNEL, KERNEL_P, ...)                                                     \
-    do {                                                                                        \
-        if (queue) {                                                                            \
-            const int g_ = persistent_grid(KERNEL_P, n_walk);                                   \
-            if (g_ <= 0) return hipErrorInvalidValue;                                           \
-            hipLaunchKernelGGL(KERNEL_P, dim3(g_), dim3(kWave), 0, st, __VA_ARGS__, queue);     \
-        } else {                                                                                \
-            hipLaunchKernelGGL(KERNEL, dim3(n_walk), dim3(kWave), 0, st, __VA_ARGS__, nullptr); \
-        }                                                                                       \
+// One launch: ordinary (grid = n_walk, waves waves per walk) or, with a queue,
+// persistent.
+#define SPHK_LAUNCH(KERNEL, KERNEL_P, waves, ...)                                                       \
+    do {                                                                                                 \
+        if (queue) {                                                                                     \
+            const int g_ = persistent_grid(KERNEL_P, n_walk);                                            \
+            if (g_ <= 0) return hipErrorInvalidValue;                                                    \
+            hipLaunchKernelGGL(KERNEL_P, dim3(g_), dim3(kWave), 0, st, __VA_ARGS__, queue);              \
+        } else {                                                                                         \
+            hipLaunchKernelGGL(KERNEL, dim3(n_walk), dim3(kWave * (waves)), 0, st, __VA_ARGS__, nullptr); \
+        }                                                                                                \
     } while (0)
-
 hipError_t launch_density(hipStream_t st, int n_walk, const int32_t *i_off, const int32_t *j_off,
                           const int32_t *j_idx, const sphk_dens_src &pi, const sphk_dens_src &pj,
                           const sphk_dens_out &out, double eta_ksrh, double hmax, bool mixed, int list_cap,
@@ -1271,7 +1402,7 @@ hipError_t launch_density(hipStream_t st, int n_walk, const int32_t *i_off, cons
 {
     if (n_walk <= 0) return hipSuccess;
 #define SPHK_LAUNCH_D(M, CAPV)                                                                           \
-    SPHK_LAUNCH((density_kernel<M, CAPV, false>), (density_kernel<M, CAPV, true>), n_walk, i_off, j_off, \
+    SPHK_LAUNCH((density_kernel<M, CAPV, false>), (density_kernel<M, CAPV, true>), 1, n_walk, i_off, j_off, \
                 j_idx, pi, pj, out, eta_ksrh, hmax)
     if (list_cap == 192) {
         if (mixed)
@@ -1293,12 +1424,21 @@ hipError_t launch_hydro(hipStream_t st, int n_walk, const int32_t *i_off, const 
                         const sphk_hydro_out &out, bool mixed, int *queue)
 {
     if (n_walk <= 0) return hipSuccess;
-    if (mixed)
-        SPHK_LAUNCH((hydro_kernel<true, false>), (hydro_kernel<true, true>), n_walk, i_off, j_off, j_idx, pi, pj,
-                    out);
-    else
-        SPHK_LAUNCH((hydro_kernel<false, false>), (hydro_kernel<false, true>), n_walk, i_off, j_off, j_idx, pi,
-                    pj, out);
+#define SPHK_LAUNCH_H(M, W) \
+    SPHK_LAUNCH((hydro_kernel<M, false, W>), (hydro_kernel<M, true, 1>), W, n_walk, i_off, j_off, j_idx, pi, pj, out)
+#define SPHK_LAUNCH_HM(W) SPHK_LAUNCH_H(true, W)
+#define SPHK_LAUNCH_HD(W) SPHK_LAUNCH_H(false, W)
+    switch (waves_per_walk(n_walk, mixed ? kHydroRule : kHydroF64Rule) + (mixed ? 0 : 8)) {
+    case 4: SPHK_LAUNCH_HM(4); break;
+    case 2: SPHK_LAUNCH_HM(2); break;
+    case 1: SPHK_LAUNCH_HM(1); break;
+    case 8 + 4: SPHK_LAUNCH_HD(4); break;
+    case 8 + 2: SPHK_LAUNCH_HD(2); break;
+    default: SPHK_LAUNCH_HD(1); break;
+    }
+#undef SPHK_LAUNCH_HM
+#undef SPHK_LAUNCH_HD
+#undef SPHK_LAUNCH_H
     return hipGetLastError();
 }
 
@@ -1308,23 +1448,36 @@ hipError_t launch_gravity(hipStream_t st, int n_walk, const int32_t *i_off, cons
                           const sphk_grav_out &out, bool mixed, bool uniform, int *queue)
 {
     if (n_walk <= 0) return hipSuccess;
-#define SPHK_LAUNCH_G(M, U, E)                                                                   \
-    SPHK_LAUNCH((gravity_kernel<M, U, E, false>), (gravity_kernel<M, U, E, true>), n_walk, i_off, \
-                j_off, j_idx, pj, s_off, s_idx, ps, pi, out)
-    const bool eta = out.eta != nullptr;
-    if (mixed && uniform) {
-        if (eta) SPHK_LAUNCH_G(true, true, true);
-        else SPHK_LAUNCH_G(true, true, false);
-    } else if (mixed) {
-        if (eta) SPHK_LAUNCH_G(true, false, true);
-        else SPHK_LAUNCH_G(true, false, false);
-    } else if (uniform) {
-        if (eta) SPHK_LAUNCH_G(false, true, true);
-        else SPHK_LAUNCH_G(false, true, false);
-    } else {
-        if (eta) SPHK_LAUNCH_G(false, false, true);
-        else SPHK_LAUNCH_G(false, false, false);
+#define SPHK_LAUNCH_G(M, U, E, W)                                                                            \
+    SPHK_LAUNCH((gravity_kernel<M, U, E, false, W>), (gravity_kernel<M, U, E, true, 1>), W, n_walk, i_off, j_off, \
+                j_idx, pj, s_off, s_idx, ps, pi, out)
+    // the kernel of one (precision, softening, eta), by its waves per walk; the
+    // rel path (mixed, uniform) has no use for 8
+#define SPHK_REL(E)                               \
+    switch (waves) {                              \
+    case 4: SPHK_LAUNCH_G(true, true, E, 4); break; \
+    case 2: SPHK_LAUNCH_G(true, true, E, 2); break; \
+    default: SPHK_LAUNCH_G(true, true, E, 1); break; \
     }
+#define SPHK_GEN(M, U, E)                      \
+    switch (waves) {                           \
+    case 8: SPHK_LAUNCH_G(M, U, E, 8); break;  \
+    case 4: SPHK_LAUNCH_G(M, U, E, 4); break;  \
+    default: SPHK_LAUNCH_G(M, U, E, 1); break; \
+    }
+    const bool eta = out.eta != nullptr;
+    const int waves = waves_per_walk(n_walk, mixed && uniform ? kGravRelRule : kGravRule);
+    if (mixed && uniform) {
+        if (eta) SPHK_REL(true) else SPHK_REL(false)
+    } else if (mixed) {
+        if (eta) SPHK_GEN(true, false, true) else SPHK_GEN(true, false, false)
+    } else if (uniform) {
+        if (eta) SPHK_GEN(false, true, true) else SPHK_GEN(false, true, false)
+    } else {
+        if (eta) SPHK_GEN(false, false, true) else SPHK_GEN(false, false, false)
+    }
+#undef SPHK_REL
+#undef SPHK_GEN
 #undef SPHK_LAUNCH_G
     return hipGetLastError();
 }
