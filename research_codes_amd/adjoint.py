@@ -18,13 +18,12 @@ import torch
 from torch.utils.checkpoint import checkpoint
 
 from . import _lib as L
-from ._lib import check, lib
+from ._lib import check, lib, raw_stream
 from .device import FP64, Context, Walks
 from .tree import DeviceTree, morton_order_dev
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+_stream = raw_stream
 
 
 class TreeGravity:

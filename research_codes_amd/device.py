@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from ._lib import check, lib
+from ._lib import check, lib, raw_stream
 
 FP64 = L.SPHK_FP64
 MIXED = L.SPHK_MIXED
@@ -38,8 +38,14 @@ def _ptr(t: torch.Tensor | None, name: str, dtype=None):
 
 
 def _mk(cls, fields, d: dict | None):
-    d = d or {}
-    return cls(**{f: _ptr(d.get(f), f) for f in fields})
+    get = (d or {}).get
+    return cls(*[_ptr(get(f), f) for f in fields])
+
+
+def _mk2(cls, fields, a: dict | None, b: dict | None):
+    """The structs of both sides of a functor, made once where they are one dict."""
+    first = _mk(cls, fields, a)
+    return first, first if b is a else _mk(cls, fields, b)
 
 
 def to_device(a: np.ndarray | torch.Tensor, device="cuda") -> torch.Tensor:
@@ -161,21 +167,19 @@ class Context:
                     uniform_softening=bool(self._params.uniform_softening), list_cap=self._params.list_cap,
                     persistent=bool(self._params.persistent))
 
-    @staticmethod
-    def _stream():
-        return torch.cuda.current_stream().cuda_stream
+    _stream = staticmethod(raw_stream)
 
     def density(self, w: Walks, pi: dict, pj: dict, out: dict, precision: int = FP64):
+        si, sj = _mk2(L.DensSrc, L.DENS_SRC, pi, pj)
         check(lib().sphk_density_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                     None if w.j_idx is None else w.j_idx.data_ptr(),
-                                     _mk(L.DensSrc, L.DENS_SRC, pi), _mk(L.DensSrc, L.DENS_SRC, pj),
+                                     None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
                                      _mk(L.DensOut, L.DENS_OUT, out), int(precision),
                                      self._stream()), "sphk_density_dev")
 
     def hydro(self, w: Walks, pi: dict, pj: dict, out: dict, precision: int = FP64):
+        si, sj = _mk2(L.HydroSrc, L.HYDRO_SRC, pi, pj)
         check(lib().sphk_hydro_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                   None if w.j_idx is None else w.j_idx.data_ptr(),
-                                   _mk(L.HydroSrc, L.HYDRO_SRC, pi), _mk(L.HydroSrc, L.HYDRO_SRC, pj),
+                                   None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
                                    _mk(L.HydroOut, L.HYDRO_OUT, out), int(precision),
                                    self._stream()), "sphk_hydro_dev")
 
@@ -203,12 +207,12 @@ class Context:
 
     def gravity(self, w: Walks, pj: dict, pi: dict, out: dict, ps: dict | None = None,
                 precision: int = FP64):
+        sj, si = _mk2(L.GravSrc, L.GRAV_SRC, pj, pi)
         check(lib().sphk_gravity_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                     None if w.j_idx is None else w.j_idx.data_ptr(),
-                                     _mk(L.GravSrc, L.GRAV_SRC, pj),
+                                     None if w.j_idx is None else w.j_idx.data_ptr(), sj,
                                      None if w.s_off is None else w.s_off.data_ptr(),
                                      None if w.s_idx is None else w.s_idx.data_ptr(),
-                                     _mk(L.GravSrc, L.GRAV_SRC, ps), _mk(L.GravSrc, L.GRAV_SRC, pi),
+                                     _mk(L.GravSrc, L.GRAV_SRC, ps), si,
                                      _mk(L.GravOut, L.GRAV_OUT, out), int(precision),
                                      self._stream()), "sphk_gravity_dev")
 

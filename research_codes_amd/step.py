@@ -25,7 +25,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from ._lib import check, lib
+from ._lib import check, lib, raw_stream
 from .device import FP64, MIXED, Context, Walks, _mk, to_device
 from .tree import DeviceTree, HostTree, morton_order, morton_order_dev, permute_dev
 
@@ -302,8 +302,7 @@ class SPHSystem:
         return best, table
 
     # ---------------------------------------------------------------- kernels
-    def _st(self):
-        return torch.cuda.current_stream().cuda_stream
+    _st = staticmethod(raw_stream)
 
     def _softening(self):
         check(lib().sphk_softening_dev(self.ctx.handle, self.n, self.s["ksr"].data_ptr(), KSRH,

@@ -12,7 +12,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._lib import _DP, _I32P, _P, check, lib
+from ._lib import _DP, _I32P, _P, check, lib, raw_stream
 
 
 def _f64(a):
@@ -131,9 +131,7 @@ def _dptr(t):
     return t.data_ptr()
 
 
-def _stream():
-    import torch
-    return torch.cuda.current_stream().cuda_stream
+_stream = raw_stream
 
 
 def _copy_out(ptr, n: int, dtype):
