@@ -150,18 +150,27 @@ void *sphk_stream(const sphk_ctx *ctx);
 int sphk_synchronize(sphk_ctx *ctx);
 
 /* ---- device-resident launches (pointers are device pointers) ---------- */
+/* The _dev_n entries are the _dev entries with the number of i-particles of
+ * the walks (0: not known, as the _dev entries take it).  Few or long walks
+ * then run with several waves each; the results are the same bit for bit. */
 
 /* Density functor over n_walk walks; replaces DensKernel
  * (hdr_densityGPU.cu:454-484) launched by DispatchKernel_Dens (:496-592). */
 int sphk_density_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
                      const int32_t *j_idx, sphk_dens_src pi, sphk_dens_src pj,
                      sphk_dens_out out, int precision, void *stream);
+int sphk_density_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off,
+                       const int32_t *j_off, const int32_t *j_idx, sphk_dens_src pi, sphk_dens_src pj,
+                       sphk_dens_out out, int precision, void *stream);
 
 /* Hydro functor; replaces HydroForceKernel (hdr_hydroGPU.cu:319-363)
  * launched by DispatchKernel_HydroForce (:371-477). */
 int sphk_hydro_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
                    const int32_t *j_idx, sphk_hydro_src pi, sphk_hydro_src pj,
                    sphk_hydro_out out, int precision, void *stream);
+int sphk_hydro_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off,
+                       const int32_t *j_off, const int32_t *j_idx, sphk_hydro_src pi, sphk_hydro_src pj,
+                       sphk_hydro_out out, int precision, void *stream);
 
 /* Gravity functor over the EPJ list then the SPJ list of each walk; replaces
  * GravityForceKernel (hdr_gravityGPU.cu:330-374) launched by
@@ -170,6 +179,10 @@ int sphk_hydro_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_
  * may be NULL: the softening-gradient sum is then not formed (callers that
  * do not use it, e.g. under a constant softening). */
 int sphk_gravity_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off,
+                     const int32_t *j_off, const int32_t *j_idx, sphk_grav_src pj,
+                     const int32_t *s_off, const int32_t *s_idx, sphk_grav_src ps,
+                     sphk_grav_src pi, sphk_grav_out out, int precision, void *stream);
+int sphk_gravity_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off,
                      const int32_t *j_off, const int32_t *j_idx, sphk_grav_src pj,
                      const int32_t *s_off, const int32_t *s_idx, sphk_grav_src ps,
                      sphk_grav_src pi, sphk_grav_out out, int precision, void *stream);

@@ -88,6 +88,10 @@ SIGNATURES = {
     "sphk_hydro_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, HydroSrc, HydroSrc, HydroOut, C.c_int, _P]),
     "sphk_gravity_dev": (C.c_int, [_P, C.c_int, _P, _P, _P, GravSrc, _P, _P, GravSrc, GravSrc,
                                    GravOut, C.c_int, _P]),
+    "sphk_density_dev_n": (C.c_int, [_P, C.c_int, C.c_int64, _P, _P, _P, DensSrc, DensSrc, DensOut, C.c_int, _P]),
+    "sphk_hydro_dev_n": (C.c_int, [_P, C.c_int, C.c_int64, _P, _P, _P, HydroSrc, HydroSrc, HydroOut, C.c_int, _P]),
+    "sphk_gravity_dev_n": (C.c_int, [_P, C.c_int, C.c_int64, _P, _P, _P, GravSrc, _P, _P, GravSrc, GravSrc,
+                                   GravOut, C.c_int, _P]),
     "sphk_density_dispatch": (C.c_int, [_P, C.c_int, C.c_int, _P, _P, DensSrc, DensSrc, C.c_int]),
     "sphk_density_retrieve": (C.c_int, [_P, C.c_int, C.c_int, _P, DensOut]),
     "sphk_hydro_dispatch": (C.c_int, [_P, C.c_int, C.c_int, _P, _P, HydroSrc, HydroSrc, C.c_int]),

@@ -1,8 +1,8 @@
 // sphk_kernels.hip -- gfx950 kernels for the SPH interaction functors.
 //
 // Launch shape (all three kernels): one workgroup per walk, of one 64-lane
-// wavefront (several for the hydro and gravity functors of a launch of few
-// walks, see WaveRule).  A walk's i-particles are processed in chunks of <= 64.  Inside a
+// wavefront (several where walks are few or long, see WaveRule).  A walk's
+// i-particles are processed in chunks of <= 64.  Inside a
 // chunk of ni particles the wave is split into S = floor(64/ni) j-slices:
 // lane l holds i = l mod ni and slice l / ni (lanes beyond S*ni idle), so a
 // walk of 5 particles keeps 60 of 64 lanes busy.  j-entries are staged
@@ -99,33 +99,52 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Waves per walk of the hydro and gravity functors.  A launch of few walks
-// leaves SIMDs idle at one wave per walk, and each walk's list is a serial
-// chain of tiles; so NW waves of one workgroup take a walk's tiles in turn.
-// Every wave sums its tile in the pair type as a single wave would, and the
-// tiles' sums are folded into FP64 in list order (wave q keeps quantities q,
-// q + NW, ...): the results do not depend on NW, bit for bit, so the choice
-// may follow the size of the launch.  It costs a walk's set-up once per wave,
-// two barriers per NW tiles and LDS, so large launches take one wave.  The
-// lines lie where the two sides measured equal (us, NW = 1 / 2 / 4 / 8):
-//   gravity, FP64, softening per particle: 1007 walks 82 / 68 / 48 / 44, 2144
-//     155 / 124 / 89 / 86, 9198 385 / 349 / 309 / 354, 22946 656 / 682 / 623,
-//     51463 1463 / 1612 / 1518; mixed alike (9198: 250 / 194 / 178 / 192)
-//   gravity, mixed, uniform softening (blocks of 256 records): 1007 walks 41 /
-//     29 / 23 / 25, 4660 81 / 62 / 58 / 81, 9198 153 / 121 / 125, 22946 228 /
-//     220 / 245, 51463 479 / 513
-//   hydro, mixed: 1007 walks 31 / 26 / 22 / 24, 4660 90 / 78 / 73 (eta 1.6) and
-//     57 / 53 / 54 (1.25), 9198 89 / 97; FP64 (twice the LDS): 1007 48 / 44 /
-//     33 / 45, 3302 148 / 116 / 115, 4660 88 / 92 / 108
-struct WaveRule {
-    int w8, w4, w2;   // most walks for 8, 4 and 2 waves per walk
+// Waves per walk of the three functors.  A launch of few walks leaves SIMDs
+// idle at one wave per walk, and each walk's list is a serial chain of tiles;
+// so NW waves of one workgroup take a walk's tiles in turn.  Hydro and
+// gravity: every wave sums its tile in the pair type as a single wave would,
+// and the tiles' sums are folded into FP64 in list order (wave q keeps
+// quantities q, q + NW, ...).  Density: see there.  The results do not depend
+// on NW, bit for bit, so the choice may follow the launch.  It costs a walk's
+// set-up once per wave, two barriers per NW tiles and LDS, so it pays where
+// the walks are few or long.  Their length is known to the caller only as the
+// mean number m of i-particles (a walk of more of them has a longer list too);
+// without it one wave is taken.  The lines lie where both sides measured
+// equal, in us for walks (m):
+//   gravity, FP64, softening per particle, NW = 1 / 4 / 8: 635 (4.7) 29 / 18 /
+//     16, 1000 (3.0) 28 / 17 / 16, 2144 (9.3) 155 / 87 / 86, 3852 (2.6) 48 /
+//     47, 4127 (17) 480 / 281 / 280, 7585 (5.3) 148 / 141, 13487 (5.2) 229 /
+//     224, 15589 (9.6) 530 / 496, 35089 (8.5) 904 / 884, 51463 (19) 1463 /
+//     1518; mixed alike (13487: 135 / 133); FP64, uniform: 6885 (2.9) 63 / 67,
+//     13487 (5.2) 165 / 177, 15589 (9.6) 370 / 334, 44603 (18) 1888 / 1808
+//   gravity, mixed, uniform softening (blocks of 256 records), NW = 1 / 2 / 4:
+//     635 (4.7) 16 / 13 / 11, 1000 (3.0) 12.6 / 14.1 / 11.1, 1958 (5.1) 26 / 21 /
+//     21, 4477 (4.5) 34 / 32 / 33, 4660 (8.6) 76 / 60 / 60, 7464 (20) 254 / 206 /
+//     200, 13487 (5.2) 87 / 88, 15589 (9.6) 173 / 170, 51463 (19) 479 / 513
+//   hydro, mixed, NW = 1 / 4: 635 (4.7) 18 / 21, 1007 (9.9) 33 / 23, 2144 (9.3)
+//     45 / 36, 4660 (8.6) 60 / 57, 7464 (20) 197 / 180, 15691 (19) 310 / 325;
+//     FP64 (twice the LDS), NW = 1 / 2 / 4: 1007 (9.9) 50 / 47 / 40, 2144
+//     (9.3) 71 / 65 / 65, 4127 (17) 244 / 199 / 206, 4660 (8.6) 94 / 98, 7464
+//     (20) 326 / 335
+//   density, FP64, NW = 1 / 2: 1000 (3.0) 29 / 25, 3852 (2.6) 42 / 61, 4477
+//     (4.5) 71 / 69, 7165 (9.8) 200 / 171, 7585 (5.3) 112 / 117, 15589 (9.6)
+//     324 / 325, 15691 (19) 906 / 845, 35089 (8.5) 534 / 565; mixed alike; 4
+//     waves were slower than 2
+struct WaveLine {
+    double k, m0;   // up to k (m - m0) walks of m i-particles on average
 };
-constexpr WaveRule kGravRule{1500, 23000, 23000}, kGravRelRule{0, 6000, 23000};
-constexpr WaveRule kHydroRule{0, 4700, 6500}, kHydroF64Rule{0, 2000, 4000};
+struct WaveRule {
+    WaveLine w8, w4, w2;   // lines for 8, 4 and 2 waves per walk
+};
+constexpr WaveLine kNever{0., 0.};
+constexpr WaveRule kGravRule{{200., 0.}, {2500., 1.5}, kNever}, kGravRelRule{kNever, {500., 2.}, {3000., 3.}};
+constexpr WaveRule kHydroRule{kNever, {600., 5.}, kNever}, kHydroF64Rule{kNever, {250., 4.}, {450., 4.5}};
+constexpr WaveRule kDensRule{kNever, kNever, {2000., 2.2}};
 
-int waves_per_walk(int n_walk, const WaveRule &r)
+int waves_per_walk(int n_walk, int64_t n_i, const WaveRule &r)
 {
-    return n_walk <= r.w8 ? 8 : n_walk <= r.w4 ? 4 : n_walk <= r.w2 ? 2 : 1;
+    const auto within = [&](const WaveLine &l) { return n_walk <= l.k * ((double)n_i / n_walk - l.m0); };
+    return n_i <= 0 ? 1 : within(r.w8) ? 8 : within(r.w4) ? 4 : within(r.w2) ? 2 : 1;
 }
 
 // Lane map of one i-chunk: S = floor(64/ni) slices.
@@ -185,7 +204,7 @@ __device__ __forceinline__ double exact_r(double dx, double dy, double dz)
 {
 #pragma clang fp contract(off)
     const double r2 = dx * dx + dy * dy + dz * dz;
-    return __builtin_sqrt(r2);
+    return sqrt_ieee(r2);
 }
 
 struct Pass1 {
@@ -268,23 +287,36 @@ __device__ __forceinline__ void dens_finish(const sphk_dens_out &out, int i, con
     out.grdh[i] = omgi;
 }
 
-// Wave-wide inclusive prefix sum and maximum.
-__device__ __forceinline__ int wave_scan_incl(int v, int lane)
+// Wave-wide inclusive prefix sum and maximum (of values >= 0), all 64 lanes
+// active: row shifts and row broadcasts in the VALU (no LDS round trips: each
+// of the six steps of a shuffle waits for one).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int v)
 {
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int t = __shfl_up(v, d, kWave);
-        if (lane >= d) v += t;
-    }
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);   // 0 where there is no source lane
+}
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
+__device__ __forceinline__ int wave_scan_incl(int v)
+{
+    v += dpp0<kRowShr + 1, 0xf>(v);
+    v += dpp0<kRowShr + 2, 0xf>(v);
+    v += dpp0<kRowShr + 4, 0xf>(v);
+    v += dpp0<kRowShr + 8, 0xf>(v);
+    v += dpp0<kRowBcast15, 0xa>(v);
+    v += dpp0<kRowBcast31, 0xc>(v);
     return v;
 }
 
 __device__ __forceinline__ int wave_max(int v)
 {
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int t = __shfl_xor(v, d, kWave);
-        v = t > v ? t : v;
-    }
-    return v;
+    v = max(v, dpp0<kRowShr + 1, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 2, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 4, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 8, 0xf>(v));
+    v = max(v, dpp0<kRowBcast15, 0xa>(v));
+    v = max(v, dpp0<kRowBcast31, 0xc>(v));
+    return __builtin_amdgcn_readlane(v, kWave - 1);
 }
 
 // New H from rho: hdr_density.hpp:296-300 (eta * kappa * (m / rho)^(1/3), capped).
@@ -292,29 +324,6 @@ __device__ __forceinline__ double dens_next_h(double eta_ksrh, double m, double 
 {
     const double h = eta_ksrh * cbrt_f64(m / dens);
     return h < hmax ? h : hmax;
-}
-
-// Per-i sums of the five grad-h partials over the slices of a full sweep.
-// The mixed kernel's reduction buffer holds two FP64 quantities, so the five
-// are combined two, two and one at a time.
-template <bool MIXED>
-__device__ __forceinline__ void dens_reduce_grad(double (&acc)[5], double *red, const Map &M, int lane)
-{
-    if (!MIXED) {
-        slice_reduce<5>(acc, red, M, lane);
-        return;
-    }
-    double a[2] = {acc[0], acc[1]};
-    slice_reduce<2>(a, red, M, lane);
-    double b[2] = {acc[2], acc[3]};
-    slice_reduce<2>(b, red, M, lane);
-    double c[1] = {acc[4]};
-    slice_reduce<1>(c, red, M, lane);
-    acc[0] = a[0];
-    acc[1] = a[1];
-    acc[2] = b[0];
-    acc[3] = b[1];
-    acc[4] = c[0];
 }
 
 // Walks whose j-list holds at most kDensCap records keep the whole list in
@@ -329,6 +338,13 @@ __device__ __forceinline__ void dens_reduce_grad(double (&acc)[5], double *red, 
 // together; the lanes are shared out so that every taken i needs at most
 // T = ceil(C / (64 - n)) steps (C entries over n particles).  If an H_k of
 // the iteration exceeds R_i the chunk continues with full sweeps.
+//
+// NW = 2: two waves per walk share the staging, the marking (a tile each in
+// turn) and the h-passes (step or tile t belongs to wave t mod 2);
+// per-particle work is wave 0's, and so is the mixed grad-h pass, whose FP32
+// sums depend on their order.  FP64 sums that the waves share are formed by
+// parity, the even steps (tiles) in order and the odd ones, and added, whatever
+// NW is: results do not depend on it, bit for bit.
 constexpr int kDensCap = 256;        // largest resident capacity (instantiated: 192, 256)
 constexpr int kDensComp = 1728;
 constexpr int kDensR = 12;           // members per lane held in registers for the h-passes
@@ -363,10 +379,73 @@ __device__ __forceinline__ DensI dens_load_i(const sphk_dens_src &pi, int i)
                  pi.id[i]};
 }
 
-// Lists longer than kDensCap: every sweep streams the list through one
-// 64-record LDS tile.
-template <bool MIXED>
-__device__ void density_streaming(int lane, const Map &M, int i, int jb, int je,
+// The parities that one of NW waves sums: kPar of them, wave wv's u-th is
+// wv + u.
+template <int NW>
+constexpr int kPar = 2 / NW;
+
+// Combination of the waves' values of one lane, kWave apart.
+template <int NW>
+__device__ __forceinline__ double wave_comb(const double *r)
+{
+    if constexpr (NW == 1) return r[0];
+    return r[0] + r[kWave];
+}
+
+// An h-pass's sums and neighbour counts of the waves over lanes first, first +
+// step, ... (cnt of them), in one loop: it is bound by the latency of its LDS
+// reads (1.46 -> 1.44 ms mixed, 1.60 -> 1.54 FP64 at 10^6 particles against a
+// loop each).
+template <int NW>
+__device__ __forceinline__ void lanes_pass(const double *r, const int *rn, int first, int cnt, int step, double &sum,
+                                           long long &n)
+{
+    double s = wave_comb<NW>(r + first);
+    int c = rn[first] + (NW == 2 ? rn[kWave + first] : 0);
+#pragma unroll 4
+    for (int t = 1; t < cnt; t++) {
+        const int l = first + t * step;
+        s += wave_comb<NW>(r + l);
+        c += rn[l] + (NW == 2 ? rn[kWave + l] : 0);
+    }
+    sum = s;
+    n = c;
+}
+
+// Per-particle sums of five quantities over the lanes of each particle; valid where `owner`.  ALL: both waves hold
+// parts of them; else wave 0 alone.
+template <int NW, bool ALL>
+__device__ __forceinline__ void dens_sum5(const double (&part)[5], double (&acc)[5], double *red, int wv, int lane,
+                                          bool owner, int cnt, int step)
+{
+    constexpr int kN = ALL ? NW : 1;
+#pragma unroll
+    for (int q0 = 0; q0 < 5; q0 += 2) {
+        const bool two = q0 + 1 < 5;
+        __syncthreads();
+        if (ALL || wv == 0) {
+            red[wv * kWave + lane] = part[q0];
+            if (two) red[(NW + wv) * kWave + lane] = part[q0 + 1];
+        }
+        __syncthreads();
+        if (owner) {
+            const double *r = red + lane, *r2 = red + NW * kWave + lane;
+            double a = wave_comb<kN>(r), b = two ? wave_comb<kN>(r2) : 0.;
+#pragma unroll 4
+            for (int t = 1; t < cnt; t++) {
+                a += wave_comb<kN>(r + t * step);
+                if (two) b += wave_comb<kN>(r2 + t * step);
+            }
+            acc[q0] = a;
+            if (two) acc[q0 + 1] = b;
+        }
+    }
+}
+
+// Lists longer than kDensCap: every sweep streams the list through 64-record
+// LDS tiles, one per wave.
+template <bool MIXED, int NW>
+__device__ void density_streaming(int lane, int wv, const Map &M, int i, int jb, int je,
                                   const int32_t *__restrict__ j_idx, const sphk_dens_src &pi,
                                   const sphk_dens_src &pj, const sphk_dens_out &out, double eta_ksrh,
                                   double hmax, double4 *sp, R4<real_t<MIXED>> *sv, double *red,
@@ -375,34 +454,48 @@ __device__ void density_streaming(int lane, const Map &M, int i, int jb, int je,
     using R = real_t<MIXED>;
     const int ntile = (je - jb + kTile - 1) / kTile;
     const DensI I = dens_load_i(pi, i);
+    const bool owner = M.lead && wv == 0;
+    int *redn = reinterpret_cast<int *>(red + NW * kWave);
     double hs = I.ksr;
     double dens = 0.;
     long long np = 0;
+    double4 *const tp = sp + wv * kTile;
+    R4<R> *const tv = sv + wv * kTile;
 
     for (int rep = 0; rep < 3; rep++) {
         const double hi = 1. / hs;
         const double hi3 = hi * hi * hi;
-        Pass1 a{0., 0};
-        for (int t = 0; t < ntile; t++) {
-            __syncthreads();
-            dens_stage<MIXED>(lane, jb + t * kTile, je, j_idx, pj, sp, sv, false);
-            __syncthreads();
-            const int nt = min(kTile, je - jb - t * kTile);   // records of this tile
-            int k = M.slice;
-            for (; k + 3 * M.S < nt; k += 4 * M.S) {
-                const double4 j0 = sp[k], j1 = sp[k + M.S], j2 = sp[k + 2 * M.S], j3 = sp[k + 3 * M.S];
-                dens_pass1_pair(j0, I.x, I.y, I.z, hi, hi3, a);
-                dens_pass1_pair(j1, I.x, I.y, I.z, hi, hi3, a);
-                dens_pass1_pair(j2, I.x, I.y, I.z, hi, hi3, a);
-                dens_pass1_pair(j3, I.x, I.y, I.z, hi, hi3, a);
+        double sum = 0.;
+        int nq = 0;
+#pragma unroll
+        for (int u = 0; u < kPar<NW>; u++) {
+            double P = 0.;
+            for (int t = wv + u; t < ntile; t += 2) {
+                wave_sync();
+                dens_stage<MIXED>(lane, jb + t * kTile, je, j_idx, pj, tp, tv, false);
+                wave_sync();
+                Pass1 a{0., 0};
+                const int nt = min(kTile, je - jb - t * kTile);   // records of this tile
+                int k = M.slice;
+                for (; k + 3 * M.S < nt; k += 4 * M.S) {
+                    const double4 j0 = tp[k], j1 = tp[k + M.S], j2 = tp[k + 2 * M.S], j3 = tp[k + 3 * M.S];
+                    dens_pass1_pair(j0, I.x, I.y, I.z, hi, hi3, a);
+                    dens_pass1_pair(j1, I.x, I.y, I.z, hi, hi3, a);
+                    dens_pass1_pair(j2, I.x, I.y, I.z, hi, hi3, a);
+                    dens_pass1_pair(j3, I.x, I.y, I.z, hi, hi3, a);
+                }
+                for (; k < nt; k += M.S) dens_pass1_pair(tp[k], I.x, I.y, I.z, hi, hi3, a);
+                P += a.rh;
+                nq += a.nj;
             }
-            for (; k < nt; k += M.S) dens_pass1_pair(sp[k], I.x, I.y, I.z, hi, hi3, a);
+            sum = u == 0 ? P : sum + P;
         }
-        double v[2] = {a.rh, (double)a.nj};
-        slice_reduce<2>(v, red, M, lane);
-        if (M.lead) {
-            dens = v[0];
-            np = (long long)v[1];
+        __syncthreads();
+        red[wv * kWave + lane] = sum;
+        redn[wv * kWave + lane] = nq;
+        __syncthreads();
+        if (owner) {
+            lanes_pass<NW>(red, redn, M.il, M.S, M.ni, dens, np);
             shs[M.il] = dens_next_h(eta_ksrh, I.m, dens, hmax);
         }
         __syncthreads();
@@ -413,51 +506,65 @@ __device__ void density_streaming(int lane, const Map &M, int i, int jb, int je,
     const R hi = (R)hi_d;
     const R hi4 = (R)(hi_d * (hi_d * hi_d * hi_d));
     const R vx = (R)I.vx, vy = (R)I.vy, vz = (R)I.vz;
-    double acc[5] = {0., 0., 0., 0., 0.};
-    for (int t = 0; t < ntile; t++) {
-        __syncthreads();
-        dens_stage<MIXED>(lane, jb + t * kTile, je, j_idx, pj, sp, sv, true);
-        __syncthreads();
-        Pass2<R> a{R(0), R(0), R(0), R(0), R(0)};
-        const int nt = min(kTile, je - jb - t * kTile);
-        int k = M.slice;
-        for (; k + M.S < nt; k += 2 * M.S) {
-            dens_pass2_pair<R>(sp[k], sv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-            dens_pass2_pair<R>(sp[k + M.S], sv[k + M.S], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+    double part[5];
+#pragma unroll
+    for (int u = 0; u < kPar<NW>; u++) {
+        double P[5] = {0., 0., 0., 0., 0.};
+        for (int t = wv + u; t < ntile; t += 2) {
+            wave_sync();
+            dens_stage<MIXED>(lane, jb + t * kTile, je, j_idx, pj, tp, tv, true);
+            wave_sync();
+            Pass2<R> a{R(0), R(0), R(0), R(0), R(0)};
+            const int nt = min(kTile, je - jb - t * kTile);
+            int k = M.slice;
+            for (; k + M.S < nt; k += 2 * M.S) {
+                dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+                dens_pass2_pair<R>(tp[k + M.S], tv[k + M.S], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+            }
+            for (; k < nt; k += M.S)
+                dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+            P[0] += (double)a.g;
+            P[1] += (double)a.dv;
+            P[2] += (double)a.rx;
+            P[3] += (double)a.ry;
+            P[4] += (double)a.rz;
         }
-        for (; k < nt; k += M.S)
-            dens_pass2_pair<R>(sp[k], sv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-        acc[0] += (double)a.g;
-        acc[1] += (double)a.dv;
-        acc[2] += (double)a.rx;
-        acc[3] += (double)a.ry;
-        acc[4] += (double)a.rz;
+#pragma unroll
+        for (int q = 0; q < 5; q++) part[q] = u == 0 ? P[q] : part[q] + P[q];
     }
-    dens_reduce_grad<MIXED>(acc, red, M, lane);
-    if (M.lead) dens_finish(out, i, acc, dens, np, hs, I.rs);
+    double acc[5];
+    dens_sum5<NW, true>(part, acc, red, wv, lane, owner, M.S, M.ni);
+    if (owner) dens_finish(out, i, acc, dens, np, hs, I.rs);
 }
 
-// Launch bound: 3 waves per SIMD (at most 168 VGPRs; a few spill), the
-// occupancy the 192-record LDS layout allows.
-template <bool MIXED, int CAP, bool PERSIST>
-__global__ __launch_bounds__(kWave, 3) void density_kernel(
+// Launch bound: 3 waves per SIMD (at most 168 VGPRs; a few spill).  Between its
+// sweeps the kernel is bound by latency, so scans go through DPP, lane sums
+// run in one loop for all quantities, and distances take sqrt_ieee: 10^6
+// particles, one wave per walk, 1.38 -> 1.30 ms mixed and 1.67 -> 1.44 FP64
+// (there also 20 instead of 22 KB of LDS: 8 walks per CU).
+template <bool MIXED, int CAP, bool PERSIST, int NW>
+__global__ __launch_bounds__(kWave *NW, 3) void density_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_dens_src pi, sphk_dens_src pj, sphk_dens_out out,
     double eta_ksrh, double hmax, int *queue)
 {
     using R = real_t<MIXED>;
-    static_assert(CAP % kTile == 0 && CAP <= kDensCap, "list capacity");
-    constexpr int kWords = CAP / kTile;
+    static_assert(CAP % kTile == 0 && CAP <= kDensCap && CAP >= NW * kTile, "list capacity");
+    static_assert(!PERSIST || NW == 1, "persistent launches take one wave per walk");
+    constexpr int kWords = CAP / kTile, kMine = (kWords + NW - 1) / NW;   // tiles, and those a wave marks
     constexpr int kDensPad = CAP;   // inert record after the list, target of idle steps
-    constexpr int kRed = MIXED ? 2 * kWave : 5 * kWave;   // doubles (mixed reduces two at a time)
+    constexpr int kRegs = kDensR / NW;
+    static_assert((NW == 1 || NW == 2) && kDensR % 2 == 0, "steps are dealt to the waves by parity");
     __shared__ double4 sp[CAP + 1];     // x, y, z, m
     __shared__ R4<R> sv[CAP + 1];       // vx, vy, vz, id
     __shared__ uint8_t cidx[kDensComp];
-    __shared__ double red[kRed];
+    __shared__ double red[2 * NW * kWave];
     __shared__ double shs[kWave];
     __shared__ int s_own[kWave];
     __shared__ uint16_t s_ci[kWave], s_coff[kWave];
-    int *s_cnt = reinterpret_cast<int *>(red);   // membership counts, before any reduction
+    int *const redn = reinterpret_cast<int *>(red + NW * kWave);
+    uint8_t *const s_cnt = reinterpret_cast<uint8_t *>(red);   // membership counts [lane][tile], before any reduction
+    const int wv = NW > 1 ? (int)threadIdx.x / kWave : 0;
 
     auto walk = [&](const int w, const int lane) {
         const int ib = i_off[w], ie = i_off[w + 1];
@@ -468,31 +575,32 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
         if (nj > CAP) {
             for (int c0 = ib; c0 < ie; c0 += kWave) {
                 const Map M(min(kWave, ie - c0), lane);
-                density_streaming<MIXED>(lane, M, c0 + M.il, jb, je, j_idx, pi, pj, out, eta_ksrh, hmax,
-                                         sp, sv, red, shs);
+                density_streaming<MIXED, NW>(lane, wv, M, c0 + M.il, jb, je, j_idx, pi, pj, out, eta_ksrh, hmax,
+                                             sp, sv, red, shs);
             }
             return;
         }
 
         // one burst: every record of the list, padded to whole tiles, plus the inert record
-        for (int e = lane; e < ntile * kTile; e += kWave) dens_stage<MIXED>(e, jb, je, j_idx, pj, sp, sv, true);
-        if (lane == 0) dens_stage<MIXED>(kDensPad, 0, 0, j_idx, pj, sp, sv, true);
+        for (int e = wv * kWave + lane; e < ntile * kTile; e += kWave * NW)
+            dens_stage<MIXED>(e, jb, je, j_idx, pj, sp, sv, true);
+        if (lane == 0 && wv == 0) dens_stage<MIXED>(kDensPad, 0, 0, j_idx, pj, sp, sv, true);
 
         for (int c0 = ib; c0 < ie;) {
             const Map M(min(kWave, ie - c0), lane);
             __syncthreads();   // staging done; LDS of the previous chunk no longer read
 
-            // -- membership sweep: lane (i, slice) marks its records within R_i
-            uint64_t wd[kWords];
-            int cnt = 0;
+            // -- membership sweep: lane (i, slice) marks its records within R_i, tile by tile
+            uint64_t wd[kMine];
             {
                 const int i = c0 + M.il;
                 const double px = pi.x[i], py = pi.y[i], pz = pi.z[i];
                 const double h0 = pi.ksr[i], rs = pi.rs[i];
                 const double rme = (h0 > rs ? h0 : rs) * (1. + 1e-12);
                 const double rm2 = rme * rme;
-    #pragma unroll
-                for (int t = 0; t < kWords; t++) {
+#pragma unroll
+                for (int u = 0; u < kMine; u++) {
+                    const int t = wv + NW * u;
                     uint64_t b = 0;
                     if (t < ntile) {
                         const double4 *tp = sp + t * kTile;
@@ -514,36 +622,49 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
                             b |= (uint64_t)(dx * dx + dy * dy + dz * dz < rm2) << k;
                         }
                     }
-                    wd[t] = b;
-                    cnt += __popcll(b);
+                    wd[u] = b;
+                    if (t < 4) s_cnt[4 * lane + t] = (uint8_t)__popcll(b);
                 }
-                s_cnt[lane] = cnt;
+                if (kWords < 4 && wv == 0) s_cnt[4 * lane + 3] = 0;
             }
             __syncthreads();
+            // entries of a lane over its tiles (at most 256: four bytes summed)
+            auto lane_cnt = [&](int l) {
+                return (int)__builtin_amdgcn_sad_u8(reinterpret_cast<const uint32_t *>(s_cnt)[l], 0u, 0u);
+            };
             int start = 0, ci = 0;
-            if (M.slice < M.S)
-                for (int s2 = 0; s2 < M.slice; s2++) start += s_cnt[M.il + M.ni * s2];
-            if (M.lead)
-                for (int s2 = 0; s2 < M.S; s2++) ci += s_cnt[M.il + M.ni * s2];
+#pragma unroll 4
+            for (int s2 = 0; s2 < M.S; s2++) {
+                const int c = lane_cnt(M.il + M.ni * s2);
+                start += s2 < M.slice ? c : 0;
+                ci += c;
+            }
+            ci = M.lead ? ci : 0;
+            const uint32_t own_cnt = reinterpret_cast<const uint32_t *>(s_cnt)[lane];
             // take the leading i-particles whose lists fit in kDensComp entries
             // (every single list fits: c_i <= kDensCap)
-            const int incl = wave_scan_incl(ci, lane);   // leads are lanes 0 .. ni-1
+            const int incl = wave_scan_incl(ci);   // leads are lanes 0 .. ni-1
             const bool fits = M.lead && incl <= kDensComp;
             const int n_take = __popcll(__ballot(fits));
-            const int total = __shfl(incl, n_take - 1, kWave);
+            const int total = __builtin_amdgcn_readlane(incl, n_take - 1);
             const bool take = M.il < n_take;             // lane works on a taken i
 
-            if (M.lead && take) {
-                s_coff[M.il] = (uint16_t)(incl - ci);
-                s_ci[M.il] = (uint16_t)ci;
+            if (wv == 0) {
+                if (M.lead && take) {
+                    s_coff[M.il] = (uint16_t)(incl - ci);
+                    s_ci[M.il] = (uint16_t)ci;
+                }
+                s_own[lane] = -1;
             }
-            s_own[lane] = -1;
             __syncthreads();
             if (take && M.slice < M.S) {
-                int o = s_coff[M.il] + start;
-    #pragma unroll
-                for (int t = 0; t < kWords; t++) {
-                    uint64_t b = wd[t];
+                const int o0 = s_coff[M.il] + start;
+#pragma unroll
+                for (int u = 0; u < kMine; u++) {
+                    const int t = wv + NW * u;
+                    uint64_t b = t < kWords ? wd[u] : 0;
+                    // entries of the lane's tiles before t
+                    int o = o0 + (t == 0 ? 0 : (int)__builtin_amdgcn_sad_u8(own_cnt << (8 * (4 - min(t, 4))), 0u, 0u));
                     while (b) {
                         cidx[o++] = (uint8_t)(t * kTile + __builtin_ctzll(b));
                         b &= b - 1;
@@ -553,14 +674,15 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
             // lanes per taken i: max(1, ceil(c_i / T)), T = ceil(C / (64 - n)); they sum to <= 64
             const int tsteps = n_take < kWave ? max(1, (total + (kWave - n_take) - 1) / (kWave - n_take)) : 1;
             const int si = (M.lead && take) ? (n_take < kWave ? max(1, (ci + tsteps - 1) / tsteps) : 1) : 0;
-            const int lincl = wave_scan_incl(si, lane);
-            if (si > 0)
+            const int lincl = wave_scan_incl(si);
+            if (si > 0 && wv == 0)
                 for (int s2 = 0; s2 < si; s2++) s_own[lincl - si + s2] = M.il | (s2 << 8) | (si << 16);
             __syncthreads();
             const int own = s_own[lane];
 
-            // lane's particle and compacted range; every lane runs the wave's
-            // largest step count, idle steps read the inert record
+            // lane's particle and compacted range (the same in every wave);
+            // every lane runs the wave's largest step count, idle steps read
+            // the inert record
             int my = own >= 0 ? (own & 0xff) : 0;
             int e0 = 0, n_e = 0, stride = 1;
             const uint8_t *myidx = cidx;
@@ -572,139 +694,26 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
             }
             const int nsteps = wave_max(n_e > e0 ? (n_e - e0 + stride - 1) / stride : 0);
             bool compact = true;
-            bool owner = own >= 0 && e0 == 0;
+            bool owner = own >= 0 && e0 == 0 && wv == 0;
             DensI I = dens_load_i(pi, c0 + my);
             const Map MF(n_take, lane);   // full sweeps over the taken i-particles
             double hs = I.ksr;
             double dens = 0.;
             long long np = 0;
 
-            // -- three fixed-point passes: rho(H_k), n(H_k), H_{k+1} (hdr_density.hpp:264-302).
-            // When every lane has at most kDensR members, their exact distances
-            // and masses are held in registers for the passes (one sqrt per
-            // member instead of one rsqrt refinement per member and pass); the
-            // passes that remain after an H beyond R_i run below.
-            int rep0 = 0;
-            if (nsteps <= kDensR) {
-                double rr[kDensR], mm[kDensR];
-    #pragma unroll
-                for (int t = 0; t < kDensR; t++) {
-                    if (t < nsteps) {
-                        const int e = e0 + t * stride;
-                        const double4 j = sp[e < n_e ? myidx[e] : kDensPad];
-                        rr[t] = exact_r(I.x - j.x, I.y - j.y, I.z - j.z);
-                        mm[t] = j.w;
-                    }
-                }
-                for (; rep0 < 3; rep0++) {
-                    const double hi = 1. / hs;
-                    const double hi3 = hi * hi * hi;
-                    double rh = 0.;
-                    int nq = 0;
-    #pragma unroll
-                    for (int t = 0; t < kDensR; t++) {
-                        if (t < nsteps) {
-                            const double q = rr[t] * hi;
-                            rh += mm[t] * hi3 * kernel0th(q);
-                            nq += (q < 1.) ? 1 : 0;
-                        }
-                    }
-                    __syncthreads();
-                    red[lane] = rh;
-                    red[kWave + lane] = (double)nq;
-                    __syncthreads();
-                    double v0 = red[lane], v1 = red[kWave + lane];
-                    if (owner)
-                        for (int t = 1; t < stride; t++) {
-                            v0 += red[lane + t];
-                            v1 += red[kWave + lane + t];
-                        }
-                    int viol = 0;
-                    if (owner) {
-                        dens = v0;
-                        np = (long long)v1;
-                        const double hnew = dens_next_h(eta_ksrh, I.m, dens, hmax);
-                        shs[my] = hnew;
-                        viol = hnew > (I.ksr > I.rs ? I.ksr : I.rs);
-                    }
-                    if (__syncthreads_or(viol)) {   // full sweeps from the next pass on
-                        if (owner) {
-                            red[my] = dens;
-                            red[kWave + my] = (double)np;
-                        }
-                        __syncthreads();
-                        compact = false;
-                        my = MF.il;
-                        owner = MF.lead;
-                        I = dens_load_i(pi, c0 + my);
-                        dens = red[my];
-                        np = (long long)red[kWave + my];
-                        hs = shs[my];
-                        rep0++;
-                        break;
-                    }
-                    hs = shs[my];
-                }
-            }
-            for (int rep = rep0; rep < 3; rep++) {
-                const double hi = 1. / hs;
-                const double hi3 = hi * hi * hi;
-                Pass1 a{0., 0};
-                double v[2];
-                if (compact) {
-                    int st = 0, e = e0;
-                    for (; st + 4 <= nsteps; st += 4, e += 4 * stride) {
-                        const int k0 = e < n_e ? myidx[e] : kDensPad;
-                        const int k1 = e + stride < n_e ? myidx[e + stride] : kDensPad;
-                        const int k2 = e + 2 * stride < n_e ? myidx[e + 2 * stride] : kDensPad;
-                        const int k3 = e + 3 * stride < n_e ? myidx[e + 3 * stride] : kDensPad;
-                        const double4 j0 = sp[k0], j1 = sp[k1], j2 = sp[k2], j3 = sp[k3];
-                        dens_pass1_pair(j0, I.x, I.y, I.z, hi, hi3, a);
-                        dens_pass1_pair(j1, I.x, I.y, I.z, hi, hi3, a);
-                        dens_pass1_pair(j2, I.x, I.y, I.z, hi, hi3, a);
-                        dens_pass1_pair(j3, I.x, I.y, I.z, hi, hi3, a);
-                    }
-                    for (; st < nsteps; st++, e += stride)
-                        dens_pass1_pair(sp[e < n_e ? myidx[e] : kDensPad], I.x, I.y, I.z, hi, hi3, a);
-                    __syncthreads();
-                    red[lane] = a.rh;
-                    red[kWave + lane] = (double)a.nj;
-                    __syncthreads();
-                    v[0] = red[lane];
-                    v[1] = red[kWave + lane];
-                    if (owner)
-                        for (int t = 1; t < stride; t++) {
-                            v[0] += red[lane + t];
-                            v[1] += red[kWave + lane + t];
-                        }
-                } else {
-                    for (int t = 0; t < ntile; t++) {
-                        const double4 *tp = sp + t * kTile;
-                        const int nt = min(kTile, nj - t * kTile);
-                        int k = MF.slice;
-                        for (; k + 3 * MF.S < nt; k += 4 * MF.S) {
-                            const double4 j0 = tp[k], j1 = tp[k + MF.S], j2 = tp[k + 2 * MF.S], j3 = tp[k + 3 * MF.S];
-                            dens_pass1_pair(j0, I.x, I.y, I.z, hi, hi3, a);
-                            dens_pass1_pair(j1, I.x, I.y, I.z, hi, hi3, a);
-                            dens_pass1_pair(j2, I.x, I.y, I.z, hi, hi3, a);
-                            dens_pass1_pair(j3, I.x, I.y, I.z, hi, hi3, a);
-                        }
-                        for (; k < nt; k += MF.S) dens_pass1_pair(tp[k], I.x, I.y, I.z, hi, hi3, a);
-                    }
-                    v[0] = a.rh;
-                    v[1] = (double)a.nj;
-                    slice_reduce<2>(v, red, MF, lane);
-                }
+            // After a pass's sums (in red, redn): rho, n and the next H of the
+            // owners; with an H beyond R_i the compacted lists are incomplete:
+            // full sweeps from the next pass on, wave 0's lead lanes of MF take
+            // over ownership.
+            auto pass_end = [&]() {
                 int viol = 0;
                 if (owner) {
-                    dens = v[0];
-                    np = (long long)v[1];
+                    const int first = compact ? lane : MF.il, cnt = compact ? stride : MF.S, step = compact ? 1 : MF.ni;
+                    lanes_pass<NW>(red, redn, first, cnt, step, dens, np);
                     const double hnew = dens_next_h(eta_ksrh, I.m, dens, hmax);
                     shs[my] = hnew;
                     viol = compact && hnew > (I.ksr > I.rs ? I.ksr : I.rs);
                 }
-                // an H beyond R_i leaves the compacted lists incomplete: full
-                // sweeps from here on, the lead lanes of MF take over ownership
                 if (__syncthreads_or(viol)) {
                     if (owner) {
                         red[my] = dens;
@@ -713,12 +722,92 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
                     __syncthreads();
                     compact = false;
                     my = MF.il;
-                    owner = MF.lead;
+                    owner = MF.lead && wv == 0;
                     I = dens_load_i(pi, c0 + my);
                     dens = red[my];
                     np = (long long)red[kWave + my];
                 }
                 hs = shs[my];
+            };
+            auto pass_put = [&](double sum, int nq) {
+                __syncthreads();
+                red[wv * kWave + lane] = sum;
+                redn[wv * kWave + lane] = nq;
+                __syncthreads();
+            };
+
+            // -- three fixed-point passes: rho(H_k), n(H_k), H_{k+1} (hdr_density.hpp:264-302).
+            // When every lane has at most kDensR members, their exact distances
+            // and masses are held in registers for the passes (one sqrt per
+            // member instead of one rsqrt refinement per member and pass); the
+            // passes that remain after an H beyond R_i run below.
+            int rep0 = 0;
+            if (nsteps <= kDensR) {
+                double rr[kRegs], mm[kRegs];
+#pragma unroll
+                for (int u = 0; u < kRegs; u++) {
+                    const int t = wv + NW * u;
+                    if (t < nsteps) {
+                        const int e = e0 + t * stride;
+                        const double4 j = sp[e < n_e ? myidx[e] : kDensPad];
+                        rr[u] = exact_r(I.x - j.x, I.y - j.y, I.z - j.z);
+                        mm[u] = j.w;
+                    }
+                }
+                for (; rep0 < 3 && compact; rep0++) {
+                    const double hi = 1. / hs;
+                    const double hi3 = hi * hi * hi;
+                    double sum = 0.;
+                    int nq = 0;
+#pragma unroll
+                    for (int v = 0; v < kPar<NW>; v++) {
+                        double P = 0.;
+#pragma unroll
+                        for (int u = v; u < kRegs; u += kPar<NW>) {
+                            if (wv + NW * u < nsteps) {
+                                const double q = rr[u] * hi;
+                                P += mm[u] * hi3 * kernel0th(q);
+                                nq += (q < 1.) ? 1 : 0;
+                            }
+                        }
+                        sum = v == 0 ? P : sum + P;
+                    }
+                    pass_put(sum, nq);
+                    pass_end();
+                }
+            }
+            for (int rep = rep0; rep < 3; rep++) {
+                const double hi = 1. / hs;
+                const double hi3 = hi * hi * hi;
+                Pass1 a[kPar<NW>] = {};
+                if (compact) {
+                    // four members in flight, of both parities where the wave has both
+                    for (int t0 = 0; t0 < nsteps; t0 += 4 * NW) {
+                        double4 j[4];
+#pragma unroll
+                        for (int m = 0; m < 4; m++) {
+                            const int e = e0 + (t0 + wv + m * NW) * stride;
+                            j[m] = sp[e < n_e ? myidx[e] : kDensPad];
+                        }
+#pragma unroll
+                        for (int m = 0; m < 4; m++)
+                            if (t0 + m * NW < nsteps)
+                                dens_pass1_pair(j[m], I.x, I.y, I.z, hi, hi3, a[m % kPar<NW>]);
+                    }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < kPar<NW>; u++)
+                        for (int t = wv + u; t < ntile; t += 2) {
+                            const double4 *tp = sp + t * kTile;
+                            const int nt = min(kTile, nj - t * kTile);
+                            for (int k = MF.slice; k < nt; k += MF.S)
+                                dens_pass1_pair(tp[k], I.x, I.y, I.z, hi, hi3, a[u]);
+                        }
+                }
+                const double sum = NW == 1 ? a[0].rh + a[kPar<NW> - 1].rh : a[0].rh;
+                const int nq = NW == 1 ? a[0].nj + a[kPar<NW> - 1].nj : a[0].nj;
+                pass_put(sum, nq);
+                pass_end();
             }
 
             // -- grad-h, divergence, curl with H_3 (hdr_density.hpp:304-349)
@@ -726,67 +815,65 @@ __global__ __launch_bounds__(kWave, 3) void density_kernel(
             const R hi = (R)hi_d;
             const R hi4 = (R)(hi_d * (hi_d * hi_d * hi_d));
             const R vx = (R)I.vx, vy = (R)I.vy, vz = (R)I.vz;
-            double acc[5] = {0., 0., 0., 0., 0.};
-            if (compact) {
-                // pair terms summed in R over at most 16 entries, then folded
+            double part[5] = {0., 0., 0., 0., 0.}, acc[5];
+            auto pair2 = [&](int e, Pass2<R> &a) {
+                const int k = e < n_e ? myidx[e] : kDensPad;
+                dens_pass2_pair<R>(sp[k], sv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+            };
+            auto add2 = [&](double (&p)[5], const Pass2<R> &a) {
+                p[0] += (double)a.g;
+                p[1] += (double)a.dv;
+                p[2] += (double)a.rx;
+                p[3] += (double)a.ry;
+                p[4] += (double)a.rz;
+            };
+            if (compact && MIXED) {
+                // pair terms summed in FP32 over at most 16 entries, then folded
                 // into FP64 (as the full sweep folds each 64-record tile)
-                Pass2<R> a{R(0), R(0), R(0), R(0), R(0)};
-                double part[5] = {0., 0., 0., 0., 0.};
-                auto fold = [&]() {
-                    part[0] += (double)a.g;
-                    part[1] += (double)a.dv;
-                    part[2] += (double)a.rx;
-                    part[3] += (double)a.ry;
-                    part[4] += (double)a.rz;
-                    a = Pass2<R>{R(0), R(0), R(0), R(0), R(0)};
-                };
-                int st = 0, e = e0;
-                for (; st + 2 <= nsteps; st += 2, e += 2 * stride) {
-                    const int k0 = e < n_e ? myidx[e] : kDensPad;
-                    const int k1 = e + stride < n_e ? myidx[e + stride] : kDensPad;
-                    dens_pass2_pair<R>(sp[k0], sv[k0], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-                    dens_pass2_pair<R>(sp[k1], sv[k1], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-                    if ((st & 14) == 14) fold();
-                }
-                if (st < nsteps) {
-                    const int k0 = e < n_e ? myidx[e] : kDensPad;
-                    dens_pass2_pair<R>(sp[k0], sv[k0], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-                }
-                fold();
-                // per-i sums over the i's lanes in FP64, two quantities per round
-                for (int q0 = 0; q0 < 5; q0 += 2) {
-                    const int nq = q0 + 1 < 5 ? 2 : 1;
-                    __syncthreads();
-                    for (int q = 0; q < nq; q++) red[q * kWave + lane] = part[q0 + q];
-                    __syncthreads();
-                    if (owner)
-                        for (int q = 0; q < nq; q++) {
-                            double s = red[q * kWave + lane];
-                            for (int t = 1; t < stride; t++) s += red[q * kWave + lane + t];
-                            acc[q0 + q] = s;
-                        }
-                }
-            } else {
-                for (int t = 0; t < ntile; t++) {
-                    const double4 *tp = sp + t * kTile;
-                    const R4<R> *tv = sv + t * kTile;
+                if (wv == 0) {
                     Pass2<R> a{R(0), R(0), R(0), R(0), R(0)};
-                    const int nt = min(kTile, nj - t * kTile);   // records of this tile
-                    int k = MF.slice;
-                    for (; k + MF.S < nt; k += 2 * MF.S) {
-                        dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-                        dens_pass2_pair<R>(tp[k + MF.S], tv[k + MF.S], I.x, I.y, I.z, vx, vy, vz, I.id, hi,
-                                           hi4, a);
+                    int st = 0, e = e0;
+                    for (; st + 2 <= nsteps; st += 2, e += 2 * stride) {
+                        pair2(e, a);
+                        pair2(e + stride, a);
+                        if ((st & 14) == 14) {
+                            add2(part, a);
+                            a = Pass2<R>{R(0), R(0), R(0), R(0), R(0)};
+                        }
                     }
-                    for (; k < nt; k += MF.S)
-                        dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
-                    acc[0] += (double)a.g;
-                    acc[1] += (double)a.dv;
-                    acc[2] += (double)a.rx;
-                    acc[3] += (double)a.ry;
-                    acc[4] += (double)a.rz;
+                    if (st < nsteps) pair2(e, a);
+                    add2(part, a);
                 }
-                dens_reduce_grad<MIXED>(acc, red, MF, lane);
+                dens_sum5<NW, false>(part, acc, red, wv, lane, owner, stride, 1);
+            } else {
+#pragma unroll
+                for (int u = 0; u < kPar<NW>; u++) {
+                    double P[5] = {0., 0., 0., 0., 0.};
+                    Pass2<R> a{R(0), R(0), R(0), R(0), R(0)};
+                    if (compact) {
+                        for (int t = wv + u; t < nsteps; t += 2) pair2(e0 + t * stride, a);
+                        add2(P, a);
+                    } else {
+                        for (int t = wv + u; t < ntile; t += 2) {
+                            const double4 *tp = sp + t * kTile;
+                            const R4<R> *tv = sv + t * kTile;
+                            const int nt = min(kTile, nj - t * kTile);   // records of this tile
+                            a = Pass2<R>{R(0), R(0), R(0), R(0), R(0)};
+                            int k = MF.slice;
+                            for (; k + MF.S < nt; k += 2 * MF.S) {
+                                dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+                                dens_pass2_pair<R>(tp[k + MF.S], tv[k + MF.S], I.x, I.y, I.z, vx, vy, vz, I.id, hi,
+                                                   hi4, a);
+                            }
+                            for (; k < nt; k += MF.S)
+                                dens_pass2_pair<R>(tp[k], tv[k], I.x, I.y, I.z, vx, vy, vz, I.id, hi, hi4, a);
+                            add2(P, a);
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < 5; q++) part[q] = u == 0 ? P[q] : part[q] + P[q];
+                }
+                dens_sum5<NW, true>(part, acc, red, wv, lane, owner, compact ? stride : MF.S, compact ? 1 : MF.ni);
             }
             if (owner) dens_finish(out, c0 + my, acc, dens, np, hs, I.rs);
             c0 += n_take;
@@ -1273,7 +1360,7 @@ __global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(PERSI
     static_assert(NW == 1 || NW * kWaveBytes >= kRedBytes, "reduction buffer");
     __shared__ __attribute__((aligned(32))) char smem[NW * kWaveBytes];
     __shared__ R part[NW > 1 ? NW : 1][5][NW > 1 ? kWave : 1];   // the waves' block sums
-    const int wv = NW > 1 ? (int)threadIdx.x / kWave : 0;
+    const int wv = NW > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) : 0;
     char *mine = smem + wv * kWaveBytes;
     double *red = reinterpret_cast<double *>(smem);
 
@@ -1395,54 +1482,64 @@ static int persistent_grid(K kernel, int n_walk)
             hipLaunchKernelGGL(KERNEL, dim3(n_walk), dim3(kWave * (waves)), 0, st, __VA_ARGS__, nullptr); \
         }                                                                                                \
     } while (0)
-hipError_t launch_density(hipStream_t st, int n_walk, const int32_t *i_off, const int32_t *j_off,
+hipError_t launch_density(hipStream_t st, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                           const int32_t *j_idx, const sphk_dens_src &pi, const sphk_dens_src &pj,
                           const sphk_dens_out &out, double eta_ksrh, double hmax, bool mixed, int list_cap,
                           int *queue)
 {
     if (n_walk <= 0) return hipSuccess;
-#define SPHK_LAUNCH_D(M, CAPV)                                                                           \
-    SPHK_LAUNCH((density_kernel<M, CAPV, false>), (density_kernel<M, CAPV, true>), 1, n_walk, i_off, j_off, \
+#define SPHK_LAUNCH_D(M, CAPV, W)                                                                              \
+    SPHK_LAUNCH((density_kernel<M, CAPV, false, W>), (density_kernel<M, CAPV, true, 1>), W, n_walk, i_off, j_off, \
                 j_idx, pi, pj, out, eta_ksrh, hmax)
+#define SPHK_DENS(M, CAPV)                        \
+    do {                                          \
+        if (waves == 2)                           \
+            SPHK_LAUNCH_D(M, CAPV, 2);            \
+        else                                      \
+            SPHK_LAUNCH_D(M, CAPV, 1);            \
+    } while (0)
+    const int waves = waves_per_walk(n_walk, n_i, kDensRule);
     if (list_cap == 192) {
         if (mixed)
-            SPHK_LAUNCH_D(true, 192);
+            SPHK_DENS(true, 192);
         else
-            SPHK_LAUNCH_D(false, 192);
+            SPHK_DENS(false, 192);
     } else {
         if (mixed)
-            SPHK_LAUNCH_D(true, 256);
+            SPHK_DENS(true, 256);
         else
-            SPHK_LAUNCH_D(false, 256);
+            SPHK_DENS(false, 256);
     }
+#undef SPHK_DENS
 #undef SPHK_LAUNCH_D
     return hipGetLastError();
 }
 
-hipError_t launch_hydro(hipStream_t st, int n_walk, const int32_t *i_off, const int32_t *j_off,
+hipError_t launch_hydro(hipStream_t st, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                         const int32_t *j_idx, const sphk_hydro_src &pi, const sphk_hydro_src &pj,
                         const sphk_hydro_out &out, bool mixed, int *queue)
 {
     if (n_walk <= 0) return hipSuccess;
 #define SPHK_LAUNCH_H(M, W) \
     SPHK_LAUNCH((hydro_kernel<M, false, W>), (hydro_kernel<M, true, 1>), W, n_walk, i_off, j_off, j_idx, pi, pj, out)
-#define SPHK_LAUNCH_HM(W) SPHK_LAUNCH_H(true, W)
-#define SPHK_LAUNCH_HD(W) SPHK_LAUNCH_H(false, W)
-    switch (waves_per_walk(n_walk, mixed ? kHydroRule : kHydroF64Rule) + (mixed ? 0 : 8)) {
-    case 4: SPHK_LAUNCH_HM(4); break;
-    case 2: SPHK_LAUNCH_HM(2); break;
-    case 1: SPHK_LAUNCH_HM(1); break;
-    case 8 + 4: SPHK_LAUNCH_HD(4); break;
-    case 8 + 2: SPHK_LAUNCH_HD(2); break;
-    default: SPHK_LAUNCH_HD(1); break;
+    const int waves = waves_per_walk(n_walk, n_i, mixed ? kHydroRule : kHydroF64Rule);
+    if (mixed) {
+        if (waves == 4)
+            SPHK_LAUNCH_H(true, 4);
+        else
+            SPHK_LAUNCH_H(true, 1);
+    } else {
+        switch (waves) {
+        case 4: SPHK_LAUNCH_H(false, 4); break;
+        case 2: SPHK_LAUNCH_H(false, 2); break;
+        default: SPHK_LAUNCH_H(false, 1); break;
+        }
     }
-#undef SPHK_LAUNCH_HM
-#undef SPHK_LAUNCH_HD
 #undef SPHK_LAUNCH_H
     return hipGetLastError();
 }
 
-hipError_t launch_gravity(hipStream_t st, int n_walk, const int32_t *i_off, const int32_t *j_off,
+hipError_t launch_gravity(hipStream_t st, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                           const int32_t *j_idx, const sphk_grav_src &pj, const int32_t *s_off,
                           const int32_t *s_idx, const sphk_grav_src &ps, const sphk_grav_src &pi,
                           const sphk_grav_out &out, bool mixed, bool uniform, int *queue)
@@ -1466,7 +1563,7 @@ hipError_t launch_gravity(hipStream_t st, int n_walk, const int32_t *i_off, cons
     default: SPHK_LAUNCH_G(M, U, E, 1); break; \
     }
     const bool eta = out.eta != nullptr;
-    const int waves = waves_per_walk(n_walk, mixed && uniform ? kGravRelRule : kGravRule);
+    const int waves = waves_per_walk(n_walk, n_i, mixed && uniform ? kGravRelRule : kGravRule);
     if (mixed && uniform) {
         if (eta) SPHK_REL(true) else SPHK_REL(false)
     } else if (mixed) {

@@ -446,7 +446,7 @@ int *walk_queue(sphk_ctx *ctx)
 }
 }  // namespace
 
-int sphk_density_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+int sphk_density_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                      const int32_t *j_idx, sphk_dens_src pi, sphk_dens_src pj, sphk_dens_out out,
                      int precision, void *stream)
 {
@@ -462,7 +462,7 @@ int sphk_density_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int3
         return set_error(SPHK_E_ARG, "density: null field pointer");
     hipStream_t st = pick_stream(ctx, stream);
     Timer t(ctx, 0, st);
-    SPHK_HIP(launch_density(st, n_walk, i_off, j_off, j_idx, pi, pj, out,
+    SPHK_HIP(launch_density(st, n_walk, n_i, i_off, j_off, j_idx, pi, pj, out,
                             ctx->params.eta * ctx->params.ksrh, ctx->params.hmax,
                             precision == SPHK_MIXED, ctx->params.list_cap == 192 ? 192 : 256,
                             walk_queue(ctx)));
@@ -470,7 +470,14 @@ int sphk_density_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int3
     return SPHK_OK;
 }
 
-int sphk_hydro_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+int sphk_density_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                     const int32_t *j_idx, sphk_dens_src pi, sphk_dens_src pj, sphk_dens_out out,
+                     int precision, void *stream)
+{
+    return sphk_density_dev_n(ctx, n_walk, 0, i_off, j_off, j_idx, pi, pj, out, precision, stream);
+}
+
+int sphk_hydro_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                    const int32_t *j_idx, sphk_hydro_src pi, sphk_hydro_src pj, sphk_hydro_out out,
                    int precision, void *stream)
 {
@@ -491,13 +498,20 @@ int sphk_hydro_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_
         if (!fo[k]) return set_error(SPHK_E_ARG, "hydro: null output field %d", k);
     hipStream_t st = pick_stream(ctx, stream);
     Timer t(ctx, 1, st);
-    SPHK_HIP(launch_hydro(st, n_walk, i_off, j_off, j_idx, pi, pj, out, precision == SPHK_MIXED,
+    SPHK_HIP(launch_hydro(st, n_walk, n_i, i_off, j_off, j_idx, pi, pj, out, precision == SPHK_MIXED,
                           walk_queue(ctx)));
     t.stop();
     return SPHK_OK;
 }
 
-int sphk_gravity_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+int sphk_hydro_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                   const int32_t *j_idx, sphk_hydro_src pi, sphk_hydro_src pj, sphk_hydro_out out,
+                   int precision, void *stream)
+{
+    return sphk_hydro_dev_n(ctx, n_walk, 0, i_off, j_off, j_idx, pi, pj, out, precision, stream);
+}
+
+int sphk_gravity_dev_n(sphk_ctx *ctx, int n_walk, int64_t n_i, const int32_t *i_off, const int32_t *j_off,
                      const int32_t *j_idx, sphk_grav_src pj, const int32_t *s_off,
                      const int32_t *s_idx, sphk_grav_src ps, sphk_grav_src pi, sphk_grav_out out,
                      int precision, void *stream)
@@ -516,10 +530,18 @@ int sphk_gravity_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int3
         return set_error(SPHK_E_ARG, "gravity: null output pointer");
     hipStream_t st = pick_stream(ctx, stream);
     Timer t(ctx, 2, st);
-    SPHK_HIP(launch_gravity(st, n_walk, i_off, j_off, j_idx, pj, s_off, s_idx, ps, pi, out,
+    SPHK_HIP(launch_gravity(st, n_walk, n_i, i_off, j_off, j_idx, pj, s_off, s_idx, ps, pi, out,
                             precision == SPHK_MIXED, ctx->params.uniform_softening != 0, walk_queue(ctx)));
     t.stop();
     return SPHK_OK;
+}
+
+int sphk_gravity_dev(sphk_ctx *ctx, int n_walk, const int32_t *i_off, const int32_t *j_off,
+                     const int32_t *j_idx, sphk_grav_src pj, const int32_t *s_off,
+                     const int32_t *s_idx, sphk_grav_src ps, sphk_grav_src pi, sphk_grav_out out,
+                     int precision, void *stream)
+{
+    return sphk_gravity_dev_n(ctx, n_walk, 0, i_off, j_off, j_idx, pj, s_off, s_idx, ps, pi, out, precision, stream);
 }
 
 // ---- host dispatch / retrieve -------------------------------------------
@@ -553,7 +575,7 @@ int sphk_density_dispatch(sphk_ctx *ctx, int tag, int n_walk, const int32_t *nip
     slot.kind = kDensity;
     slot.n_walk = n_walk;
     slot.ni_tot = ni;
-    return sphk_density_dev(ctx, n_walk, (const int32_t *)(slot.din.p + items[0].off),
+    return sphk_density_dev_n(ctx, n_walk, (int64_t)ni, (const int32_t *)(slot.din.p + items[0].off),
                             (const int32_t *)(slot.din.p + items[1].off), nullptr, di, dj, dout,
                             precision, (void *)ctx->stream);
 }
@@ -592,7 +614,7 @@ int sphk_hydro_dispatch(sphk_ctx *ctx, int tag, int n_walk, const int32_t *nip, 
     slot.kind = kHydro;
     slot.n_walk = n_walk;
     slot.ni_tot = ni;
-    return sphk_hydro_dev(ctx, n_walk, (const int32_t *)(slot.din.p + items[0].off),
+    return sphk_hydro_dev_n(ctx, n_walk, (int64_t)ni, (const int32_t *)(slot.din.p + items[0].off),
                           (const int32_t *)(slot.din.p + items[1].off), nullptr, di, dj, dout,
                           precision, (void *)ctx->stream);
 }
@@ -640,7 +662,7 @@ int sphk_gravity_dispatch(sphk_ctx *ctx, int tag, int n_walk, const int32_t *nip
     slot.kind = kGravity;
     slot.n_walk = n_walk;
     slot.ni_tot = ni;
-    return sphk_gravity_dev(ctx, n_walk, (const int32_t *)(slot.din.p + items[0].off),
+    return sphk_gravity_dev_n(ctx, n_walk, (int64_t)ni, (const int32_t *)(slot.din.p + items[0].off),
                             (const int32_t *)(slot.din.p + items[1].off), nullptr, dj,
                             nsp ? (const int32_t *)(slot.din.p + items[2].off) : nullptr, nullptr,
                             ds, di, dout, precision, (void *)ctx->stream);

@@ -102,6 +102,12 @@ class Walks:
                                entries_spj=h[4] if len(h) > 3 else 0)
         return self._sizes
 
+    def n_i_or(self, outputs: torch.Tensor | None) -> int:
+        """The i-particles, if known without a read from the device, else the
+        number of outputs (0 without any): chooses the waves per walk."""
+        n = self.__dict__.get("n_i")
+        return n if n is not None else 0 if outputs is None else outputs.numel()
+
     def __getattr__(self, name):
         # sizes of device-built tables (interaction-list entries = sum over
         # walks of n_i * n_j), computed lazily: list builds need not wait
@@ -171,17 +177,17 @@ class Context:
 
     def density(self, w: Walks, pi: dict, pj: dict, out: dict, precision: int = FP64):
         si, sj = _mk2(L.DensSrc, L.DENS_SRC, pi, pj)
-        check(lib().sphk_density_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                     None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
-                                     _mk(L.DensOut, L.DENS_OUT, out), int(precision),
-                                     self._stream()), "sphk_density_dev")
+        check(lib().sphk_density_dev_n(self._h, w.n_walk, w.n_i_or((out or {}).get("dens")), w.i_off.data_ptr(),
+                                       w.j_off.data_ptr(), None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
+                                       _mk(L.DensOut, L.DENS_OUT, out), int(precision), self._stream()),
+              "sphk_density_dev")
 
     def hydro(self, w: Walks, pi: dict, pj: dict, out: dict, precision: int = FP64):
         si, sj = _mk2(L.HydroSrc, L.HYDRO_SRC, pi, pj)
-        check(lib().sphk_hydro_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                   None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
-                                   _mk(L.HydroOut, L.HYDRO_OUT, out), int(precision),
-                                   self._stream()), "sphk_hydro_dev")
+        check(lib().sphk_hydro_dev_n(self._h, w.n_walk, w.n_i_or((out or {}).get("ax")), w.i_off.data_ptr(),
+                                     w.j_off.data_ptr(), None if w.j_idx is None else w.j_idx.data_ptr(), si, sj,
+                                     _mk(L.HydroOut, L.HYDRO_OUT, out), int(precision), self._stream()),
+              "sphk_hydro_dev")
 
     def hydro_vjp(self, w: Walks, src: dict, cot: dict, grad: dict):
         """Add to grad (HYDRO_GRAD fields) the vector-Jacobian product of the
@@ -208,13 +214,13 @@ class Context:
     def gravity(self, w: Walks, pj: dict, pi: dict, out: dict, ps: dict | None = None,
                 precision: int = FP64):
         sj, si = _mk2(L.GravSrc, L.GRAV_SRC, pj, pi)
-        check(lib().sphk_gravity_dev(self._h, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
-                                     None if w.j_idx is None else w.j_idx.data_ptr(), sj,
-                                     None if w.s_off is None else w.s_off.data_ptr(),
-                                     None if w.s_idx is None else w.s_idx.data_ptr(),
-                                     _mk(L.GravSrc, L.GRAV_SRC, ps), si,
-                                     _mk(L.GravOut, L.GRAV_OUT, out), int(precision),
-                                     self._stream()), "sphk_gravity_dev")
+        check(lib().sphk_gravity_dev_n(self._h, w.n_walk, w.n_i_or((out or {}).get("ax")), w.i_off.data_ptr(),
+                                       w.j_off.data_ptr(), None if w.j_idx is None else w.j_idx.data_ptr(), sj,
+                                       None if w.s_off is None else w.s_off.data_ptr(),
+                                       None if w.s_idx is None else w.s_idx.data_ptr(),
+                                       _mk(L.GravSrc, L.GRAV_SRC, ps), si,
+                                       _mk(L.GravOut, L.GRAV_OUT, out), int(precision),
+                                       self._stream()), "sphk_gravity_dev")
 
     # --- timing (HIP events recorded around each launch on its stream) ---
     def timing(self, enable: bool = True):
