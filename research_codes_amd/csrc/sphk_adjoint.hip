@@ -399,47 +399,63 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
 // H_{k+1} = min(eta kappa (m / rho_k)^(1/3), hmax), with S_k = sum m r^2 t^3
 // (so that d rho_k / d h_k = 3 rho_k / h_k - 5 C1 h_k^4 S_k), then the grad-h
 // sums at H_3.  The reverse runs the outputs' cotangents back through
-// Omega, div v and |curl v| (per particle), through the grad-h pair sums (one
-// sweep), down the chain H_3 -> rho_2 -> H_2 -> rho_1 -> H_1 -> rho_0 -> H_0
-// (per particle), and through the three h-passes' pair sums (one sweep with
-// the three kernel weights).  Gather lists are not symmetric, so the j-side
+// Omega, div v and |curl v| (per particle), down the chain H_3 -> rho_2 -> H_2
+// -> rho_1 -> H_1 -> rho_0 -> H_0 (per particle; the derivative by h_3 comes
+// from sums of the forward sweep), and through the pair sums of grad-h and of
+// the h-passes (one sweep).  Gather lists are not symmetric, so the j-side
 // position and velocity cotangents collect in LDS per tile (atomic adds) and
 // leave with one global FP64 atomic per record and component.
+// A list holds the neighbours of a whole walk, about a fifth of it within
+// reach of any one particle: a lane first marks its records of a tile by
+// distance and runs the pair terms over the marked ones.  Bound by the latency
+// of the sweeps' loads and sums, so registers are held to 128 (4 waves per
+// SIMD; 144 as the compiler chose, 5 waves spill) and the sums across slices
+// take the tile's LDS.  2x10^5 particles: 0.99 ms with the terms of every
+// listed pair and a reverse sweep each for grad-h and the h-passes, 0.68 with
+// marks and one reverse sweep, 0.63 so.
 // ---------------------------------------------------------------------------
+// Square root of r2 >= 0 as sqrt_ieee, with 0 (self pairs) and r2 < 1e-300
+// on the same path.
+__device__ __forceinline__ double sqrt_r2(double r2)
+{
+    return sqrt_refine(r2, __builtin_amdgcn_rsq(r2 > 1e-300 ? r2 : 1e-300));
+}
+
 struct DRec {
     double x, y, z, m, vx, vy, vz;
-    int32_t id;
 };
 
-// Per-i sums over the S slices (fixed order), visible to every lane of the i.
+// Per-i sums over the S slices (fixed order), visible to every lane of the i;
+// one loop for all of them, as it is bound by the latency of its LDS reads.
 template <int N>
 __device__ __forceinline__ void slice_total(double (&v)[N], double *red, int lane, int il, int ni, int S)
 {
-#pragma unroll
-    for (int q = 0; q < N; q++) {
-        __syncthreads();
-        red[q * kWave + lane] = v[q];
-    }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < N; q++) {
-        double s = 0.;
-        for (int t = 0; t < S; t++) s += red[q * kWave + il + ni * t];
-        v[q] = s;
+    for (int q = 0; q < N; q++) red[q * kWave + lane] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < N; q++) v[q] = red[q * kWave + il];
+#pragma unroll 2
+    for (int t = 1; t < S; t++) {
+#pragma unroll
+        for (int q = 0; q < N; q++) v[q] += red[q * kWave + il + ni * t];
     }
 }
 
-__global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const int32_t *__restrict__ i_off,
+__global__ __launch_bounds__(kWave, 4) void density_vjp_kernel(int n_walk, const int32_t *__restrict__ i_off,
                                                             const int32_t *__restrict__ j_off,
                                                             const int32_t *__restrict__ j_idx, sphk_dens_src src,
                                                             double eta_ksrh, double hmax, sphk_dens_cot cot,
                                                             sphk_dens_grad grad)
 {
     constexpr double C0 = kCeff0, k5 = -5. * kCeff1;
-    __shared__ DRec sp[kTile];
+    // a tile and its cotangents; between sweeps the sums across slices
+    __shared__ __attribute__((aligned(16))) char smem[kTile * (sizeof(DRec) + 6 * sizeof(double))];
     __shared__ int32_t sj[kTile];
-    __shared__ double jb[6 * kTile];
-    __shared__ double red[6 * kWave];
+    DRec *const sp = reinterpret_cast<DRec *>(smem);
+    double *const jb = reinterpret_cast<double *>(sp + kTile), *const red = reinterpret_cast<double *>(smem);
+    static_assert(10 * kWave * sizeof(double) <= sizeof(smem), "reduction buffer");
     if ((int)blockIdx.x >= n_walk) return;
     const int w = xcd_walk_adj(blockIdx.x, n_walk);
     const int lane = threadIdx.x;
@@ -447,23 +463,39 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
     const int kb = j_off[w], ke = j_off[w + 1];
 
     // one sweep over the walk's list: f(record, k-th slot) per pair of this
-    // lane's slice; with FLUSH the j-side cotangents in jb[0..5][k] go to grad
-    auto sweep = [&](auto &&f, bool flush, int slice, int S) {
+    // lane's slice that is not beyond sqrt(R2) of (px, py, pz); with FLUSH the
+    // j-side cotangents in jb[0..5][k] go to grad
+    auto sweep = [&](auto &&f, double px, double py, double pz, double R2, bool vel, bool flush, int slice, int S) {
         for (int t0 = kb; t0 < ke; t0 += kTile) {
             const int nt = min(kTile, ke - t0);
             __syncthreads();
             if (lane < nt) {
                 const int j = j_idx ? j_idx[t0 + lane] : t0 + lane;
-                sp[lane] = DRec{src.x[j], src.y[j], src.z[j], src.m[j], src.vx[j], src.vy[j], src.vz[j], src.id[j]};
+                sp[lane].x = src.x[j];
+                sp[lane].y = src.y[j];
+                sp[lane].z = src.z[j];
+                sp[lane].m = src.m[j];
+                if (vel) {
+                    sp[lane].vx = src.vx[j];
+                    sp[lane].vy = src.vy[j];
+                    sp[lane].vz = src.vz[j];
+                }
                 sj[lane] = j;
-            } else {
-                sp[lane] = DRec{1e15, 1e15, 1e15, 0., 0., 0., 0., -1};
-                sj[lane] = -1;
             }
             if (flush)
                 for (int q = 0; q < 6; q++) jb[q * kTile + lane] = 0.;
             __syncthreads();
-            for (int k = slice; k < nt; k += S) f(sp[k], k);
+            uint64_t near = 0;
+#pragma unroll 4
+            for (int k = slice; k < nt; k += S) {
+                const double dx = px - sp[k].x, dy = py - sp[k].y, dz = pz - sp[k].z;
+                near |= (uint64_t)!(dx * dx + dy * dy + dz * dz >= R2) << k;
+            }
+            while (near) {
+                const int k = __builtin_ctzll(near);
+                near &= near - 1;
+                f(sp[k], k);
+            }
             if (flush) {
                 __syncthreads();
                 if (lane < nt) {
@@ -477,6 +509,8 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
             }
         }
     };
+    // squared radius of every pair that counts at a smoothing length H
+    auto reach = [](double H) { return fmax(H * H * (1. + 1e-12), 1e-300); };
 
     for (int c0 = ib; c0 < ie; c0 += kWave) {
         const int ni = min(kWave, ie - c0);
@@ -498,12 +532,12 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
             sweep([&](const DRec &r, int) {
                 const double dx = px - r.x, dy = py - r.y, dz = pz - r.z;
                 const double r2 = dx * dx + dy * dy + dz * dz;
-                const double q = __builtin_sqrt(r2) * h;
+                const double q = sqrt_r2(r2) * h;
                 const double t = q < 1. ? 1. - q : 0.;
                 const double t2 = t * t;
                 v[0] += r.m * (C0 * t2 * t2 * (1. + 4. * q));
                 v[1] += r.m * r2 * (t2 * t);
-            }, false, slice, S);
+            }, px, py, pz, reach(H[k]), false, false, slice, S);
             slice_total<2>(v, red, lane, il, ni, S);
             rho[k] = v[0] * (h * h * h);
             Sk[k] = v[1];
@@ -514,22 +548,35 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
         // -- forward grad-h sums at H_3
         const double h3 = 1. / H[3];
         const double h3_4 = (h3 * h3) * (h3 * h3), h3_5 = h3_4 * h3;
-        double fg[5] = {0., 0., 0., 0., 0.};   // gsum, dvsum, rot x, y, z (dw folded in)
+        // gsum, dvsum, rot x, y, z (dw folded in); then the sums of which
+        // d L / d h_3 is made: its weights are known per particle below, so
+        // that one reverse sweep serves the grad-h sums and the h-passes
+        double fg[10] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
         sweep([&](const DRec &r, int) {
             const double dx = px - r.x, dy = py - r.y, dz = pz - r.z;
             const double dvx = pvx - r.vx, dvy = pvy - r.vy, dvz = pvz - r.vz;
             const double r2 = dx * dx + dy * dy + dz * dz;
-            const double q = __builtin_sqrt(r2) * h3;
+            const double rr = sqrt_r2(r2);
+            const double q = rr * h3;
             const double t = q < 1. ? 1. - q : 0.;
-            const double t3 = t * t * t;
+            const double t2 = t * t, t3 = t2 * t;
             const double dw = k5 * r.m * h3_5 * t3;
-            fg[0] += r.m * t3 * (3. + q * (9. - 32. * q));
-            fg[1] += (dvx * dx + dvy * dy + dvz * dz) * dw;
-            fg[2] += (dvy * dz - dvz * dy) * dw;
-            fg[3] += (dvz * dx - dvx * dz) * dw;
-            fg[4] += (dvx * dy - dvy * dx) * dw;
-        }, false, slice, S);
-        slice_total<5>(fg, red, lane, il, ni, S);
+            const double P = 3. + q * (9. - 32. * q), Pp = 9. - 64. * q;
+            const double dd = dvx * dx + dvy * dy + dvz * dz;
+            const double cx = dvy * dz - dvz * dy, cy = dvz * dx - dvx * dz, cz = dvx * dy - dvy * dx;
+            fg[0] += r.m * t3 * P;
+            fg[1] += dd * dw;
+            fg[2] += cx * dw;
+            fg[3] += cy * dw;
+            fg[4] += cz * dw;
+            const double mt2 = r.m * t2, u = mt2 * (5. * t - 3. * q);
+            fg[5] += mt2 * (t * Pp - 3. * P) * rr;
+            fg[6] += dd * u;
+            fg[7] += cx * u;
+            fg[8] += cy * u;
+            fg[9] += cz * u;
+        }, px, py, pz, reach(H[3]), true, false, slice, S);
+        slice_total<10>(fg, red, lane, il, ni, S);
         const double g = -C0 * h3_4 * fg[0];
         const double dvv = -fg[1];
         const double rho2 = rho[2];
@@ -559,55 +606,7 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
         const double gsb = -C0 * h3_4 * gb;            // d L / d gsum
         double h3b = gb * (-4. * C0 * h3 * h3 * h3 * fg[0]);
 
-        // -- reverse grad-h sweep
-        double gi[6] = {0., 0., 0., 0., 0., 0.};   // x, y, z, vx, vy, vz of i
-        double hsum = 0.;
-        sweep([&](const DRec &r, int k) {
-            const double dx = px - r.x, dy = py - r.y, dz = pz - r.z;
-            const double dvx = pvx - r.vx, dvy = pvy - r.vy, dvz = pvz - r.vz;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            const double rr = __builtin_sqrt(r2);
-            const double q = rr * h3;
-            if (!live || !(q < 1.)) return;
-            const double t = 1. - q;
-            const double t2 = t * t, t3 = t2 * t;
-            const double dw = k5 * r.m * h3_5 * t3;
-            const double P = 3. + q * (9. - 32. * q), Pp = 9. - 64. * q;
-            const double cx = dvy * dz - dvz * dy, cy = dvz * dx - dvx * dz, cz = dvx * dy - dvy * dx;
-            const double Sdw = dvsb * (dvx * dx + dvy * dy + dvz * dz) + rb[0] * cx + rb[1] * cy + rb[2] * cz;
-            // explicit d and dv terms
-            double db[3] = {dw * (dvsb * dvx + (rb[1] * dvz - rb[2] * dvy)),
-                            dw * (dvsb * dvy + (rb[2] * dvx - rb[0] * dvz)),
-                            dw * (dvsb * dvz + (rb[0] * dvy - rb[1] * dvx))};
-            const double vb[3] = {dw * (dvsb * dx + (dy * rb[2] - dz * rb[1])),
-                                  dw * (dvsb * dy + (dz * rb[0] - dx * rb[2])),
-                                  dw * (dvsb * dz + (dx * rb[1] - dy * rb[0]))};
-            // d L / d q: through gsum's m t^3 P(q) and through dw (t = 1 - q)
-            const double qb = gsb * r.m * t2 * (t * Pp - 3. * P) - 3. * Sdw * k5 * r.m * h3_5 * t2;
-            hsum += Sdw * 5. * k5 * r.m * h3_4 * t3 + qb * rr;
-            const double rb_ = qb * h3;
-            if (rr > 0.) {
-                const double f = rb_ / rr;
-                db[0] += f * dx;
-                db[1] += f * dy;
-                db[2] += f * dz;
-            }
-            gi[0] += db[0];
-            gi[1] += db[1];
-            gi[2] += db[2];
-            gi[3] += vb[0];
-            gi[4] += vb[1];
-            gi[5] += vb[2];
-            atomicAdd(&jb[0 * kTile + k], -db[0]);
-            atomicAdd(&jb[1 * kTile + k], -db[1]);
-            atomicAdd(&jb[2 * kTile + k], -db[2]);
-            atomicAdd(&jb[3 * kTile + k], -vb[0]);
-            atomicAdd(&jb[4 * kTile + k], -vb[1]);
-            atomicAdd(&jb[5 * kTile + k], -vb[2]);
-        }, true, slice, S);
-        double hs[1] = {hsum};
-        slice_total<1>(hs, red, lane, il, ni, S);
-        h3b += hs[0];
+        h3b += gsb * fg[5] + k5 * h3_4 * (dvsb * fg[6] + rb[0] * fg[7] + rb[1] * fg[8] + rb[2] * fg[9]);
         H3b += h3b * (-h3 * h3);
 
         // -- reverse down the smoothing-length chain (per particle)
@@ -622,18 +621,20 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
         }
         // Hb is now d L / d H_0
 
-        // -- reverse of the three h-passes' pair sums (positions only)
+        // -- reverse of the pair sums: grad-h, and the three h-passes
+        // (positions only)
         double wk[3], hk[3];
         for (int k = 0; k < 3; k++) {
             hk[k] = 1. / H[k];
             const double h2 = hk[k] * hk[k];
             wk[k] = rhob[k] * k5 * (h2 * h2 * hk[k]);   // rho_bar h^5 (-5 C1)
         }
+        double gi[6] = {0., 0., 0., 0., 0., 0.};   // x, y, z, vx, vy, vz of i
         sweep([&](const DRec &r, int k) {
             if (!live) return;
             const double dx = px - r.x, dy = py - r.y, dz = pz - r.z;
-            const double rr = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
-            double c = 0.;
+            const double rr = sqrt_r2(dx * dx + dy * dy + dz * dz);
+            double c = 0.;   // along d
             for (int q = 0; q < 3; q++) {
                 const double qq = rr * hk[q];
                 if (qq < 1.) {
@@ -641,15 +642,44 @@ __global__ __launch_bounds__(kWave) void density_vjp_kernel(int n_walk, const in
                     c += wk[q] * (t * t * t);
                 }
             }
-            if (c == 0.) return;
             c *= r.m;
-            gi[0] += c * dx;
-            gi[1] += c * dy;
-            gi[2] += c * dz;
-            atomicAdd(&jb[0 * kTile + k], -c * dx);
-            atomicAdd(&jb[1 * kTile + k], -c * dy);
-            atomicAdd(&jb[2 * kTile + k], -c * dz);
-        }, true, slice, S);
+            double db[3] = {0., 0., 0.};
+            const double q = rr * h3;
+            if (q < 1.) {
+                const double dvx = pvx - r.vx, dvy = pvy - r.vy, dvz = pvz - r.vz;
+                const double t = 1. - q;
+                const double t2 = t * t, t3 = t2 * t;
+                const double dw = k5 * r.m * h3_5 * t3;
+                const double P = 3. + q * (9. - 32. * q), Pp = 9. - 64. * q;
+                const double cx = dvy * dz - dvz * dy, cy = dvz * dx - dvx * dz, cz = dvx * dy - dvy * dx;
+                const double Sdw = dvsb * (dvx * dx + dvy * dy + dvz * dz) + rb[0] * cx + rb[1] * cy + rb[2] * cz;
+                // explicit d and dv terms
+                db[0] = dw * (dvsb * dvx + (rb[1] * dvz - rb[2] * dvy));
+                db[1] = dw * (dvsb * dvy + (rb[2] * dvx - rb[0] * dvz));
+                db[2] = dw * (dvsb * dvz + (rb[0] * dvy - rb[1] * dvx));
+                const double vb[3] = {dw * (dvsb * dx + (dy * rb[2] - dz * rb[1])),
+                                      dw * (dvsb * dy + (dz * rb[0] - dx * rb[2])),
+                                      dw * (dvsb * dz + (dx * rb[1] - dy * rb[0]))};
+                // d L / d q: through gsum's m t^3 P(q) and through dw (t = 1 - q)
+                const double qb = gsb * r.m * t2 * (t * Pp - 3. * P) - 3. * Sdw * k5 * r.m * h3_5 * t2;
+                if (rr > 0.) c += qb * h3 * rcp_f64(rr);
+                gi[3] += vb[0];
+                gi[4] += vb[1];
+                gi[5] += vb[2];
+                atomicAdd(&jb[3 * kTile + k], -vb[0]);
+                atomicAdd(&jb[4 * kTile + k], -vb[1]);
+                atomicAdd(&jb[5 * kTile + k], -vb[2]);
+            }
+            db[0] += c * dx;
+            db[1] += c * dy;
+            db[2] += c * dz;
+            gi[0] += db[0];
+            gi[1] += db[1];
+            gi[2] += db[2];
+            atomicAdd(&jb[0 * kTile + k], -db[0]);
+            atomicAdd(&jb[1 * kTile + k], -db[1]);
+            atomicAdd(&jb[2 * kTile + k], -db[2]);
+        }, px, py, pz, live ? reach(fmax(fmax(H[0], H[1]), fmax(H[2], H[3]))) : -1., true, true, slice, S);
 
         // -- i-side totals
         slice_total<6>(gi, red, lane, il, ni, S);

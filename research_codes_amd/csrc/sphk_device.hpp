@@ -34,16 +34,20 @@ __device__ __forceinline__ double rsqrt_f64(double x)
 // two residual corrections, as an IEEE square root is formed but without its
 // scaling, which only arguments near the ends of the range need (those, zero
 // among them, take the general one): 52 against 86 cycles a wave.
-__device__ __forceinline__ double sqrt_ieee(double x)
+// sqrt_refine: that from the seed y ~ 1/sqrt(x).
+__device__ __forceinline__ double sqrt_refine(double x, double y)
 {
-    if (!(x > 1e-270 && x < 1e270)) return __builtin_sqrt(x);
-    const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
     return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ double sqrt_ieee(double x)
+{
+    if (!(x > 1e-270 && x < 1e270)) return __builtin_sqrt(x);
+    return sqrt_refine(x, __builtin_amdgcn_rsq(x));
 }
 
 // 1/x in FP64: v_rcp_f64 seed and two Newton-Raphson steps.

@@ -85,3 +85,34 @@ def test_gravity_vjp_edges(ctx, packed, nodes):
     # accumulated onto what was there
     assert float((g.cpu() - 1.0 - want).abs().max()) <= TOL * max(1.0, float(want.abs().max()))
     assert float((gn.cpu() - 1.0 - want_n).abs().max()) <= TOL * max(1.0, float(want_n.abs().max()))
+
+
+@pytest.mark.parametrize("radius", [0.02, 0.3, 2.0])   # the particle itself, a few, every record within reach
+def test_density_vjp_edges(ctx, radius):
+    """Against torch autograd of the restatement over the same lists, some
+    particles without a cotangent; 1e-10 of a field's largest gradient, as
+    the smoothing-length chain multiplies rounding by a few hundred."""
+    from research_codes_amd.device import Walks
+    from research_codes_amd.sph_adjoint import _DENS_IN, _density_t, density_dev, expand_pairs
+    from research_codes_amd.step import KSRH
+    rng = np.random.default_rng(7)
+    sizes, lengths = [1, 2, 31, 33, 63, 64, 70, 1], [64, 65, 63, 128, 129, 64, 200, 1]
+    n, eta, hmax = sum(sizes), 0.7, 4.0
+    i_off = np.concatenate([[0], np.cumsum(sizes)])
+    lists = []
+    for a, b, k in zip(i_off[:-1], i_off[1:], lengths):     # its own particles, then others
+        rest = np.setdiff1d(np.arange(n), np.arange(a, b))
+        lists.append(rng.permutation(np.concatenate([np.arange(a, b), rng.permutation(rest)[:k - (b - a)]])))
+    w = Walks(i_off, np.concatenate([[0], np.cumsum(lengths)]), np.concatenate(lists))
+    f = {k: torch.from_numpy(rng.uniform(0.0, 1.0, n)).cuda() for k in _DENS_IN}
+    f["ksr"] = radius * (1.0 + 0.1 * f["ksr"])
+    m = torch.from_numpy(rng.uniform(0.5, 1.5, n)).cuda()
+    ids = torch.arange(n, dtype=torch.int32, device="cuda")
+    dens = torch.from_numpy(rng.standard_normal((5, n)) * (rng.random(n) < 0.7)).cuda()
+    ctx.set_params(eta=eta, ksrh=KSRH, hmax=hmax)
+    got_in = {k: f[k].clone().requires_grad_(True) for k in _DENS_IN}
+    got = torch.autograd.grad(density_dev(w, ctx, hmax, m, ids, got_in), list(got_in.values()), list(dens))
+    ref_in = {k: f[k].clone().requires_grad_(True) for k in _DENS_IN}
+    ref = torch.autograd.grad(_density_t(ref_in, m, expand_pairs(w), hmax, eta, KSRH), list(ref_in.values()), list(dens))
+    for k, a, b in zip(_DENS_IN, got, ref):
+        assert float((a - b).abs().max()) <= 1e-10 * max(float(b.abs().max()), 1e-3), k
