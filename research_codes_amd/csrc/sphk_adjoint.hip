@@ -199,9 +199,10 @@ __global__ __launch_bounds__(kWave) void gravity_vjp_kernel(
 // wave and a division 59 against 4 for an FMA, so 1/r, 1/(rho_P + rho_Q) and
 // the signal-speed root come from Newton-refined v_rsq / v_rcp.  2x10^5
 // particles, 3.5x10^7 entries: 0.97 ms with two one-sided reverses per pair
-// and IEEE roots and divisions, 0.56 ms so.  205 VGPRs, 2 waves per SIMD;
-// held to 168 (3 waves) it spills and takes 2.8 ms, and tiles of 32 or 48
-// records measure 0.58 and 0.57 ms.
+// and IEEE roots and divisions, 0.55 ms so, 0.49 ms with the pairs of a tile
+// that are not beyond both supports (about a third) marked first.  205 VGPRs,
+// 2 waves per SIMD; held to 168 (3 waves) it spills and takes 2.8 ms, and
+// tiles of 32 or 48 records were 3 % slower.
 // ---------------------------------------------------------------------------
 struct HP {           // one particle's hydro inputs (hinv^5 derived)
     double x, y, z, vx, vy, vz, h, h5, p, pc, b, d, c, al, au, u, et, m;
@@ -369,9 +370,19 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
                 sp[lane] = HRecV{load_hp(src, j), load_cot(cot, j), src.id[j]};
             }
             __syncthreads();
+            // the slice's records not beyond both supports, then their pairs
+            uint64_t near = 0;
+#pragma unroll 4
             for (int k = slice; k < nt; k += S) {
-                const HRecV &Q = sp[k];
-                if (Q.id != id) hydro_pair_vjp(P, Q.p, cp, Q.c, g);
+                const HP &q = sp[k].p;
+                const double dx = P.x - q.x, dy = P.y - q.y, dz = P.z - q.z, h = fmin(P.h, q.h);
+                const bool far = (dx * dx + dy * dy + dz * dz) * (h * h) >= 1. + 1e-12;
+                near |= (uint64_t)(!far && sp[k].id != id) << k;
+            }
+            while (near) {
+                const int k = __builtin_ctzll(near);
+                near &= near - 1;
+                hydro_pair_vjp(P, sp[k].p, cp, sp[k].c, g);
             }
         }
         // per i: the S slices' partials in slice order, then one plain add
