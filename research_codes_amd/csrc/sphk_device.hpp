@@ -151,4 +151,36 @@ struct LaneMap {
     }
 };
 
+// Wave-wide inclusive prefix sum and maximum (of values >= 0), all 64 lanes
+// active: row shifts and row broadcasts in the VALU (no LDS round trips: each
+// of the six steps of a shuffle waits for one).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);   // 0 where there is no source lane
+}
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
+__device__ __forceinline__ int wave_scan_incl(int v)
+{
+    v += dpp0<kRowShr + 1, 0xf>(v);
+    v += dpp0<kRowShr + 2, 0xf>(v);
+    v += dpp0<kRowShr + 4, 0xf>(v);
+    v += dpp0<kRowShr + 8, 0xf>(v);
+    v += dpp0<kRowBcast15, 0xa>(v);
+    v += dpp0<kRowBcast31, 0xc>(v);
+    return v;
+}
+
+__device__ __forceinline__ int wave_max(int v)
+{
+    v = max(v, dpp0<kRowShr + 1, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 2, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 4, 0xf>(v));
+    v = max(v, dpp0<kRowShr + 8, 0xf>(v));
+    v = max(v, dpp0<kRowBcast15, 0xa>(v));
+    v = max(v, dpp0<kRowBcast31, 0xc>(v));
+    return __builtin_amdgcn_readlane(v, kWave - 1);
+}
+
 }  // namespace sphk

@@ -38,6 +38,7 @@
 
 #include "sphk.h"
 #include "sphk_adjoint.h"
+#include "sphk_device.hpp"
 #include "sphk_dtree.h"
 #include "sphk_internal.hpp"
 
@@ -1148,17 +1149,13 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
                     continue;
                 }
             }
-            int incl = sz;
-            for (int d = 1; d < 64; d <<= 1) {
-                const int u = __shfl_up(incl, d, 64);
-                if (lane >= d) incl += u;
-            }
+            const int incl = sphk::wave_scan_incl(sz);
             if (MODE == 2) {
                 for (int q = 0; q < sz; q++) {
                     const int64_t at = count + incl - sz + q;
                     if (at < room) room_out[at] = (int32_t)e.x + q;
                 }
-                count += __shfl(incl, 63, 64);
+                count += __builtin_amdgcn_readlane(incl, 63);
                 sp -= P;
                 continue;
             }
@@ -1167,12 +1164,12 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
             if (take > 0) {
                 if (lane < take)
                     for (int q = 0; q < sz; q++) cand[nc + incl - sz + q] = (int32_t)e.x + q;
-                nc += __shfl(incl, take - 1, 64);
+                nc += __builtin_amdgcn_readlane(incl, take - 1);
                 sp -= take;
                 if (nc >= kRoomBatch) drain(false);
             } else {   // one leaf of more particles than fit: from its range
                 drain(true);
-                const int b = __shfl((int)e.x, 0, 64), n = __shfl(sz, 0, 64);
+                const int b = __builtin_amdgcn_readlane((int)e.x, 0), n = __builtin_amdgcn_readlane(sz, 0);
                 for (int c = 0; c < n; c += kRoomBatch) test([&](int k) { return b + c + k; }, min(kRoomBatch, n - c));
                 sp -= 1;
             }

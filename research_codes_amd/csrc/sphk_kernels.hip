@@ -287,38 +287,6 @@ __device__ __forceinline__ void dens_finish(const sphk_dens_out &out, int i, con
     out.grdh[i] = omgi;
 }
 
-// Wave-wide inclusive prefix sum and maximum (of values >= 0), all 64 lanes
-// active: row shifts and row broadcasts in the VALU (no LDS round trips: each
-// of the six steps of a shuffle waits for one).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp0(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);   // 0 where there is no source lane
-}
-constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
-
-__device__ __forceinline__ int wave_scan_incl(int v)
-{
-    v += dpp0<kRowShr + 1, 0xf>(v);
-    v += dpp0<kRowShr + 2, 0xf>(v);
-    v += dpp0<kRowShr + 4, 0xf>(v);
-    v += dpp0<kRowShr + 8, 0xf>(v);
-    v += dpp0<kRowBcast15, 0xa>(v);
-    v += dpp0<kRowBcast31, 0xc>(v);
-    return v;
-}
-
-__device__ __forceinline__ int wave_max(int v)
-{
-    v = max(v, dpp0<kRowShr + 1, 0xf>(v));
-    v = max(v, dpp0<kRowShr + 2, 0xf>(v));
-    v = max(v, dpp0<kRowShr + 4, 0xf>(v));
-    v = max(v, dpp0<kRowShr + 8, 0xf>(v));
-    v = max(v, dpp0<kRowBcast15, 0xa>(v));
-    v = max(v, dpp0<kRowBcast31, 0xc>(v));
-    return __builtin_amdgcn_readlane(v, kWave - 1);
-}
-
 // New H from rho: hdr_density.hpp:296-300 (eta * kappa * (m / rho)^(1/3), capped).
 __device__ __forceinline__ double dens_next_h(double eta_ksrh, double m, double dens, double hmax)
 {
