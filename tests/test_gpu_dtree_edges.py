@@ -49,3 +49,26 @@ def test_tree_equals_host(kind, n, n_leaf, n_group):
     finally:
         ht.close()
         dt.close()
+
+
+@pytest.mark.parametrize("n", [1024, 1025, 8192, 8193])
+def test_offsets_of_one_particle_walks(n):
+    """As many walks as particles, around the sizes where the scan of their
+    counts gives a thread another walk and where it changes its kernel."""
+    rng = np.random.default_rng(n)
+    x, y, z = rng.random((3, n))
+    perm = morton_order(x, y, z)
+    x, y, z = (np.ascontiguousarray(a[perm]) for a in (x, y, z))
+    m, eps2, h = np.full(n, 1.0 / n), np.full(n, 1e-4), rng.uniform(0.01, 0.05, n)
+    d = lambda a: torch.from_numpy(a).cuda()   # noqa: E731
+    ht = HostTree(x, y, z, m, eps2, 1, 1)
+    dt = DeviceTree(*map(d, (x, y, z, m, eps2)), 1, 1)
+    try:
+        assert dt.n_walk == ht.n_walk == n
+        for name, hl, dl in (("gather", ht.gather(h), dt.gather(d(h))), ("symmetry", ht.symmetry(h), dt.symmetry(d(h))),
+                             ("long", ht.long(0.7), dt.long(0.7))):
+            for a, b in zip(hl, dl):
+                assert np.array_equal(a, b.cpu().numpy()), name
+    finally:
+        ht.close()
+        dt.close()
