@@ -54,8 +54,9 @@ class TreeGravity:
             return tuple(o * self.G for o in out[:4]) + (out[4],)
         inv = torch.empty_like(perm)
         inv[perm] = torch.arange(perm.numel(), device=perm.device)
-        out = _GravityFn.apply(x[perm], y[perm], z[perm], perm, self)
-        return tuple(o[inv] * self.G for o in out[:4]) + (out[4][inv],)
+        out = _GravityFn.apply(*(_Take.apply(c, perm, inv) for c in (x, y, z)), perm, self)
+        out = [_Take.apply(o, inv, perm) for o in out]
+        return tuple(o * self.G for o in out[:4]) + (out[4],)
 
     # forward on sorted particles; returns the outputs and what the backward
     # pass needs (the tree, its lists and monopoles)
@@ -95,6 +96,22 @@ class _Saved:
 
     def __init__(self, tree, walks, mom, ms, e2):
         self.tree, self.walks, self.mom, self.ms, self.e2 = tree, walks, mom, ms, e2
+
+
+class _Take(torch.autograd.Function):
+    """v[perm] for a permutation with inverse inv.  The reverse is g[inv];
+    that of plain indexing must allow for repeated indices and sorts them (60
+    launches and 0.6 of 4.3 ms for the gradient of 2x10^5 particles)."""
+
+    @staticmethod
+    def forward(ctx, v, perm, inv):
+        ctx.save_for_backward(perm, inv)
+        return v[perm]
+
+    @staticmethod
+    def backward(ctx, g):
+        perm, inv = ctx.saved_tensors
+        return _Take.apply(g, inv, perm), None, None
 
 
 class _GravityFn(torch.autograd.Function):
