@@ -17,12 +17,12 @@
 //   4. Groups: a node is a walk if it holds <= n_group particles (or is a
 //      leaf) and its parent holds more; walks are ordered by first particle.
 //   5. Lists, the host's element for element, each in one pass into a room
-//      per walk.  Long list: the host's depth-first traversal, 8 lanes per
-//      walk (the children of one opened node at a time, a stack of pending
-//      entries in LDS).  Short-range lists: one wave per walk, up to 8 nodes
-//      opened at a time, the reached leaves' particles tested for exact
-//      membership on the way.  A walk that overflows its room or stack sends
-//      the build through count and fill walks at scanned offsets.
+//      per walk: the host's depth-first traversal by one wave per walk, up
+//      to 8 nodes opened at a time, a stack of pending entries in LDS; for
+//      the short-range lists the reached leaves' particles are tested for
+//      exact membership on the way.  A walk that overflows its room or stack
+//      sends the build through count and fill walks (8 lanes per walk) at
+//      scanned offsets.
 #include <hip/hip_runtime.h>
 
 #include <cstring>   // rocPRIM's iterator headers use memset without including it
@@ -1001,7 +1001,7 @@ __global__ __launch_bounds__(64) void member_kernel(int ng, TreeView t, const do
 // outskirts that open nodes one after the other (VALU issue 16 %, 1.8 waves
 // per SIMD), and the long list, issue-bound, paid two emissions per 8 nodes
 // looked at.  10^6 particles, before and now: gather and symmetry with their
-// member kernels 2.0 and 1.85 ms, 0.79 and 0.80; long 1.42, 0.95.
+// member kernels 2.0 and 1.85 ms, 0.75 and 0.76; long 1.42, 0.90.
 //
 // A node of a short-range list is skipped if no particle of it can be a
 // member: its tight box must meet the box of the walk's spheres (or its own

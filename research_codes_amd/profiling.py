@@ -113,12 +113,12 @@ _KDK_STAGES = (
     ("long list (EPJ + SPJ): one walk into rooms (count + fill on overflow)", ("list_kernel<2",)),
     ("symmetry list: candidates in one walk, exact members", ("list_kernel<1", "member_kernel<1")),
     ("gather list: candidates in one walk, exact members", ("list_kernel<0", "member_kernel<0")),
-    ("list bookkeeping (walk boxes, offsets, packing the lists)", ("walk_box", "offsets_kernel", "member_copy",
-                                                                   "room_copy")),
+    ("list bookkeeping (walk boxes, offsets, packing the lists)", ("walk_box", "offsets_kernel", "list_scan",
+                                                                   "member_copy", "room_copy")),
     ("scans and sorts (rocPRIM)", ("rocprim",)),
     ("tree rebuild (keys, levels, moments, node records, groups)",
-     ("split_kernel", "moments_kernel", "obox_kernel", "pack_", "bbox_", "keys_kernel",
-      "unsorted_kernel", "root_kernel", "group_", "head_flag", "fill_kernel")),
+     ("span_kernel", "block_scan", "node_kernel", "moments_", "obox_", "bbox_", "keys_kernel", "group_",
+      "fill_kernel")),
     ("Morton reorder of the state, unchanged-input tests of the rebuilds",
      ("permute_kernel", "equal_kernel", "flag_zero_kernel")),
     ("density functor", ("density_kernel",)),
