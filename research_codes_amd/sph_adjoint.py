@@ -40,7 +40,7 @@ import torch
 
 from . import _lib as L
 from . import ic
-from .adjoint import TreeGravity
+from .adjoint import TreeGravity, _Take
 from .device import FP64, Context, Walks
 from .step import SPHSystem
 
@@ -470,7 +470,9 @@ def step_t(S: dict, m, rec: dict, sysm: SPHSystem, dt: float) -> dict:
     P["ksr"] = S["ksr"]
     perm = rec["perm"]
     if perm is not None:
-        P = {k: v[perm] for k, v in P.items()}
+        inv = torch.empty_like(perm)
+        inv[perm] = torch.arange(perm.numel(), dtype=perm.dtype, device=perm.device)
+        P = {k: _Take.apply(v, perm, inv) for k, v in P.items()}
         m = m[perm]
     f = force_t(P, m, rec, sysm)
     out = {"x": P["x"], "y": P["y"], "z": P["z"]}
