@@ -116,3 +116,39 @@ def test_density_vjp_edges(ctx, radius):
     ref = torch.autograd.grad(_density_t(ref_in, m, expand_pairs(w), hmax, eta, KSRH), list(ref_in.values()), list(dens))
     for k, a, b in zip(_DENS_IN, got, ref):
         assert float((a - b).abs().max()) <= 1e-10 * max(float(b.abs().max()), 1e-3), k
+
+
+def test_tree_gravity_reuses_handles(ctx):
+    """Calls whose trees are freed, kept (several graphs alive at once) and
+    used on another stream give the forward of a new operator bit for bit and
+    its gradient to the order of the atomic sums; at most two handles stay."""
+    from research_codes_amd.adjoint import TreeGravity
+    rng = np.random.default_rng(11)
+    n = 3000
+    m = torch.from_numpy(rng.uniform(0.5, 1.5, n)).cuda()
+    sets = [[torch.from_numpy(rng.standard_normal(n) * s).cuda().requires_grad_(True) for _ in range(3)]
+            for s in (1.0, 0.3, 2.0, 1.0)]
+    cot = [torch.from_numpy(rng.standard_normal(n)).cuda() for _ in range(4)]
+
+    def run(op, pos):
+        out = op(*pos)
+        return out, torch.autograd.grad(out, pos, cot, retain_graph=True)
+
+    want = [run(TreeGravity(ctx, m, 0.05), pos) for pos in sets]
+    op = TreeGravity(ctx, m, 0.05)
+    side = torch.cuda.Stream()
+    for again in range(3):
+        alive = []
+        for k, pos in enumerate(sets):
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side if (again + k) % 3 == 2 else torch.cuda.current_stream()):
+                got = run(op, pos)
+            torch.cuda.synchronize()
+            if k % 2:
+                alive.append(got)          # this graph keeps its tree
+            for a, b in zip(got[0], want[k][0]):
+                assert torch.equal(a, b)
+            for a, b in zip(got[1], want[k][1]):
+                assert float((a - b).abs().max()) <= TOL * float(b.abs().max())
+        del alive, got
+        assert 1 <= len(op._idle) <= 2
