@@ -38,6 +38,7 @@
 
 #include "sphk.h"
 #include "sphk_adjoint.h"
+#include "sphk_buffers.hpp"
 #include "sphk_device.hpp"
 #include "sphk_dtree.h"
 #include "sphk_internal.hpp"
@@ -55,36 +56,25 @@ constexpr int kBlock = 256;
         if (e_ != hipSuccess) return set_error(SPHK_E_DEVICE, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
-// Device array with capacity; grow() keeps the contents.
-template <typename T>
-struct DArr {
-    T *p = nullptr;
-    size_t cap = 0;
-    hipError_t reserve(size_t n, bool keep, hipStream_t st)
+struct HipAlloc {
+    using Error = hipError_t;
+    using Stream = hipStream_t;
+    static constexpr hipError_t ok = hipSuccess;
+    static hipError_t alloc(void **p, size_t bytes)
     {
-        if (n <= cap) return hipSuccess;
-        T *q = nullptr;
-        hipError_t e = hipMalloc(&q, n * sizeof(T));
-        if (e != hipSuccess) return e;
-        if (keep && p && cap) e = hipMemcpyAsync(q, p, cap * sizeof(T), hipMemcpyDeviceToDevice, st);
-        // queued work may still read the old block: wait before freeing it
-        if (e == hipSuccess && p) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) {
-            (void)hipFree(q);
-            return e;
-        }
-        if (p) (void)hipFree(p);
-        p = q;
-        cap = n;
-        return hipSuccess;
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();   // not left for the check of a later launch
+        return e;
     }
-    void release()
+    static void free(void *p) { (void)hipFree(p); }
+    static hipError_t copy(void *to, const void *from, size_t bytes, hipStream_t st)
     {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        cap = 0;
+        return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, st);
     }
+    static hipError_t wait(hipStream_t st) { return hipStreamSynchronize(st); }
 };
+template <typename T>
+using DArr = sphk::DeviceArray<T, HipAlloc>;
 
 struct DLists {
     DArr<int32_t> j_off, j_idx, s_off, s_idx;
@@ -1326,15 +1316,13 @@ constexpr int64_t kRoomLongStart = 8192;      // long-list particles per walk
 constexpr int64_t kRoomMax = 1 << 16;
 constexpr int64_t kRoomMaxEntries = 1ll << 31;  // scratch entries (8 GiB)
 
-struct sphk_dtree {
+struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     int n = 0, n_leaf = 8, n_group = 16;
     hipStream_t st = nullptr;
-    DArr<double> x, y, z, part, frame, len;
+    DArr<double> x, y, z, part, frame;
     DArr<uint64_t> key;
-    DArr<int32_t> begin, end, child, nchild, level, parent;
     std::vector<int> level_start;   // node index of the first node of each level
     int n_node = 0;
-    DArr<double> box_lo, box_hi, mm, mx, my, mz, me, sx, sy, sz, se;
     DArr<int32_t> head, group, i_off, hist;
     // Rooms of the lists by kind, kept apart so that a list stays in its rooms
     // when another is built: with one scratch it was packed first, wanted or
@@ -1345,8 +1333,6 @@ struct sphk_dtree {
     DArr<int64_t> levels;   // starts of the levels and the node count; the group count; the unsorted flag
     int n_walk = 0;
     DArr<double> wbox;
-    DArr<BoxRec> brec;
-    DArr<MacRec> mrec;
     DArr<OboxRec> orec;
     DArr<int64_t> i64a, i64b, i64c, i64d;
     DArr<int64_t> total;
@@ -1363,22 +1349,17 @@ struct sphk_dtree {
     NodeArrays nodes() { return NodeArrays{begin.p, end.p, child.p, nchild.p, level.p, parent.p, len.p}; }
     Moments moments()
     {
-        return Moments{box_lo.p, box_hi.p, mm.p, mx.p, my.p, mz.p, me.p, sx.p, sy.p, sz.p, se.p, box_lo.cap / 3};
+        return Moments{box_lo.p, box_hi.p, mm.p, mx.p, my.p, mz.p, me.p, sx.p, sy.p, sz.p, se.p, node_cap};
     }
     void release()
     {
-        for (auto *a : {&x, &y, &z, &part, &frame, &len, &box_lo, &box_hi, &mm, &mx, &my, &mz, &me, &sx, &sy,
-                        &sz, &se})
-            a->release();
+        release_nodes();
+        for (auto *a : {&x, &y, &z, &part, &frame}) a->release();
         key.release();
-        for (auto *a : {&begin, &end, &child, &nchild, &level, &parent, &head, &group, &i_off, &hist, &mscr[0],
-                        &mscr[1], &mscr[2]})
-            a->release();
+        for (auto *a : {&head, &group, &i_off, &hist, &mscr[0], &mscr[1], &mscr[2]}) a->release();
         span.release();
         levels.release();
         wbox.release();
-        brec.release();
-        mrec.release();
         orec.release();
         for (auto *a : {&i64a, &i64b, &i64c, &i64d, &total}) a->release();
         scratch.release();
@@ -1393,21 +1374,6 @@ struct sphk_dtree {
 };
 
 namespace {
-
-int reserve_nodes(sphk_dtree *t, size_t cap)
-{
-    for (auto *a : {&t->begin, &t->end, &t->child, &t->nchild, &t->level, &t->parent})
-        SPHK_TRY(a->reserve(cap, false, t->st));
-    SPHK_TRY(t->len.reserve(cap, false, t->st));
-    for (auto *a : {&t->mm, &t->mx, &t->my, &t->mz, &t->me, &t->sx, &t->sy, &t->sz, &t->se})
-        SPHK_TRY(a->reserve(cap, false, t->st));
-    // the box arrays are [3][cap]
-    SPHK_TRY(t->box_lo.reserve(3 * cap, false, t->st));
-    SPHK_TRY(t->box_hi.reserve(3 * cap, false, t->st));
-    SPHK_TRY(t->brec.reserve(cap, false, t->st));
-    SPHK_TRY(t->mrec.reserve(cap, false, t->st));
-    return SPHK_OK;
-}
 
 // exclusive scan of n int64 counts (queued on st)
 int scan64(sphk_dtree *t, const int64_t *in, int64_t *out, int n)
@@ -1770,8 +1736,8 @@ int build_tree(sphk_dtree *t, int n, const double *x, const double *y, const dou
     t->n_node = (int)nn;
     t->level_start.clear();
     for (int L = 0; L <= kLevels && (L == 0 || h[L] > h[L - 1]); L++) t->level_start.push_back((int)h[L]);
-    if (nn > t->begin.cap)
-        if (int rc = reserve_nodes(t, std::max<size_t>(nn, 2 * (size_t)n / std::max(1, n_leaf) + 16))) return fail(rc);
+    if (t->reserve_nodes(nn, 2 * (size_t)n / std::max(1, n_leaf) + 16, st) != hipSuccess)
+        return fail(set_error(SPHK_E_DEVICE, "dtree: allocation failed"));
     hipLaunchKernelGGL(fill_kernel, dim3(grid((int)nn)), dim3(kBlock), 0, st, (int)nn, t->nchild.p, 0);
     hipLaunchKernelGGL(node_kernel, dim3(nb), dim3(kSpanTile), 0, st, n, t->key.p, t->span.p, t->hist.p, t->nodes(),
                        t->frame.p);
