@@ -16,6 +16,8 @@
 namespace sphk {
 namespace {
 
+// List positions are formed unsigned, as in the forward kernels: one past the
+// end of a list may lie beyond 2^31 - 1.
 __device__ __forceinline__ int xcd_walk_adj(int b, int n_walk)
 {
     // as the forward kernels: chunks of 64 walks dealt to the 8 XCDs in turn
@@ -63,11 +65,11 @@ struct VRec {
     int32_t j;
 };
 
-__device__ __forceinline__ VRec vjp_load(const sphk_grav_src &src, const int32_t *__restrict__ idx, int k, int ke)
+__device__ __forceinline__ VRec vjp_load(const sphk_grav_src &src, const int32_t *__restrict__ idx, uint32_t k, uint32_t ke)
 {
     VRec r{1e15, 1e15, 1e15, 0., -1};   // past the end: far away and massless
     if (k < ke) {
-        r.j = idx ? idx[k] : k;
+        r.j = idx ? idx[k] : (int32_t)k;
         r.x = src.x[r.j];
         r.y = src.y[r.j];
         r.z = src.z[r.j];
@@ -81,12 +83,12 @@ __device__ __forceinline__ VRec vjp_load(const sphk_grav_src &src, const int32_t
 // pair term, m_r (T abar - pbar w^3 d + 3 ebar w^5 d) with T = w^3 I - 3 w^5
 // d d^T and d = x_i - x_r; the i-side gets its negative.
 template <bool PACKED>
-__device__ __forceinline__ void vjp_list(int lane, int n, int kb, int ke, const int32_t *__restrict__ idx,
+__device__ __forceinline__ void vjp_list(int lane, int n, uint32_t kb, uint32_t ke, const int32_t *__restrict__ idx,
                                          const sphk_grav_src &src, const VI *sI, double *sv, int32_t *sj, double e2,
                                          double (&gi)[kVjpI][3], double *outx, double *outy, double *outz)
 {
     VRec nx = vjp_load(src, idx, kb + lane, ke);
-    for (int t0 = kb; t0 < ke; t0 += kWave) {
+    for (uint32_t t0 = kb; t0 < ke; t0 += kWave) {
         const VRec r = nx;
         nx = vjp_load(src, idx, t0 + kWave + lane, ke);
         double jx = 0., jy = 0., jz = 0.;
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
     const int w = xcd_walk_adj(blockIdx.x, n_walk);
     const int lane = threadIdx.x;
     const int ib = i_off[w], ie = i_off[w + 1];
-    const int kb = j_off[w], ke = j_off[w + 1];
+    const uint32_t kb = j_off[w], ke = j_off[w + 1];
     for (int c0 = ib; c0 < ie; c0 += kWave) {
         const int ni = min(kWave, ie - c0);
         const int S = kWave / ni, il = lane % ni;
@@ -362,11 +364,11 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
         double g[kHG];
 #pragma unroll
         for (int q = 0; q < kHG; q++) g[q] = 0.;
-        for (int t0 = kb; t0 < ke; t0 += kTile) {
-            const int nt = min(kTile, ke - t0);
+        for (uint32_t t0 = kb; t0 < ke; t0 += kTile) {
+            const int nt = (int)min((uint32_t)kTile, ke - t0);
             __syncthreads();
             if (lane < nt) {
-                const int j = j_idx ? j_idx[t0 + lane] : t0 + lane;
+                const int j = j_idx ? j_idx[t0 + lane] : (int)(t0 + lane);
                 sp[lane] = HRecV{load_hp(src, j), load_cot(cot, j), src.id[j]};
             }
             __syncthreads();
@@ -471,17 +473,17 @@ __global__ __launch_bounds__(kWave, 4) void density_vjp_kernel(int n_walk, const
     const int w = xcd_walk_adj(blockIdx.x, n_walk);
     const int lane = threadIdx.x;
     const int ib = i_off[w], ie = i_off[w + 1];
-    const int kb = j_off[w], ke = j_off[w + 1];
+    const uint32_t kb = j_off[w], ke = j_off[w + 1];
 
     // one sweep over the walk's list: f(record, k-th slot) per pair of this
     // lane's slice that is not beyond sqrt(R2) of (px, py, pz); with FLUSH the
     // j-side cotangents in jb[0..5][k] go to grad
     auto sweep = [&](auto &&f, double px, double py, double pz, double R2, bool vel, bool flush, int slice, int S) {
-        for (int t0 = kb; t0 < ke; t0 += kTile) {
-            const int nt = min(kTile, ke - t0);
+        for (uint32_t t0 = kb; t0 < ke; t0 += kTile) {
+            const int nt = (int)min((uint32_t)kTile, ke - t0);
             __syncthreads();
             if (lane < nt) {
-                const int j = j_idx ? j_idx[t0 + lane] : t0 + lane;
+                const int j = j_idx ? j_idx[t0 + lane] : (int)(t0 + lane);
                 sp[lane].x = src.x[j];
                 sp[lane].y = src.y[j];
                 sp[lane].z = src.z[j];

@@ -1216,8 +1216,8 @@ __global__ __launch_bounds__(64) void member_copy_kernel(int ng, const int64_t *
     const int g = blockIdx.x;
     if (g >= ng) return;
     const int64_t s0 = soff[g];
-    const int b = j_off[g], n = j_off[g + 1] - b;
-    for (int k = threadIdx.x; k < n; k += 64) jout[b + k] = scr[s0 + k];
+    const uint32_t b = j_off[g], n = j_off[g + 1] - b;
+    for (uint32_t k = threadIdx.x; k < n; k += 64) jout[b + k] = scr[s0 + k];   // unsigned: n may be up to 2^31 - 1
 }
 
 // The lists' entries from their rooms (walk g's from g * room) to the walk

@@ -32,6 +32,10 @@ struct alignas(4 * sizeof(R)) R4 {
     R a, b, c, d;
 };
 
+// Positions in the lists: offsets run up to 2^31 - 1, and a position past a
+// list's end (the next tile's, another wave's) may lie beyond that, so the
+// kernels form them unsigned.
+
 // Inert padding record: far away (q >> 1 for any realistic H), zero mass,
 // id -1, very negative sound speed (cannot raise vsmx).
 constexpr double kFar = 1e10;
@@ -324,9 +328,9 @@ __device__ __forceinline__ void dens_stage(int e, int t0_abs, int nj_end, const 
                                            bool with_v)
 {
     using R = real_t<MIXED>;
-    const int k = t0_abs + e;
-    if (k < nj_end) {
-        const int j = j_idx ? j_idx[k] : k;
+    const uint32_t k = (uint32_t)t0_abs + (uint32_t)e;
+    if (k < (uint32_t)nj_end) {
+        const int j = j_idx ? j_idx[k] : (int)k;
         sp[e] = make_double4(pj.x[j], pj.y[j], pj.z[j], pj.m[j]);
         if (with_v) sv[e] = R4<R>{(R)pj.vx[j], (R)pj.vy[j], (R)pj.vz[j], pack_id(pj.id[j], R(0))};
     } else {
@@ -420,7 +424,7 @@ __device__ void density_streaming(int lane, int wv, const Map &M, int i, int jb,
                                   double *shs)
 {
     using R = real_t<MIXED>;
-    const int ntile = (je - jb + kTile - 1) / kTile;
+    const int ntile = (int)(((uint32_t)(je - jb) + kTile - 1) / kTile);
     const DensI I = dens_load_i(pi, i);
     const bool owner = M.lead && wv == 0;
     int *redn = reinterpret_cast<int *>(red + NW * kWave);
@@ -538,7 +542,7 @@ __global__ __launch_bounds__(kWave *NW, 3) void density_kernel(
         const int ib = i_off[w], ie = i_off[w + 1];
         const int jb = j_off[w], je = j_off[w + 1];
         const int nj = je - jb;
-        const int ntile = (nj + kTile - 1) / kTile;
+        const int ntile = (int)(((uint32_t)nj + kTile - 1) / kTile);
 
         if (nj > CAP) {
             for (int c0 = ib; c0 < ie; c0 += kWave) {
@@ -954,12 +958,12 @@ struct HRec {
 // per-record factors of the pair term are formed here in FP64: -5 C1 m_j,
 // h_j^5 = hinv_j^5 and eta_j h_j^5.
 template <typename R>
-__device__ __forceinline__ HRec<R> hydro_load(const sphk_hydro_src &pj, const int32_t *__restrict__ j_idx, int k,
-                                              int end, double cx, double cy, double cz)
+__device__ __forceinline__ HRec<R> hydro_load(const sphk_hydro_src &pj, const int32_t *__restrict__ j_idx, uint32_t k,
+                                              uint32_t end, double cx, double cy, double cz)
 {
     using PR = typename HPos<R>::rec;
     if (k < end) {
-        const int j = j_idx ? j_idx[k] : k;
+        const int j = j_idx ? j_idx[k] : (int)k;
         const double hid = pj.hinv[j];
         const double h5 = hid * (hid * hid * hid) * hid;
         return HRec<R>{PR{(R)(pj.x[j] - cx), (R)(pj.y[j] - cy), (R)(pj.z[j] - cz), (R)(-5. * kCeff1 * pj.m[j])},
@@ -1001,7 +1005,7 @@ __global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(MIXED
 
     auto walk = [&](const int w, const int lane) {
         const int ib = i_off[w], ie = i_off[w + 1];
-        const int jb = j_off[w], je = j_off[w + 1];
+        const uint32_t jb = j_off[w], je = j_off[w + 1];
 
         // mixed: positions as offsets from the walk's first particle
         const double cx = MIXED ? pi.x[ib] : 0., cy = MIXED ? pi.y[ib] : 0., cz = MIXED ? pi.z[ib] : 0.;
@@ -1037,11 +1041,11 @@ __global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(MIXED
             // each lane loads its record of the tile into registers before the
             // barrier (loading the next tile's record during the sweep measured
             // 3 % slower in mixed mode, and its registers spill in FP64)
-            for (int r0 = jb; r0 < je; r0 += NW * kTile) {
-                const int t0 = r0 + wv * kTile;
+            for (uint32_t r0 = jb; r0 < je; r0 += NW * kTile) {
+                const uint32_t t0 = r0 + wv * kTile;
                 HydroAcc<R> a{R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0), vsmx};
                 if (t0 < je) {
-                    const int nt = min(kTile, je - t0);
+                    const int nt = (int)min((uint32_t)kTile, je - t0);
                     const HRec<R> nx = hydro_load<R>(pj, j_idx, t0 + lane, je, cx, cy, cz);
                     wave_sync();
                     sp[lane] = nx.p;
@@ -1354,12 +1358,12 @@ __global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(PERSI
 #pragma unroll
             for (int q = 0; q < kOwn; q++) acc[q] = 0.;
             // the EPJ list, then the SPJ list; NW blocks at a time
-            auto list = [&](int kb, int ke, const int32_t *idx, const sphk_grav_src &src) {
-                for (int r0 = kb; r0 < ke; r0 += NW * kBlk) {
-                    const int b0 = r0 + wv * kBlk;
+            auto list = [&](uint32_t kb, uint32_t ke, const int32_t *idx, const sphk_grav_src &src) {
+                for (uint32_t r0 = kb; r0 < ke; r0 += NW * kBlk) {
+                    const uint32_t b0 = r0 + wv * kBlk;
                     GravAcc<R> a{R(0), R(0), R(0), R(0), R(0)};
                     if (b0 < ke) {
-                        const int b1 = min(ke, b0 + kBlk);
+                        const uint32_t b1 = min(ke, b0 + kBlk);
                         if constexpr (kRel)
                             a = gravity_block_rel<ETA>(M, lane, b0, b1, idx, src, cx, cy, cz, xi, yi, zi, (float)e2,
                                                        reinterpret_cast<float4 *>(mine));
