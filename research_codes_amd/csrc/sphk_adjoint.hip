@@ -67,7 +67,7 @@ struct VRec {
 
 __device__ __forceinline__ VRec vjp_load(const sphk_grav_src &src, const int32_t *__restrict__ idx, uint32_t k, uint32_t ke)
 {
-    VRec r{1e15, 1e15, 1e15, 0., -1};   // past the end: far away and massless
+    VRec r{0., 0., 0., 0., -1};   // past the end: j < 0
     if (k < ke) {
         r.j = idx ? idx[k] : (int32_t)k;
         r.x = src.x[r.j];
@@ -93,23 +93,25 @@ __device__ __forceinline__ void vjp_list(int lane, int n, uint32_t kb, uint32_t 
         nx = vjp_load(src, idx, t0 + kWave + lane, ke);
         double jx = 0., jy = 0., jz = 0.;
         asm volatile("" ::: "memory");   // read sI per tile: hoisted, it would take every register
+        if (r.j >= 0) {   // past the end a zero mass would not do: 0 times a cotangent that overflows is no 0
 #pragma unroll
-        for (int q = 0; q < kVjpI; q++) {
-            if (q < n) {
-                const VI I = sI[q];
-                const double dx = I.x - r.x, dy = I.y - r.y, dz = I.z - r.z;
-                const double w = rsqrt_f64(__builtin_fma(dz, dz, __builtin_fma(dy, dy, __builtin_fma(dx, dx, e2))));
-                const double w2 = w * w;
-                const double mw3 = r.m * (w2 * w);
-                const double dot = __builtin_fma(dx, I.ax, __builtin_fma(dy, I.ay, __builtin_fma(dz, I.az, -I.eb)));
-                const double f = mw3 * __builtin_fma(3. * w2, dot, I.pb);
-                const double cx = mw3 * I.ax - f * dx, cy = mw3 * I.ay - f * dy, cz = mw3 * I.az - f * dz;
-                jx += cx;
-                jy += cy;
-                jz += cz;
-                gi[q][0] -= cx;
-                gi[q][1] -= cy;
-                gi[q][2] -= cz;
+            for (int q = 0; q < kVjpI; q++) {
+                if (q < n) {
+                    const VI I = sI[q];
+                    const double dx = I.x - r.x, dy = I.y - r.y, dz = I.z - r.z;
+                    const double w = rsqrt_f64(__builtin_fma(dz, dz, __builtin_fma(dy, dy, __builtin_fma(dx, dx, e2))));
+                    const double w2 = w * w;
+                    const double mw3 = r.m * (w2 * w);
+                    const double dot = __builtin_fma(dx, I.ax, __builtin_fma(dy, I.ay, __builtin_fma(dz, I.az, -I.eb)));
+                    const double f = mw3 * __builtin_fma(3. * w2, dot, I.pb);
+                    const double cx = mw3 * I.ax - f * dx, cy = mw3 * I.ay - f * dy, cz = mw3 * I.az - f * dz;
+                    jx += cx;
+                    jy += cy;
+                    jz += cz;
+                    gi[q][0] -= cx;
+                    gi[q][1] -= cy;
+                    gi[q][2] -= cz;
+                }
             }
         }
         if (PACKED) {

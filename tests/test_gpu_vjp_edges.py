@@ -87,6 +87,50 @@ def test_gravity_vjp_edges(ctx, packed, nodes):
     assert float((gn.cpu() - 1.0 - want_n).abs().max()) <= TOL * max(1.0, float(want_n.abs().max()))
 
 
+@pytest.mark.parametrize("scale", [1e295, np.inf])
+@pytest.mark.parametrize("packed", [False, True])
+def test_gravity_vjp_extreme_cotangents(ctx, packed, scale):
+    """Cotangents near the end of the range, and infinite ones: the lanes
+    past the end of a list add nothing, as every listed pair alone does.
+    The gradient is linear in the cotangents, so 1e295 times the cotangents
+    gives 1e295 times it; of one pair an infinite one gives infinities."""
+    rng = np.random.default_rng(9)
+    sizes, lengths = ([1, 17, 3], [1, 65, 100]) if scale < np.inf else ([1, 1, 1], [1, 1, 1])
+    n, e2 = sum(sizes), 0.01
+    i_off, off, _ = _walks(sizes, lengths, 200, rng)
+    idx = np.concatenate([rng.permutation(200)[:k] for k in lengths]).astype(np.int32)
+    x, X = torch.from_numpy(rng.standard_normal((n, 3))), torch.from_numpy(rng.standard_normal((200, 3)))
+    M, cot = torch.from_numpy(rng.uniform(0.5, 1.5, 200)), torch.from_numpy(rng.standard_normal((n, 5)))
+    if scale < np.inf:
+        gi, _ = _gravity_ref(x, _pairs(i_off, off, idx), X, M, e2, cot)
+    else:
+        cot[:, 3] = 1.0
+        d = x - X[idx.astype(int)]
+        gi = (M[idx.astype(int)] * ((d * d).sum(1) + e2) ** -1.5)[:, None] * d
+    big = cot.clone()
+    big[:, 3] *= scale
+    if scale < np.inf:
+        big[:, [0, 1, 2, 4]] *= scale
+    dev = lambda a: a.contiguous().cuda() if isinstance(a, torch.Tensor) else torch.from_numpy(a).cuda()   # noqa: E731
+    none = np.zeros(len(sizes) + 1, np.int32)
+    keep = [dev(a) for a in (i_off, none, np.zeros(1, np.int32), off, idx, M[:n], *x.T, M, *X.T, *big.T)]
+    io, jo, ji, so, si = keep[:5]
+    src = L.GravSrc(**{k: a.data_ptr() for k, a in zip(("m", "x", "y", "z"), keep[5:9])})
+    ps = L.GravSrc(**{k: a.data_ptr() for k, a in zip(("m", "x", "y", "z"), keep[9:13])})
+    g, gn = torch.zeros(n, 3, dtype=torch.float64, device="cuda"), torch.zeros(200, 3, dtype=torch.float64, device="cuda")
+    if not packed:
+        g, gn = g.T.contiguous(), gn.T.contiguous()
+    out = (g.data_ptr(), gn.data_ptr()) if packed else tuple(r.data_ptr() for r in (*g, *gn))
+    fn = L.lib().sphk_gravity_vjp_packed_dev if packed else L.lib().sphk_gravity_vjp_dev
+    L.check(fn(ctx.handle, len(sizes), io.data_ptr(), jo.data_ptr(), ji.data_ptr(), src, so.data_ptr(), si.data_ptr(),
+               ps, src, e2, *(a.data_ptr() for a in keep[13:]), *out, torch.cuda.current_stream().cuda_stream), "vjp")
+    got = (g if packed else g.T).cpu()
+    if scale < np.inf:
+        assert float((got / scale - gi).abs().max()) <= TOL * float(gi.abs().max())
+    else:
+        assert torch.equal(got, torch.sign(gi) * np.inf)
+
+
 @pytest.mark.parametrize("radius", [0.02, 0.3, 2.0])   # the particle itself, a few, every record within reach
 def test_density_vjp_edges(ctx, radius):
     """Against torch autograd of the restatement over the same lists, some
