@@ -1,6 +1,7 @@
-// sphk_buffers.hpp -- device arrays that grow, and the node arrays of a tree
-// handle, whose sizes belong together.  The allocator is a parameter (A), so
-// that allocations that fail can be tried on the host.
+// sphk_buffers.hpp -- device arrays that grow, and two groups of them in a
+// tree handle whose sizes belong together: the node arrays and the rooms of
+// the lists.  The allocator is a parameter (A), so that allocations that fail
+// can be tried on the host.
 //
 // A: Error (a type) and ok (its value for success), Stream (a type), and
 //   static Error alloc(void **p, size_t bytes)   (a failure leaves no error behind)
@@ -87,6 +88,63 @@ struct NodeBuffers {
         brec.release();
         mrec.release();
         node_cap = 0;
+    }
+};
+
+// Scratch of the one-pass list builds: an array of rooms for each of the three
+// kinds of lists, so that a list stays in its rooms while another is built
+// (packed first, wanted or not, the three lists of 10^6 particles took 3.54 ms
+// against 3.48, for 0.2 GB less at 51463 walks), and one for the nodes of the
+// long list.  All four hold at most `most` entries together.  Where another
+// array would go beyond that, or does not fit in memory, the kinds share the
+// largest one there is, and a list that lies in it is taken out first.
+template <class A>
+struct ListRooms {
+    DeviceArray<int32_t, A> of[3], nodes;
+    int lies[3] = {-1, -1, -1};   // the array in which a kind's list lies, -1: in none
+    size_t most;
+
+    explicit ListRooms(size_t most_) : most(most_) {}
+
+    size_t held() const { return of[0].cap + of[1].cap + of[2].cap + nodes.cap; }
+
+    // The array for n entries of `kind`, whose list before is given up, and
+    // room for n_nodes; -1 if there is no memory for them.  pack(k) takes kind
+    // k's list out of its rooms; if it fails its value is in rc, and -1 comes
+    // back.
+    template <class Pack>
+    int take(int kind, size_t n, size_t n_nodes, typename A::Stream st, Pack &&pack, int &rc)
+    {
+        rc = 0;
+        lies[kind] = -1;
+        auto clear = [&](int a) {
+            for (int k = 0; k < 3 && !rc; k++)
+                if (lies[k] == a && !(rc = pack(k))) lies[k] = -1;
+            return rc == 0;
+        };
+        const size_t more = (n > of[kind].cap ? n - of[kind].cap : 0) + (n_nodes > nodes.cap ? n_nodes - nodes.cap : 0);
+        int use = kind;
+        if (held() + more > most || of[kind].reserve(n, false, st) != A::ok) {
+            use = 0;
+            for (int k = 1; k < 3; k++)
+                if (of[k].cap > of[use].cap) use = k;
+            for (int k = 0; k < 3; k++) {
+                if (k == use || !of[k].cap) continue;
+                if (!clear(k) || A::wait(st) != A::ok) return -1;
+                of[k].release();
+            }
+        }
+        if (!clear(use)) return -1;
+        if (of[use].reserve(n, false, st) != A::ok || nodes.reserve(n_nodes, false, st) != A::ok) return -1;
+        return use;
+    }
+    void release()
+    {
+        for (int k = 0; k < 3; k++) {
+            of[k].release();
+            lies[k] = -1;
+        }
+        nodes.release();
     }
 };
 

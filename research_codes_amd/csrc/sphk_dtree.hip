@@ -80,10 +80,9 @@ struct DLists {
     DArr<int32_t> j_off, j_idx, s_off, s_idx;
     int64_t n_j = 0, n_s = 0;
     bool built = false;
-    // built by one walk and not yet packed: the entries are still in the
-    // rooms of the list's scratch (walk g's from g * room_j in mscr, from
-    // g * room_s in sscr for the long list's nodes); j_off / s_off are final
-    bool in_rooms = false;
+    // of a list that was built in one walk and is not yet packed, whose
+    // entries still lie in the handle's rooms: walk g's from g * room_j there,
+    // the long list's nodes from g * room_s; j_off / s_off are final
     int64_t room_j = 0, room_s = 0;
 };
 
@@ -1314,7 +1313,8 @@ constexpr int64_t kRoomNearStart = 1024;      // short-range list entries per wa
 constexpr int64_t kRoomStart = 2048;          // SPJ nodes per walk
 constexpr int64_t kRoomLongStart = 8192;      // long-list particles per walk
 constexpr int64_t kRoomMax = 1 << 16;
-constexpr int64_t kRoomMaxEntries = 1ll << 31;  // scratch entries (8 GiB)
+constexpr int64_t kRoomMaxEntries = 1ll << 31;  // entries of one kind's rooms (8 GiB)
+constexpr size_t kRoomsHeld = 1ull << 32;       // of all rooms that a handle holds (16 GiB)
 
 struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     int n = 0, n_leaf = 8, n_group = 16;
@@ -1324,11 +1324,7 @@ struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     std::vector<int> level_start;   // node index of the first node of each level
     int n_node = 0;
     DArr<int32_t> head, group, i_off, hist;
-    // Rooms of the lists by kind, kept apart so that a list stays in its rooms
-    // when another is built: with one scratch it was packed first, wanted or
-    // not (the three lists of 10^6 particles 3.54 -> 3.48 ms, for 0.2 GB more
-    // at 51463 walks).
-    DArr<int32_t> mscr[3];
+    sphk::ListRooms<HipAlloc> rooms{kRoomsHeld};
     DArr<Span> span;
     DArr<int64_t> levels;   // starts of the levels and the node count; the group count; the unsorted flag
     int n_walk = 0;
@@ -1344,7 +1340,6 @@ struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     // overflowed them
     int64_t room[2] = {kRoomNearStart, kRoomNearStart};
     int64_t room_long[2] = {kRoomLongStart, kRoomStart};
-    DArr<int32_t> sscr;   // SPJ room of the long list
 
     NodeArrays nodes() { return NodeArrays{begin.p, end.p, child.p, nchild.p, level.p, parent.p, len.p}; }
     Moments moments()
@@ -1356,14 +1351,14 @@ struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
         release_nodes();
         for (auto *a : {&x, &y, &z, &part, &frame}) a->release();
         key.release();
-        for (auto *a : {&head, &group, &i_off, &hist, &mscr[0], &mscr[1], &mscr[2]}) a->release();
+        for (auto *a : {&head, &group, &i_off, &hist}) a->release();
+        rooms.release();
         span.release();
         levels.release();
         wbox.release();
         orec.release();
         for (auto *a : {&i64a, &i64b, &i64c, &i64d, &total}) a->release();
         scratch.release();
-        sscr.release();
         for (auto &L : lists) {
             L.j_off.release();
             L.j_idx.release();
@@ -1439,7 +1434,8 @@ int walk_offsets(sphk_dtree *t, int ng, const int64_t *a, int64_t *c, int32_t *o
 int pack_list(sphk_dtree *t, int kind, int32_t *j_idx, int32_t *s_idx)
 {
     DLists &L = t->lists[kind];
-    if (!L.built || !L.in_rooms) return SPHK_OK;
+    const int at = t->rooms.lies[kind];
+    if (!L.built || at < 0) return SPHK_OK;
     const int ng = t->n_walk;
     const bool own = j_idx == nullptr;
     if (own) {
@@ -1451,12 +1447,12 @@ int pack_list(sphk_dtree *t, int kind, int32_t *j_idx, int32_t *s_idx)
         }
     }
     hipLaunchKernelGGL(room_copy_kernel, dim3((ng + kCopyWalks - 1) / kCopyWalks), dim3(64 * kCopyWalks), 0, t->st, ng,
-                       L.room_j, L.j_off.p, t->mscr[kind].p, j_idx);
+                       L.room_j, L.j_off.p, t->rooms.of[at].p, j_idx);
     if (kind == 2 && s_idx)
         hipLaunchKernelGGL(room_copy_kernel, dim3((ng + kCopyWalks - 1) / kCopyWalks), dim3(64 * kCopyWalks), 0, t->st,
-                           ng, L.room_s, L.s_off.p, t->sscr.p, s_idx);
+                           ng, L.room_s, L.s_off.p, t->rooms.nodes.p, s_idx);
     SPHK_TRY(hipGetLastError());
-    if (own) L.in_rooms = false;
+    if (own) t->rooms.lies[kind] = -1;
     return SPHK_OK;
 }
 
@@ -1472,7 +1468,9 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
 {
     DLists &L = t->lists[MODE];
     L.built = false;
-    L.in_rooms = false;
+    t->rooms.lies[MODE] = -1;
+    auto pack = [&](int kind) { return pack_list(t, kind, nullptr, nullptr); };   // another kind's list, where rooms are shared
+    int rc_rooms = 0;
     const int ng = t->n_walk;
     // i-particles staged in LDS by the member test: a walk holds <= n_group
     // particles unless it is a leaf (<= n_leaf; more only at the deepest level)
@@ -1496,12 +1494,16 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
     if constexpr (MODE != 2) {
         // one pass into a room per walk: no count walk, one host read.  If a
         // walk overflows its room or the stack, the counted build below runs
-        // instead (and later builds get twice the room).
+        // instead (and later builds get twice the room), and so it does where
+        // the rooms do not fit in memory.
         int64_t &room = t->room[MODE];
-        if ((int64_t)ng * room <= kRoomMaxEntries) {
-            SPHK_TRY(t->mscr[MODE].reserve((size_t)ng * (size_t)room, false, t->st));
+        const int at = (int64_t)ng * room <= kRoomMaxEntries
+                           ? t->rooms.take(MODE, (size_t)ng * (size_t)room, 0, t->st, pack, rc_rooms)
+                           : -1;
+        if (rc_rooms) return rc_rooms;
+        if (at >= 0) {
             hipLaunchKernelGGL((room_list_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
-                               r, 0., t->i64b.p, t->mscr[MODE].p, room, nullptr, nullptr, 0, n_si, t->err);
+                               r, 0., t->i64b.p, t->rooms.of[at].p, room, nullptr, nullptr, 0, n_si, t->err);
             SPHK_TRY(hipGetLastError());
             if (int rc = walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr)) return rc;
             int64_t tot1[2] = {0, 0};
@@ -1513,7 +1515,7 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
                 // the members stay in their rooms until the list is read
                 L.n_j = tot1[0];
                 L.n_s = 0;
-                L.in_rooms = true;
+                t->rooms.lies[MODE] = at;
                 L.room_j = room;
                 L.room_s = 0;
                 L.built = true;
@@ -1528,11 +1530,13 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
         // build below if a walk overflows a room or the small stack (and later
         // builds get twice the room that overflowed).
         int64_t &rj = t->room_long[0], &rsp = t->room_long[1];
-        if ((int64_t)ng * rj <= kRoomMaxEntries && (int64_t)ng * rsp <= kRoomMaxEntries) {
-            SPHK_TRY(t->mscr[MODE].reserve((size_t)ng * (size_t)rj, false, t->st));
-            SPHK_TRY(t->sscr.reserve((size_t)ng * (size_t)rsp, false, t->st));
+        const int at = (int64_t)ng * rj <= kRoomMaxEntries && (int64_t)ng * rsp <= kRoomMaxEntries
+                           ? t->rooms.take(MODE, (size_t)ng * (size_t)rj, (size_t)ng * (size_t)rsp, t->st, pack, rc_rooms)
+                           : -1;
+        if (rc_rooms) return rc_rooms;
+        if (at >= 0) {
             hipLaunchKernelGGL((room_list_kernel<2>), dim3(ng), dim3(64), 0, t->st, ng, v, wb, r, inv_t2, t->i64a.p,
-                               t->mscr[MODE].p, rj, t->i64b.p, t->sscr.p, rsp, 0, t->err);
+                               t->rooms.of[at].p, rj, t->i64b.p, t->rooms.nodes.p, rsp, 0, t->err);
             SPHK_TRY(hipGetLastError());
             if (int rc = walk_offsets(t, ng, t->i64a.p, t->i64c.p, L.j_off.p, t->i64b.p, t->i64d.p, L.s_off.p))
                 return rc;
@@ -1545,7 +1549,7 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
                 // the entries stay in their rooms until the list is read
                 L.n_j = tot1[0];
                 L.n_s = tot1[1];
-                L.in_rooms = true;
+                t->rooms.lies[MODE] = at;
                 L.room_j = rj;
                 L.room_s = rsp;
                 L.built = true;
@@ -1591,15 +1595,18 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
     } else {
         // tot[0] candidates into the scratch; the members compacted in place,
         // their counts to i64b
-        SPHK_TRY(t->mscr[MODE].reserve(std::max<int64_t>(tot[0], 1), false, t->st));
+        const int at = t->rooms.take(MODE, (size_t)std::max<int64_t>(tot[0], 1), 0, t->st, pack, rc_rooms);
+        if (rc_rooms) return rc_rooms;
+        if (at < 0) return set_error(SPHK_E_DEVICE, "dtree: no memory for %lld candidates", (long long)tot[0]);
+        int32_t *const cand = t->rooms.of[at].p;
         if (big)
             hipLaunchKernelGGL((walk_list_kernel<MODE, 1, kListStack>), lg, lb, 0, t->st, ng, v, wb, r, inv_t2,
-                               nullptr, nullptr, t->i64c.p, nullptr, t->mscr[MODE].p, nullptr, t->err);
+                               nullptr, nullptr, t->i64c.p, nullptr, cand, nullptr, t->err);
         else
             hipLaunchKernelGGL((walk_list_kernel<MODE, 1, kListStackSmall>), lg, lb, 0, t->st, ng, v, wb, r,
-                               inv_t2, nullptr, nullptr, t->i64c.p, nullptr, t->mscr[MODE].p, nullptr, t->err);
+                               inv_t2, nullptr, nullptr, t->i64c.p, nullptr, cand, nullptr, t->err);
         hipLaunchKernelGGL((member_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb, r,
-                           t->i64c.p, t->i64a.p, t->mscr[MODE].p, t->i64b.p, n_si);
+                           t->i64c.p, t->i64a.p, cand, t->i64b.p, n_si);
         SPHK_TRY(hipGetLastError());
         if (int rc = walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr)) return rc;
         if (int rc = read_totals(t, tot, overflow)) return rc;
@@ -1608,7 +1615,7 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
         if (tot[0] > std::numeric_limits<int32_t>::max())
             return set_error(SPHK_E_CAPACITY, "dtree: list longer than 2^31 entries");
         SPHK_TRY(L.j_idx.reserve(std::max<int64_t>(tot[0], 1), false, t->st));
-        hipLaunchKernelGGL(member_copy_kernel, dim3(ng), dim3(64), 0, t->st, ng, t->i64c.p, L.j_off.p, t->mscr[MODE].p,
+        hipLaunchKernelGGL(member_copy_kernel, dim3(ng), dim3(64), 0, t->st, ng, t->i64c.p, L.j_off.p, cand,
                            L.j_idx.p);
         SPHK_TRY(hipGetLastError());
     }
@@ -1694,9 +1701,9 @@ int build_tree(sphk_dtree *t, int n, const double *x, const double *y, const dou
     t->st = stream;
     t->n_walk = 0;
     t->n_node = 0;
-    for (auto &L : t->lists) {
-        L.built = false;
-        L.in_rooms = false;
+    for (int k = 0; k < 3; k++) {
+        t->lists[k].built = false;
+        t->rooms.lies[k] = -1;
     }
     auto fail = [&](int rc) {
         t->n_walk = 0;
@@ -1890,7 +1897,7 @@ int sphk_dtree_list_copy(sphk_dtree *t, int kind, int32_t *j_off, int32_t *j_idx
     const size_t no = (size_t)t->n_walk + 1;
     SPHK_TRY(hipMemcpyAsync(j_off, L.j_off.p, no * sizeof(int32_t), hipMemcpyDeviceToDevice, t->st));
     if (kind == 2) SPHK_TRY(hipMemcpyAsync(s_off, L.s_off.p, no * sizeof(int32_t), hipMemcpyDeviceToDevice, t->st));
-    if (L.in_rooms) return pack_list(t, kind, j_idx, kind == 2 ? s_idx : nullptr);
+    if (t->rooms.lies[kind] >= 0) return pack_list(t, kind, j_idx, kind == 2 ? s_idx : nullptr);
     if (L.n_j > 0)
         SPHK_TRY(hipMemcpyAsync(j_idx, L.j_idx.p, (size_t)L.n_j * sizeof(int32_t), hipMemcpyDeviceToDevice, t->st));
     if (kind == 2 && L.n_s > 0)

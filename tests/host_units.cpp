@@ -94,11 +94,81 @@ int node_buffers()
     return 0;
 }
 
+// Builds of the three kinds in many orders and sizes, in memory and with a
+// bound that do not always suffice.  A list lies where it was put until its
+// array goes to another kind; then it has been packed.  What is held stays
+// within the bound.
+int list_rooms()
+{
+    unsigned seed = 1;
+    auto rnd = [&](unsigned m) { return (seed = seed * 1664525u + 1013904223u) / 65536u % m; };
+    long shared = 0, apart = 0, none = 0, failed = 0;
+    for (int round = 0; round < 4000; round++) {
+        const size_t bound = 4000;
+        FakeAlloc::reset(-1, rnd(2) ? SIZE_MAX : 4 * (size_t)(500 + rnd(6000)));
+        {
+            sphk::ListRooms<FakeAlloc> rooms(bound);
+            int packed[3] = {0, 0, 0}, refuse = rnd(4) == 0;
+            auto pack = [&](int k) {
+                if (refuse && rnd(8) == 0) return -5;
+                packed[k]++;
+                return 0;
+            };
+            for (int step = 0; step < 12; step++) {
+                const int kind = (int)rnd(3);
+                const size_t n = 1 + rnd(rnd(3) ? 600 : 2000), nn = kind == 2 ? 1 + rnd(rnd(3) ? 300 : 2000) : 0;
+                int was[3], before[3], rc = 0;
+                for (int k = 0; k < 3; k++) {
+                    was[k] = rooms.lies[k];
+                    before[k] = packed[k];
+                }
+                const int at = rooms.take(kind, n, nn, 0, pack, rc);
+                CHECK(rooms.held() <= bound);
+                CHECK(rooms.lies[kind] == -1 && packed[kind] == before[kind]);
+                for (int k = 0; k < 3; k++) {
+                    if (k == kind) continue;
+                    if (rooms.lies[k] >= 0)        // where it was, and not where the new list goes
+                        CHECK(rooms.lies[k] == was[k] && rooms.lies[k] != at && rooms.of[was[k]].cap > 0 && packed[k] == before[k]);
+                    else                           // taken out once, if it lay anywhere
+                        CHECK(packed[k] == before[k] + (was[k] >= 0));
+                }
+                if (rc) {
+                    CHECK(at == -1 && rc == -5);
+                    failed++;
+                } else if (at < 0) {
+                    CHECK(FakeAlloc::most != SIZE_MAX);
+                    none++;
+                } else {
+                    CHECK(rooms.of[at].cap >= n && FakeAlloc::live.at(rooms.of[at].p) >= 4 * n);
+                    CHECK(rooms.nodes.cap >= nn && (!nn || FakeAlloc::live.at(rooms.nodes.p) >= 4 * nn));
+                    (at == kind ? apart : shared)++;
+                    rooms.lies[kind] = at;
+                }
+            }
+            rooms.release();
+        }
+        CHECK(FakeAlloc::live.empty() && FakeAlloc::held == 0);
+    }
+    CHECK(shared > 1000 && apart > 1000 && none > 100 && failed > 100);
+    // sizes that fit: every kind keeps its own, nothing is packed or allocated again
+    FakeAlloc::reset();
+    sphk::ListRooms<FakeAlloc> rooms(4000);
+    for (int step = 0; step < 9; step++) {
+        int rc = 0;
+        const int at = rooms.take(step % 3, 1000, step % 3 == 2 ? 500 : 0, 0, [](int) { return -1; }, rc);
+        CHECK(at == step % 3 && rc == 0 && FakeAlloc::count == std::min(step + 1 + (step >= 2), 4));
+        rooms.lies[at] = at;
+    }
+    rooms.release();
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     if (argc == 2 && !std::strcmp(argv[1], "node_buffers")) return node_buffers();
+    if (argc == 2 && !std::strcmp(argv[1], "list_rooms")) return list_rooms();
     std::printf("no such check\n");
     return 2;
 }

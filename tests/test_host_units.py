@@ -16,7 +16,7 @@ def units(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["node_buffers"])
+@pytest.mark.parametrize("name", ["node_buffers", "list_rooms"])
 def test_host_unit(units, name):
     r = subprocess.run([str(units), name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
