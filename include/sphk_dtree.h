@@ -51,6 +51,13 @@ int sphk_dtree_build(int n, const double *x, const double *y, const double *z, c
  * (n_walk 0) and may only be rebuilt or freed. */
 int sphk_dtree_rebuild(sphk_dtree *t, int n, const double *x, const double *y, const double *z,
                        const double *m, const double *eps2, int n_leaf, int n_group, void *stream);
+/* The handle gives up its tree and its lists but keeps its buffers, and
+ * forgets its stream, which may be destroyed afterwards: the work queued on
+ * it so far is marked by an event, and the stream of the next rebuild waits
+ * for that.  For a handle that is kept for later.  Not while the stream is
+ * being captured (SPHK_E_STATE).  A detached handle may only be rebuilt or
+ * freed. */
+int sphk_dtree_detach(sphk_dtree *t);
 void sphk_dtree_free(sphk_dtree *t);
 
 int sphk_dtree_n_walk(const sphk_dtree *t);

@@ -32,7 +32,11 @@ class TreeGravity:
     Call with float64 CUDA position tensors (any order); returns
     (ax, ay, az, pot) times G, differentiable with respect to the positions.
     `with_eta` also returns the functor's eta sum (sum m_j w^3, no G), the
-    input of the SPH grad-h gravity term."""
+    input of the SPH grad-h gravity term.
+
+    The operator keeps the device buffers of up to two trees whose graphs are
+    gone for its next calls (0.8 GB each at 2x10^5 particles, mostly list
+    rooms); `release` gives them back."""
 
     def __init__(self, ctx: Context, m: torch.Tensor, eps: float, theta: float = 0.5, n_group: int = 32,
                  n_leaf: int = 8, precision: int = FP64, G: float = 1.0):
@@ -44,6 +48,15 @@ class TreeGravity:
         self.theta, self.n_group, self.n_leaf = theta, n_group, n_leaf
         self.precision, self.G = precision, G
         self._idle = []   # handles of freed trees, see _Saved
+
+    def release(self):
+        """Free the kept tree buffers.  Trees of graphs that are alive are not
+        touched; they may be kept again when those graphs go."""
+        while self._idle:
+            try:
+                self._idle.pop().close()
+            except IndexError:   # taken by another thread's call
+                return
 
     def __call__(self, x, y, z):
         return self.with_eta(x, y, z)[:4]
@@ -69,7 +82,6 @@ class TreeGravity:
         except IndexError:
             t = DeviceTree(x, y, z, ms, e2, self.n_leaf, self.n_group)
         else:
-            t._src = None   # built anew, whatever the last inputs were
             t.rebuild(x, y, z, ms, e2, self.n_leaf, self.n_group)
         st = _Saved(t, Walks(t.i_off, *t.long(self.theta)), t.moments(), ms, e2, self._idle)
         self.ctx.set_params(uniform_softening=True)
@@ -103,9 +115,9 @@ class _Saved:
     tree's handle goes back to the operator, which keeps two of them for its
     next calls: a handle's buffers (0.8 GB of list rooms at 2x10^5 particles)
     cost 1.1 of a gradient's 3.9 ms to allocate and free, and now and then a
-    stall of 0.1 to 4 s.
-    Work queued on a handle's buffers is ordered before their next use: a
-    rebuild on another stream waits for the stream before."""
+    stall of 0.1 to 4 s.  A kept handle is detached: it holds no copies of its
+    inputs and no stream, and the work queued on its buffers is ordered before
+    their next use by an event."""
 
     KEEP = 2
 
@@ -114,8 +126,13 @@ class _Saved:
         self._idle = idle
 
     def __del__(self):
-        if len(self._idle) < self.KEEP:
-            self._idle.append(self.tree)
+        if len(self._idle) >= self.KEEP:
+            return
+        try:
+            self.tree.detach()
+        except Exception:   # not kept: its stream is gone or captured, or Python is ending
+            return
+        self._idle.append(self.tree)
 
 
 class _Take(torch.autograd.Function):

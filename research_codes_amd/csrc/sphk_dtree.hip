@@ -1319,6 +1319,9 @@ constexpr size_t kRoomsHeld = 1ull << 32;       // of all rooms that a handle ho
 struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     int n = 0, n_leaf = 8, n_group = 16;
     hipStream_t st = nullptr;
+    // a detached handle knows no stream: its last work is marked by `left`
+    bool detached = false;
+    hipEvent_t left = nullptr;
     DArr<double> x, y, z, part, frame;
     DArr<uint64_t> key;
     std::vector<int> level_start;   // node index of the first node of each level
@@ -1341,6 +1344,16 @@ struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     int64_t room[2] = {kRoomNearStart, kRoomNearStart};
     int64_t room_long[2] = {kRoomLongStart, kRoomStart};
 
+    // holds no tree and no lists
+    void forget()
+    {
+        n_walk = 0;
+        n_node = 0;
+        for (int k = 0; k < 3; k++) {
+            lists[k].built = false;
+            rooms.lies[k] = -1;
+        }
+    }
     NodeArrays nodes() { return NodeArrays{begin.p, end.p, child.p, nchild.p, level.p, parent.p, len.p}; }
     Moments moments()
     {
@@ -1693,18 +1706,15 @@ int build_tree(sphk_dtree *t, int n, const double *x, const double *y, const dou
                const double *eps2, int n_leaf, int n_group, hipStream_t stream)
 {
     // a previous user of the buffers may still be queued on the old stream
-    if (t->st != stream && hipStreamSynchronize(t->st) != hipSuccess)
+    if (t->detached ? hipStreamWaitEvent(stream, t->left, 0) != hipSuccess
+                    : t->st != stream && hipStreamSynchronize(t->st) != hipSuccess)
         return set_error(SPHK_E_DEVICE, "dtree: stream synchronisation failed");
+    t->detached = false;
     t->n = n;
     t->n_leaf = n_leaf;
     t->n_group = n_group;
     t->st = stream;
-    t->n_walk = 0;
-    t->n_node = 0;
-    for (int k = 0; k < 3; k++) {
-        t->lists[k].built = false;
-        t->rooms.lies[k] = -1;
-    }
+    t->forget();
     auto fail = [&](int rc) {
         t->n_walk = 0;
         t->n_node = 0;
@@ -1815,10 +1825,34 @@ int sphk_dtree_rebuild(sphk_dtree *t, int n, const double *x, const double *y, c
     return build_tree(t, n, x, y, z, m, eps2, n_leaf, n_group, (hipStream_t)stream);
 }
 
+int sphk_dtree_detach(sphk_dtree *t)
+{
+    if (!t) return set_error(SPHK_E_ARG, "dtree detach: null handle");
+    if (t->detached) return SPHK_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(t->st, &cs);   // an event recorded into a graph marks nothing
+    if (e == hipSuccess && cs != hipStreamCaptureStatusNone)
+        return set_error(SPHK_E_STATE, "dtree detach: the stream is being captured");
+    if (e == hipSuccess && !t->left) e = hipEventCreateWithFlags(&t->left, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(t->left, t->st);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return set_error(SPHK_E_DEVICE, "dtree detach: %s", hipGetErrorString(e));
+    }
+    t->detached = true;
+    t->st = nullptr;
+    t->forget();
+    return SPHK_OK;
+}
+
 void sphk_dtree_free(sphk_dtree *t)
 {
     if (!t) return;
-    (void)hipStreamSynchronize(t->st);
+    if (t->detached)
+        (void)hipEventSynchronize(t->left);
+    else
+        (void)hipStreamSynchronize(t->st);
+    if (t->left) (void)hipEventDestroy(t->left);
     t->release();
     delete t;
 }
@@ -1979,6 +2013,7 @@ extern "C" int sphk_dtree_spread_dev(const sphk_dtree *t, const double *m, const
     if (!t || !m || !nx || !ny || !nz || !gx || !gy || !gz) return set_error(SPHK_E_ARG, "dtree spread: null argument");
     sphk_dtree *tt = const_cast<sphk_dtree *>(t);
     const int nn = t->n_node;
+    if (nn <= 0) return set_error(SPHK_E_STATE, "dtree spread: no tree built");
     // three per-node sums, kept in the SPJ scratch of the tree
     SPHK_TRY(tt->sx.reserve(nn, false, t->st));
     SPHK_TRY(tt->sy.reserve(nn, false, t->st));

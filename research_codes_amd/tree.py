@@ -230,6 +230,16 @@ class DeviceTree:
         self._src = tuple(None if a is None else a.clone() for a in src[:5]) + src[5:]
         return self
 
+    def detach(self):
+        """Give up the tree and the copies of its inputs but keep the device
+        buffers for a later rebuild, on any stream: the stream used so far is
+        forgotten and may go (sphk_dtree_detach)."""
+        if not self._h:
+            raise RuntimeError("tree is closed")
+        check(lib().sphk_dtree_detach(self._h), "sphk_dtree_detach")
+        self._src = None
+        self.n_walk = self.n_node = 0
+
     def close(self):
         if self._h:
             lib().sphk_dtree_free(self._h)

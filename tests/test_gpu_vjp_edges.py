@@ -162,6 +162,46 @@ def test_density_vjp_edges(ctx, radius):
         assert float((a - b).abs().max()) <= 1e-10 * max(float(b.abs().max()), 1e-3), k
 
 
+def test_tree_gravity_forgets_streams(ctx):
+    """A kept handle outlives the stream of its last call; release() gives the
+    buffers back, and calls after it work as before."""
+    import ctypes as C
+    from research_codes_amd.adjoint import TreeGravity
+    rng = np.random.default_rng(13)
+    n = 20000
+    m = torch.from_numpy(rng.uniform(0.5, 1.5, n)).cuda()
+    pos = [torch.from_numpy(rng.standard_normal(n)).cuda().requires_grad_(True) for _ in range(3)]
+    cot = [torch.from_numpy(rng.standard_normal(n)).cuda() for _ in range(4)]
+
+    def run(op):
+        out = op(*pos)
+        return [o.detach() for o in out], torch.autograd.grad(out, pos, cot)
+
+    want = run(TreeGravity(ctx, m, 0.05))
+    op = TreeGravity(ctx, m, 0.05)
+    lib, stream = L.lib(), C.c_void_p()
+    assert lib.hipStreamCreate(C.byref(stream)) == 0
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(stream.value)):
+        got = [run(op)]
+    torch.cuda.synchronize()
+    assert lib.hipStreamDestroy(stream) == 0
+    assert len(op._idle) == 1 and op._idle[0]._src is None
+    got.append(run(op))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    n_walk = 200                                   # at least; 8192 + 2048 entries of rooms each
+    op.release()
+    assert not op._idle
+    assert torch.cuda.mem_get_info()[0] - free >= n_walk * (8192 + 2048) * 4
+    got.append(run(op))
+    for out, grad in got:
+        for a, b in zip(out, want[0]):
+            assert torch.equal(a, b)
+        for a, b in zip(grad, want[1]):
+            assert float((a - b).abs().max()) <= TOL * float(b.abs().max())
+
+
 def test_tree_gravity_reuses_handles(ctx):
     """Calls whose trees are freed, kept (several graphs alive at once) and
     used on another stream give the forward of a new operator bit for bit and
