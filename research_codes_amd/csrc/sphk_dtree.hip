@@ -42,12 +42,14 @@
 #include "sphk_device.hpp"
 #include "sphk_dtree.h"
 #include "sphk_internal.hpp"
+#include "sphk_spans.hpp"
 
+using sphk::kMaxLevel;
 using sphk::set_error;
+using sphk::shared_digits;
 
 namespace {
 
-constexpr int kMaxLevel = 21;
 constexpr int kBlock = 256;
 
 #define SPHK_TRY(expr)                                                                          \
@@ -249,12 +251,13 @@ struct NodeArrays {
 // a KDK step of 2x10^5 particles 5.2 -> 4.2 ms without them).
 constexpr int kLevels = kMaxLevel + 1;
 constexpr int kSpanTile = 1024;   // particles per block of the span, node and group kernels
-constexpr int kSpanHalo = 512;    // n_leaf up to this: window ends compared once per block, in LDS
-
-__device__ __forceinline__ int shared_digits(uint64_t a, uint64_t b)
-{
-    return a == b ? kMaxLevel : (__clzll(a ^ b) - 1) / 3;
-}
+// n_leaf up to this: window ends compared once per block, in LDS; larger: by
+// bisection, as the windows' cost grows with n_leaf.  A build of 10^6
+// particles in us, windows / bisection: n_leaf 8 366 / 395, 64 438 / 465, 128
+// 576 / 577, 256 886 / 869, 512 1256 / 1202, and beyond (windows read from
+// memory) 513 1648 / 1174, 2000 5462 / 3601, 10^4 18386 / 8944, most of which
+// is the serial sums over such leaves.
+constexpr int kSpanHalo = 512;
 
 struct Span {
     int8_t lo, hi;
@@ -280,7 +283,7 @@ __global__ __launch_bounds__(kSpanTile) void span_kernel(int n, const uint64_t *
         if (n_leaf <= kSpanHalo)
             for (int q = 0; q <= n_leaf; q++) l = max(l, (int)ends[t + q]);
         else
-            for (int q = 0; q <= n_leaf; q++) l = max(l, window(i - q));
+            l = sphk::deepest_full_level(key, n, n_leaf, i);
         if (i > 0 && key[i] < key[i - 1]) atomicOr(unsorted, 1);
         lo = i == 0 ? 0 : shared_digits(key[i - 1], key[i]) + 1;
         hi = min(l + 1, kMaxLevel);

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "sphk_buffers.hpp"
+#include "sphk_spans.hpp"
 
 #define CHECK(c)                                                        \
     do {                                                                \
@@ -163,12 +164,68 @@ int list_rooms()
     return 0;
 }
 
+struct CountedKeys {
+    const std::vector<uint64_t> &k;
+    mutable long reads = 0;
+    uint64_t operator[](size_t i) const
+    {
+        reads++;
+        return k.at(i);   // throws beyond the array
+    }
+};
+
+// The deepest level whose cell holds more than n_leaf particles against its
+// definition (cells counted level by level), and the keys read for it: the
+// logarithm of n_leaf, not n_leaf.
+int leaf_levels()
+{
+    uint64_t seed = 7;
+    auto rnd = [&]() {
+        seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+        return seed >> 1;   // 63 bits
+    };
+    for (int n : {1, 2, 513, 3000, 20000})
+        for (int kind = 0; kind < 4; kind++) {
+            std::vector<uint64_t> key(n);
+            for (auto &k : key) {
+                k = rnd();
+                if (kind == 1) k >>= k % 50;                  // few at the top, many in a corner
+                if (kind == 2 && k % 3) k = 1234567;          // two thirds at one place
+                if (kind == 3) k = k % 40 * 1000003;          // cells that cannot be split
+            }
+            std::sort(key.begin(), key.end());
+            std::vector<std::vector<int>> held(sphk::kMaxLevel + 1, std::vector<int>(n));
+            for (int L = 0; L <= sphk::kMaxLevel; L++)
+                for (int b = 0; b < n;) {
+                    const int shift = 3 * (sphk::kMaxLevel - L);
+                    int e = b;
+                    while (e < n && key[e] >> shift == key[b] >> shift) e++;
+                    for (int i = b; i < e; i++) held[L][i] = e - b;
+                    b = e;
+                }
+            for (int n_leaf : {1, 2, 8, 512, 513, 600, 2999, 3000, 3001, 10000, 30000}) {
+                int log2 = 0;
+                while ((1 << log2) < n_leaf) log2++;
+                for (int i = 0; i < n; i += 1 + n / 700) {
+                    int want = -1;
+                    for (int L = 0; L <= sphk::kMaxLevel; L++)
+                        if (held[L][i] > n_leaf) want = L;
+                    CountedKeys counted{key};
+                    CHECK(sphk::deepest_full_level(counted, n, n_leaf, i) == want);
+                    CHECK(counted.reads <= 5 * (log2 + 3));
+                }
+            }
+        }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     if (argc == 2 && !std::strcmp(argv[1], "node_buffers")) return node_buffers();
     if (argc == 2 && !std::strcmp(argv[1], "list_rooms")) return list_rooms();
+    if (argc == 2 && !std::strcmp(argv[1], "leaf_levels")) return leaf_levels();
     std::printf("no such check\n");
     return 2;
 }

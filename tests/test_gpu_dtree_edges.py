@@ -72,3 +72,11 @@ def test_offsets_of_one_particle_walks(n):
     finally:
         ht.close()
         dt.close()
+
+
+@pytest.mark.parametrize("kind", ["uniform", "clumped", "line"])
+@pytest.mark.parametrize("n,n_leaf,n_group", [(5000, 513, 64), (5000, 2500, 16), (5000, 4999, 5000), (5000, 5000, 64),
+                                              (5000, 9000, 1)])
+def test_large_leaves_equal_host(kind, n, n_leaf, n_group):
+    """Leaves beyond the windows held in LDS, up to more than there are particles."""
+    test_tree_equals_host(kind, n, n_leaf, n_group)

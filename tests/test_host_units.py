@@ -1,5 +1,6 @@
-"""Parts of the library that are plain C++ (buffers that grow), checked on
-the host against an allocator that can fail (host_units.cpp)."""
+"""Parts of the library that are plain C++, checked on the host
+(host_units.cpp): buffers that grow, with an allocator that can fail, and the
+levels of a tree's leaves."""
 import subprocess
 from pathlib import Path
 
@@ -16,7 +17,7 @@ def units(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["node_buffers", "list_rooms"])
+@pytest.mark.parametrize("name", ["node_buffers", "list_rooms", "leaf_levels"])
 def test_host_unit(units, name):
     r = subprocess.run([str(units), name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
