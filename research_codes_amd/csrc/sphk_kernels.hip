@@ -1006,6 +1006,7 @@ __global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(MIXED
     auto walk = [&](const int w, const int lane) {
         const int ib = i_off[w], ie = i_off[w + 1];
         const uint32_t jb = j_off[w], je = j_off[w + 1];
+        if (ib >= ie) return;   // a walk of no particles has no first one (ib may be past the last particle)
 
         // mixed: positions as offsets from the walk's first particle
         const double cx = MIXED ? pi.x[ib] : 0., cy = MIXED ? pi.y[ib] : 0., cz = MIXED ? pi.z[ib] : 0.;
