@@ -162,6 +162,64 @@ def test_density_vjp_edges(ctx, radius):
         assert float((a - b).abs().max()) <= 1e-10 * max(float(b.abs().max()), 1e-3), k
 
 
+@pytest.mark.parametrize("far", [0.5, 30.0])    # supports that end within the cluster, or not
+def test_hydro_vjp_edges(ctx, far):
+    """Against torch autograd of the restatement over the same lists:
+    clusters apart from each other (their lists hold every interacting pair in
+    both orders), walks of 1 to 70 particles, lists of 0 to 129 records (the
+    cluster and particles of other clusters, beyond every support), supports of
+    a factor of ten, so that many pairs lie within one only, and pressures and
+    energies that are equal for half of the pairs.  1e-10 of a field's largest
+    gradient, as 1/r and 1/sqrt(|dP|) multiply rounding by some hundreds."""
+    from research_codes_amd.device import Walks
+    from research_codes_amd.sph_adjoint import _hydro_t, expand_pairs, hydro_dev
+    rng = np.random.default_rng(17)
+    # walks (particles, records) by cluster
+    clusters = [[(1, 0)], [(1, 1)], [(33, 63)], [(64, 64)], [(64, 65)], [(70, 129)], [(5, 64), (28, 33)], [(2, 128), (1, 3)]]
+    n = sum(k for c in clusters for k, _ in c)
+    sizes, lists, pos, first = [], [], [], 0
+    for q, c in enumerate(clusters):
+        own = np.arange(first, first + sum(k for k, _ in c))
+        others = np.setdiff1d(np.arange(n), own)
+        for k, length in c:
+            sizes.append(k)
+            lists.append(rng.permutation(np.concatenate([own, rng.permutation(others)[:length - len(own)]]))
+                         if length else own[:0])
+        pos.append(rng.uniform(0.0, 1.0, (len(own), 3)) + [100.0 * q, 0.0, 0.0])
+        first += len(own)
+    w = Walks(np.concatenate([[0], np.cumsum(sizes)]), np.concatenate([[0], np.cumsum([len(v) for v in lists])]),
+              np.concatenate(lists))
+    f = {k: torch.from_numpy(rng.uniform(0.5, 1.5, n)).cuda() for k in L.HYDRO_GRAD}
+    f.update({k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in zip("xyz", np.concatenate(pos).T)})
+    f["hinv"] = torch.from_numpy(1.0 / (far * 10.0 ** rng.uniform(-1.0, 0.0, n))).cuda()
+    for k in ("pres", "thrm"):
+        f[k][::2] = 1.0
+    for k in ("vx", "vy", "vz"):
+        f[k] = f[k] - 1.0
+    m = torch.from_numpy(rng.uniform(0.5, 1.5, n)).cuda()
+    ids = torch.arange(n, dtype=torch.int32, device="cuda")
+    dev_in = {k: f[k].clone().requires_grad_(True) for k in L.HYDRO_GRAD}
+    dev = hydro_dev(w, ctx, m, ids, dev_in)
+    cot = {k: torch.from_numpy(rng.standard_normal(n)).cuda() for k in dev}
+    got = torch.autograd.grad(list(dev.values()), list(dev_in.values()), [cot[k] for k in dev])
+    ref_in = {k: f[k].clone().requires_grad_(True) for k in L.HYDRO_GRAD}
+    i, j = expand_pairs(w)
+    H = 1.0 / f["hinv"]
+    r2 = sum((f[c][i] - f[c][j]) ** 2 for c in "xyz")
+    keep = (i != j) & (r2 < torch.maximum(H[i], H[j]) ** 2)
+    d = {k: ref_in[k] for k in ("hinv", "presc", "thrm", "vsnd", "dens", "pres", "eta")}
+    h = _hydro_t({k: ref_in[k] for k in ("x", "y", "z", "vx", "vy", "vz", "alph", "alphu")}, m, (i[keep], j[keep]),
+                 dict(d, bswt_half=ref_in["bswt"]), 1.0)
+    ref = {"ax": h["achx"], "ay": h["achy"], "az": h["achz"], "udot": h["udot"], "diffu": h["diffu"],
+           "gx": h["g1x"], "gy": h["g1y"], "gz": h["g1z"]}
+    want = torch.autograd.grad([ref[k] for k in dev], list(ref_in.values()), [cot[k] for k in dev])
+    for k, a, b in zip(L.HYDRO_GRAD, got, want):
+        assert float((a - b).abs().max()) <= 1e-10 * float(b.abs().max()), k
+    one = torch.tensor([s == 1 and len(v) < 2 for s, v in zip(sizes, lists) for _ in range(s)])
+    for a in got:                                   # no neighbours, no gradient
+        assert not a[one.cuda()].any()
+
+
 def test_tree_gravity_forgets_streams(ctx):
     """A kept handle outlives the stream of its last call; release() gives the
     buffers back, and calls after it work as before."""
