@@ -53,7 +53,10 @@ __device__ __forceinline__ int xcd_walk_range(int b, int n_walk)
 // 1.39 ms, one range each 1.19).  More chunks of i-particles mean more
 // atomics: kVjpI = 8 / 12 / 16 take 2.4 / 1.9 / 1.6 ms unpacked, and 16 is
 // what leaves 3 waves per SIMD (160 VGPRs).  Before, every pair was evaluated
-// twice (a sweep per side, 64-record LDS tiles): 1.7 ms.
+// twice (a sweep per side, 64-record LDS tiles): 1.7 ms.  A walk of more than
+// kVjpI particles sends its records' sums once per chunk and still gains: walk
+// groups of 64 and 128 (17 and 35 particles a walk) 1.67 -> 1.48 and 2.89 ->
+// 1.73 ms packed, 1.64 and 1.75 unpacked.
 constexpr int kVjpI = 16;
 
 struct alignas(16) VI {
@@ -202,9 +205,11 @@ __global__ __launch_bounds__(kWave) void gravity_vjp_kernel(
 // pair.  Bound by FP64 issue: an IEEE FP64 square root measures 86 cycles per
 // wave and a division 59 against 4 for an FMA, so 1/r, 1/(rho_P + rho_Q) and
 // the signal-speed root come from Newton-refined v_rsq / v_rcp.  2x10^5
-// particles, 3.5x10^7 entries: 0.97 ms with two one-sided reverses per pair
-// and IEEE roots and divisions, 0.55 ms so, 0.49 ms with the pairs of a tile
-// that are not beyond both supports (about a third) marked first.  205 VGPRs,
+// particles, 3.5x10^7 entries: 0.98 ms with two one-sided reverses per pair
+// and IEEE roots and divisions, 0.53 ms so, 0.46 ms with the pairs of a tile
+// that are not beyond both supports (about a third) marked first.  Against
+// 80-bit values of the same sums each field's error is 1.96e-16 to 4.6e-16 of
+// its norm (with IEEE roots and divisions 1.98e-16 to 5.1e-16).  205 VGPRs,
 // 2 waves per SIMD; held to 168 (3 waves) it spills and takes 2.8 ms, and
 // tiles of 32 or 48 records were 3 % slower.
 // ---------------------------------------------------------------------------
@@ -427,7 +432,7 @@ __global__ __launch_bounds__(kWave) void hydro_vjp_kernel(int n_walk, const int3
 // SIMD; 144 as the compiler chose, 5 waves spill) and the sums across slices
 // take the tile's LDS.  2x10^5 particles: 0.99 ms with the terms of every
 // listed pair and a reverse sweep each for grad-h and the h-passes, 0.68 with
-// marks and one reverse sweep, 0.63 so.
+// marks and one reverse sweep, 0.62 so.
 // ---------------------------------------------------------------------------
 // Square root of r2 >= 0 as sqrt_ieee, with 0 (self pairs) and r2 < 1e-300
 // on the same path.
