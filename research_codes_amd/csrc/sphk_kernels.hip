@@ -1317,8 +1317,12 @@ __device__ __forceinline__ GravAcc<float> gravity_block_rel(const Map &M, int la
 
 // ETA false: the caller does not need the softening-gradient sum (out.eta
 // NULL, e.g. under a constant softening, where it does not enter).
+// Persistent mixed launches: at least 8 waves per SIMD, but 5 with uniform
+// softening, whose four staged records would spill 29 registers at 8 (10^5
+// particles: 208 us, 323 with the spills, 297 before the records were staged
+// together).
 template <bool MIXED, bool UNIFORM, bool ETA, bool PERSIST, int NW>
-__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(PERSIST && MIXED ? 8 : 1))) void gravity_kernel(
+__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(PERSIST && MIXED ? (UNIFORM ? 5 : 8) : 1))) void gravity_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_grav_src pj, const int32_t *__restrict__ s_off,
     const int32_t *__restrict__ s_idx, sphk_grav_src ps, sphk_grav_src pi, sphk_grav_out out, int *queue)
