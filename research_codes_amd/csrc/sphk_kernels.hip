@@ -509,13 +509,27 @@ __device__ void density_streaming(int lane, int wv, const Map &M, int i, int jb,
     if (owner) dens_finish(out, i, acc, dens, np, hs, I.rs);
 }
 
-// Launch bound: 3 waves per SIMD (at most 168 VGPRs; a few spill).  Between its
-// sweeps the kernel is bound by latency, so scans go through DPP, lane sums
-// run in one loop for all quantities, and distances take sqrt_ieee: 10^6
-// particles, one wave per walk, 1.38 -> 1.30 ms mixed and 1.67 -> 1.44 FP64
-// (there also 20 instead of 22 KB of LDS: 8 walks per CU).
-template <bool MIXED, int CAP, bool PERSIST, int NW>
-__global__ __launch_bounds__(kWave *NW, 3) void density_kernel(
+// Launch bound: OCC waves per SIMD, 3 for launches that fill the chip (at most
+// 168 VGPRs; a few spill).  Between its sweeps the kernel is bound by latency,
+// so scans go through DPP, lane sums run in one loop for all quantities, and
+// distances take sqrt_ieee: 10^6 particles, one wave per walk, 1.38 -> 1.30 ms
+// mixed and 1.67 -> 1.44 FP64 (there also 20 instead of 22 KB of LDS: 8 walks
+// per CU).
+// Mixed launches of few walks with a wave each wait for their longest walks,
+// in which each spilled register is reloaded, and have no use for a third
+// wave: OCC 2 (197 VGPRs, none spills).  Persistent mixed launches, whose loop
+// over walks costs registers, take it always.  In us with 3 / 2, capacity 256
+// (192), walks (particles on average): 572 (17) 213 / 198 (212 / 198), 1797
+// (2.8) 53 / 46 (52 / 46), 3980 (5.0) 71 / 65 (70 / 66), 5385 (19) 998 / 921
+// (987 / 935), 7358 (2.7) 83 / 76 (77 / 77), 10952 (9.1) 277 / 260 (274 / 264),
+// 14449 (2.8) 106 / 110 (99 / 112), 42605 (9.4) 567 / 571 (546 / 614).  Where the
+// mean is known, 8000 walks of more particles have two waves each; where it is
+// not, walks may be long, and the line lies further out.  FP64 at capacity
+// 256 is held to 2 waves by its LDS.
+constexpr int kDensFew = 8192, kDensFewUnknown = 12288;
+
+template <bool MIXED, int CAP, bool PERSIST, int NW, int OCC>
+__global__ __launch_bounds__(kWave *NW, OCC) void density_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_dens_src pi, sphk_dens_src pj, sphk_dens_out out,
     double eta_ksrh, double hmax, int *queue)
@@ -1465,17 +1479,20 @@ hipError_t launch_density(hipStream_t st, int n_walk, int64_t n_i, const int32_t
                           int *queue)
 {
     if (n_walk <= 0) return hipSuccess;
-#define SPHK_LAUNCH_D(M, CAPV, W)                                                                              \
-    SPHK_LAUNCH((density_kernel<M, CAPV, false, W>), (density_kernel<M, CAPV, true, 1>), W, n_walk, i_off, j_off, \
-                j_idx, pi, pj, out, eta_ksrh, hmax)
-#define SPHK_DENS(M, CAPV)                        \
-    do {                                          \
-        if (waves == 2)                           \
-            SPHK_LAUNCH_D(M, CAPV, 2);            \
-        else                                      \
-            SPHK_LAUNCH_D(M, CAPV, 1);            \
+#define SPHK_LAUNCH_D(M, CAPV, W, OCC)                                                                    \
+    SPHK_LAUNCH((density_kernel<M, CAPV, false, W, OCC>), (density_kernel<M, CAPV, true, 1, M ? 2 : 3>), W, \
+                n_walk, i_off, j_off, j_idx, pi, pj, out, eta_ksrh, hmax)
+#define SPHK_DENS(M, CAPV)                             \
+    do {                                               \
+        if (waves == 2)                                \
+            SPHK_LAUNCH_D(M, CAPV, 2, 3);              \
+        else if (M && few)                             \
+            SPHK_LAUNCH_D(M, CAPV, 1, M ? 2 : 3);      \
+        else                                           \
+            SPHK_LAUNCH_D(M, CAPV, 1, 3);              \
     } while (0)
     const int waves = waves_per_walk(n_walk, n_i, kDensRule);
+    const bool few = n_walk <= (n_i > 0 ? kDensFew : kDensFewUnknown);
     if (list_cap == 192) {
         if (mixed)
             SPHK_DENS(true, 192);

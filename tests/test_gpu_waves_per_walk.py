@@ -98,3 +98,36 @@ def test_results_do_not_depend_on_waves(precision, shift, functor):
         for k, v in o.items():
             assert torch.equal(v, out[0][k]), k
     assert float(sum(v.abs().sum() for v in out[0].values())) > 0.0
+
+
+@pytest.mark.parametrize("list_cap", [192, 256])
+@pytest.mark.parametrize("known,n_walk", [(True, 8192), (True, 8193), (False, 12288), (False, 12289)])
+def test_density_does_not_depend_on_occupancy(list_cap, known, n_walk):
+    """Around the numbers of walks up to which a mixed launch of one wave per
+    walk takes more registers (the mean number of particles known, or not)."""
+    rng = np.random.default_rng(31)
+    lengths = [1, 64, 65, 130, 192, 193, 256, 257]
+    n, n_all = sum(SIZES), sum(SIZES) + n_walk
+    f = {k: torch.from_numpy(rng.uniform(0.0, 1.0, n_all)).cuda() for k in L.DENS_SRC}
+    f["id"] = torch.arange(n_all, dtype=torch.int32, device="cuda")
+    f["ksr"] = f["ksr"] * 0.0 + 0.45
+    f["rs"] = 1.1 * f["ksr"]
+    i_off, j_off, j_idx = _table(rng, n, lengths)
+    out = []
+    with Context(0, eta=0.3, hmax=10.0) as ctx:
+        ctx.set_params(list_cap=list_cap)
+        for tables in ((i_off, j_off), _padded(i_off, j_off, n_walk, 1)):
+            w = Walks(*tables, j_idx)
+            o = {k: torch.zeros(n_all, dtype=torch.float64, device="cuda") for k in ("dens", "divv", "rotv", "grdh", "ksr")}
+            o["np"] = torch.zeros(n_all, dtype=torch.int64, device="cuda")
+            o["itr"] = torch.zeros(n_all, dtype=torch.uint8, device="cuda")
+            if known:
+                ctx.density(w, f, f, o, MIXED)
+            else:
+                s, d = (c(**{k: v.data_ptr() for k, v in t.items()}) for c, t in ((L.DensSrc, f), (L.DensOut, o)))
+                L.check(L.lib().sphk_density_dev(ctx.handle, w.n_walk, w.i_off.data_ptr(), w.j_off.data_ptr(),
+                                                 w.j_idx.data_ptr(), s, s, d, MIXED, torch.cuda.current_stream().cuda_stream), "density")
+            out.append({k: v[:n].cpu() for k, v in o.items()})
+    for k, v in out[0].items():     # bit for bit (NaN where a walk's list holds none of its neighbours)
+        bits = (lambda a: a.view(torch.int64)) if v.dtype == torch.float64 else (lambda a: a)
+        assert torch.equal(bits(v), bits(out[1][k])), k
