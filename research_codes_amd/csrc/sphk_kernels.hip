@@ -991,9 +991,17 @@ __device__ __forceinline__ HRec<R> hydro_load(const sphk_hydro_src &pj, const in
 }
 
 // FP64: at most 168 VGPRs (3 waves per SIMD, a few spills): 11 % faster than
-// 2 waves without spills.  Mixed needs 115 VGPRs (4 waves) as written.
-template <bool MIXED, bool PERSIST, int NW>
-__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(MIXED ? (PERSIST ? 4 : 1) : 3))) void hydro_kernel(
+// 2 waves without spills at 10^6 particles.  But launches of few walks with a
+// wave each wait for the longest of them and have no use for a third wave
+// (OCC 2, none spills): in us with 3 / 2, walks (particles on average): 572
+// (17) 124 / 98, 2079 (4.8) 38 / 34, 2592 (9.6) 107 / 88, 3085 (4.9) 59 / 49,
+// 3518 (2.8) 33 / 34, 5368 (2.8) 42 / 46, 5385 (19) 298 / 237, 9189 (2.7) 60 /
+// 68: the line lies where short walks lose.  Mixed needs 115 VGPRs (4 waves)
+// as written.
+constexpr int kHydroFew = 3072;
+
+template <bool MIXED, bool PERSIST, int NW, int OCC = MIXED ? (PERSIST ? 4 : 1) : 3>
+__global__ __launch_bounds__(kWave *NW) __attribute__((amdgpu_waves_per_eu(OCC))) void hydro_kernel(
     int n_walk, const int32_t *__restrict__ i_off, const int32_t *__restrict__ j_off,
     const int32_t *__restrict__ j_idx, sphk_hydro_src pi, sphk_hydro_src pj, sphk_hydro_out out, int *queue)
 {
@@ -1526,7 +1534,12 @@ hipError_t launch_hydro(hipStream_t st, int n_walk, int64_t n_i, const int32_t *
         switch (waves) {
         case 4: SPHK_LAUNCH_H(false, 4); break;
         case 2: SPHK_LAUNCH_H(false, 2); break;
-        default: SPHK_LAUNCH_H(false, 1); break;
+        default:
+            if (n_walk <= kHydroFew)
+                SPHK_LAUNCH((hydro_kernel<false, false, 1, 2>), (hydro_kernel<false, true, 1>), 1, n_walk, i_off, j_off,
+                            j_idx, pi, pj, out);
+            else
+                SPHK_LAUNCH_H(false, 1);
         }
     }
 #undef SPHK_LAUNCH_H

@@ -131,3 +131,22 @@ def test_density_does_not_depend_on_occupancy(list_cap, known, n_walk):
     for k, v in out[0].items():     # bit for bit (NaN where a walk's list holds none of its neighbours)
         bits = (lambda a: a.view(torch.int64)) if v.dtype == torch.float64 else (lambda a: a)
         assert torch.equal(bits(v), bits(out[1][k])), k
+
+
+@pytest.mark.parametrize("n_walk", [3072, 3073])
+def test_hydro_does_not_depend_on_occupancy(n_walk):
+    """Around the number of walks up to which an FP64 launch of one wave per
+    walk takes more registers, against the several waves of a small table."""
+    rng = np.random.default_rng(37)
+    n, n_all = sum(SIZES), sum(SIZES) + n_walk
+    f = {k: torch.from_numpy(rng.uniform(0.1, 1.0, n_all)).cuda() for k in L.HYDRO_SRC}
+    f["id"] = torch.arange(n_all, dtype=torch.int32, device="cuda")
+    i_off, j_off, j_idx = _table(rng, n, LENGTHS[:len(SIZES)])
+    out = []
+    with Context(0) as ctx:
+        for tables in ((i_off, j_off), _padded(i_off, j_off, n_walk, 1)):
+            o = {k: torch.zeros(n_all, dtype=torch.float64, device="cuda") for k in L.HYDRO_OUT}
+            ctx.hydro(Walks(*tables, j_idx), f, f, o, FP64)
+            out.append({k: v[:n].cpu().view(torch.int64) for k, v in o.items()})
+    for k in out[0]:
+        assert torch.equal(out[0][k], out[1][k]), k
