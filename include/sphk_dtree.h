@@ -69,9 +69,10 @@ const int32_t *sphk_dtree_i_off(const sphk_dtree *t);
  * Each build walks the tree once into a fixed room of entries per walk in
  * the handle's scratch (1024 members per walk for kinds 0 and 1; 8192
  * particles and 2048 nodes for kind 2) and packs the result when it is read;
- * if a walk overflows its room (or the walk's small stack), the build runs
- * again as a count walk, a scan and a fill walk, and the handle doubles that
- * room for later builds.  The scratch (n_walk x room entries; one for each
+ * if a walk overflows its room, the build runs again as a count walk, a scan
+ * and a fill walk, and the handle doubles that room for later builds.  (A walk
+ * that overflows its stack is done again with a larger one; one more host
+ * read in the first such build.)  The scratch (n_walk x room entries; one for each
  * kind and one for the nodes of kind 2) is kept with the handle's other
  * buffers.  It takes at most 16 GiB in all and 8 GiB for any one of them: the
  * kinds share one where four would take more or do not fit in memory, and

@@ -20,9 +20,9 @@
 //      per walk: the host's depth-first traversal by one wave per walk, up
 //      to 8 nodes opened at a time, a stack of pending entries in LDS; for
 //      the short-range lists the reached leaves' particles are tested for
-//      exact membership on the way.  A walk that overflows its room or stack
-//      sends the build through count and fill walks (8 lanes per walk) at
-//      scanned offsets.
+//      exact membership on the way.  A walk that overflows the stack is done
+//      again with a larger one; one that overflows its room sends the build
+//      through count and fill walks (8 lanes per walk) at scanned offsets.
 #include <hip/hip_runtime.h>
 
 #include <cstring>   // rocPRIM's iterator headers use memset without including it
@@ -34,6 +34,7 @@
 #include <limits>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "sphk.h"
@@ -801,8 +802,8 @@ __device__ __forceinline__ bool member(const TreeView &t, const double *__restri
 // The particles of the leaves reached into jout (MODE 0 gather, 1 symmetry:
 // the candidates of the short-range lists), and for MODE 2 (long) the SPJ
 // nodes into sout.  FILL 0: the walk's counts go to cj/cs.  FILL 1: written
-// from the walk's offsets oj/os.  Runs only when the stack or a room of
-// room_list_kernel overflowed.
+// from the walk's offsets oj/os.  Runs only when a room of room_list_kernel
+// overflowed or does not fit in memory.
 // Bit 1 of err is set if a stack of STACK entries would overflow.
 template <int MODE, int FILL, int STACK>
 __global__ __launch_bounds__(64) void walk_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
@@ -1002,12 +1003,28 @@ __global__ __launch_bounds__(64) void member_kernel(int ng, TreeView t, const do
 // symmetry, the node's.  The distance test (half the candidates: a sphere's
 // share of its cube) leaves out only particles that the member test refuses,
 // with 1e-9 to spare for rounding, so the lists do not change.
-constexpr int kRoomStack = 384;    // entries; a walk that needs more sets bit 1 of err
+//
+// A walk that opens several nodes at once may have many entries pending (a
+// walk at the edge of a steep profile whose search box holds the centre).
+// One that would have more than kRoomStack gives up (count -1, bit 8 of err)
+// and is done again, alone, by the DEEP kernel with its larger stack.  That
+// holds every walk: where a step would leave more than kDeepLoose entries it
+// goes depth first until they are fewer again (every finished entry on top is
+// taken, then one node opened, which leaves at most 7 entries per level beside
+// those before).  Such walks sent every build through the count and fill walks
+// as well: the long list of 3x10^4 particles spread evenly over four decades of
+// radius took 1581 us, now 311 (8 lanes per walk, before: 931).  The larger stack
+// for all walks costs waves: 576 entries took the lists of 10^6 particles from
+// 3.21 to 3.47 ms.
+constexpr int kRoomStack = 384;    // entries
+constexpr int kDeepStack = 2048;
+constexpr int kDeepLoose = kDeepStack - (7 * kMaxLevel + 1);
+constexpr int kFlagStack = 1, kFlagRoom = 2, kFlagNodes = 4, kFlagDeep = 8;   // bits of err
 constexpr int kRoomCand = 512;
 constexpr int kRoomBatch = 256;    // candidates tested together
 constexpr int kRoomTake = 32;      // finished entries on top that are worth taking before the next nodes are opened
 
-template <int MODE>
+template <int MODE, bool DEEP>
 __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const double *__restrict__ wb,
                                                        const double *__restrict__ r, double inv_t2,
                                                        int64_t *__restrict__ cnt, int32_t *__restrict__ out,
@@ -1016,12 +1033,13 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
                                                        int *__restrict__ err)
 {
 #pragma clang fp contract(off)
-    __shared__ uint2 stk[kRoomStack];
+    __shared__ uint2 stk[DEEP ? kDeepStack : kRoomStack];
     __shared__ int32_t cand[MODE == 2 ? 1 : kRoomCand];
     __shared__ uint32_t s_first[8], s_count[8], s_place[8];
     extern __shared__ double4 si[];
     if ((int)blockIdx.x >= ng) return;
     const int g = xcd_chunk(blockIdx.x, ng), lane = threadIdx.x;
+    if (DEEP && cnt[g] >= 0) return;
     const uint64_t below = (1ull << lane) - 1ull;
     const size_t C = t.mo.cap;
     const int ib = t.i_off[g], ni = t.i_off[g + 1] - ib;
@@ -1122,14 +1140,14 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
         if (lane == 0) stk[0] = e;
         sp = __builtin_amdgcn_readfirstlane(e.y) != 0u ? 1 : 0;
     }
-    bool bad = false;
+    bool bad = false, tight = false;   // tight: depth first
     while (sp > 0) {
         __syncthreads();   // the entries of the last step are written
         const int W = sp < 64 ? sp : 64;
         const uint2 e = lane < W ? stk[sp - 1 - lane] : make_uint2(0u, 0u);
         const uint64_t ob = __ballot((e.y & kTyMask) == kTyOpen);
         const int P = ob ? __builtin_ctzll(ob) : W;    // finished entries on top
-        if (!ob || P >= kRoomTake) {
+        if (!ob || P >= (tight ? 1 : kRoomTake)) {
             const int sz = lane < P && (e.y & kTyMask) == kTyLeaf ? (int)(e.y & kCountMask) : 0;
             if (MODE == 2) {
                 const uint64_t sb = __ballot(lane < P && (e.y & kTyMask) == kTySpj);
@@ -1169,7 +1187,7 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
         }
         // open the first (at most 8) nodes of the window
         const int rank = __popcll(ob & below);
-        const bool sel = ((ob >> lane) & 1) && rank < 8;
+        const bool sel = ((ob >> lane) & 1) && rank < (tight ? 1 : 8);
         const uint64_t sb = __ballot(sel);
         const int n_open = __popcll(sb), last = 63 - __builtin_clzll(sb);
         if (sel) {
@@ -1187,7 +1205,11 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
         }
         const uint64_t km = __ballot(w.y != 0u);
         const int T = last + 1 - n_open + __popcll(km), base = sp - 1 - last;
-        if (base + T > kRoomStack) {
+        if (DEEP && !tight && base + T > kDeepLoose) {
+            tight = true;
+            continue;
+        }
+        if (base + T > (DEEP ? kDeepStack : kRoomStack)) {
             bad = true;
             break;
         }
@@ -1198,14 +1220,22 @@ __global__ __launch_bounds__(64) void room_list_kernel(int ng, TreeView t, const
         }
         if (w.y != 0u) stk[base + T - 1 - (place - k + __popcll(km & below))] = w;
         sp = base + T;
+        if (DEEP) tight = tight && sp > kDeepLoose - 64;
+    }
+    if (bad) {   // DEEP: not in a sound tree
+        if (lane == 0) {
+            cnt[g] = -1;
+            if (MODE == 2) cnt_s[g] = 0;
+            atomicOr(err, DEEP ? kFlagStack : kFlagDeep);
+        }
+        return;
     }
     if (MODE != 2) drain(true);
     if (lane == 0) {
-        cnt[g] = count < room ? count : room;   // what the room holds (all of it unless err bit 2)
+        cnt[g] = count < room ? count : room;   // what the room holds (all of it unless err says so)
         if (MODE == 2) cnt_s[g] = spj < room_s ? spj : room_s;
-        if (bad) atomicOr(err, 1);
-        if (count > room) atomicOr(err, 2);
-        if (MODE == 2 && spj > room_s) atomicOr(err, 4);
+        if (count > room) atomicOr(err, kFlagRoom);
+        if (MODE == 2 && spj > room_s) atomicOr(err, kFlagNodes);
     }
 }
 
@@ -1346,6 +1376,7 @@ struct sphk_dtree : sphk::NodeBuffers<HipAlloc, BoxRec, MacRec> {
     // overflowed them
     int64_t room[2] = {kRoomNearStart, kRoomNearStart};
     int64_t room_long[2] = {kRoomLongStart, kRoomStart};
+    bool deep[3] = {false, false, false};   // whether a kind's last build had walks for the deep kernel
 
     // holds no tree and no lists
     void forget()
@@ -1444,6 +1475,31 @@ int walk_offsets(sphk_dtree *t, int ng, const int64_t *a, int64_t *c, int32_t *o
     return SPHK_OK;
 }
 
+// The walks of a list into their rooms, and the walk offsets: walks(false_type)
+// queues the kernel for all of them, walks(true_type) the deep one.  A kind
+// that had deep walks in its last build has both queued at once; else the deep
+// kernel, the offsets and their read follow when the flags ask for them.
+// flags: what is left for the counted build, 0 if the list is whole.
+template <class Walks, class Offsets>
+int room_walks(sphk_dtree *t, int kind, Walks &&walks, Offsets &&offsets, int64_t (&tot)[2], int &flags)
+{
+    const bool known = t->deep[kind];
+    bool both = known;
+    walks(std::false_type{});
+    if (both) walks(std::true_type{});
+    for (;;) {
+        SPHK_TRY(hipGetLastError());
+        if (int rc = offsets()) return rc;
+        if (int rc = read_totals(t, tot, flags)) return rc;
+        if (flags != kFlagDeep || both) break;
+        t->deep[kind] = both = true;
+        walks(std::true_type{});
+    }
+    if (known) t->deep[kind] = (flags & kFlagDeep) != 0;
+    if (both) flags &= ~kFlagDeep;
+    return SPHK_OK;
+}
+
 // A list still in the rooms of the scratch: packed to its offsets, into the
 // caller's arrays (j_idx / s_idx non-NULL; the list stays in the rooms) or
 // into the handle's own (the list leaves the rooms).
@@ -1472,8 +1528,8 @@ int pack_list(sphk_dtree *t, int kind, int32_t *j_idx, int32_t *s_idx)
     return SPHK_OK;
 }
 
-// Interaction lists of every walk: one pass into rooms, and if a room or a
-// stack overflowed the counted build.  That is, for the long list, the tree
+// Interaction lists of every walk: one pass into rooms, and if a room
+// overflowed (or does not fit in memory) the counted build.  That is, for the long list, the tree
 // walk run as count, scan and fill; for the short-range lists (gather: r =
 // rs, symmetry: r = H) the tree walk (count, scan, fill) writes the particles
 // of the leaves reached into the walk's stretch of a scratch array,
@@ -1509,22 +1565,24 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
     const dim3 lg((unsigned)((ng + kListWalks - 1) / kListWalks)), lb(64);
     if constexpr (MODE != 2) {
         // one pass into a room per walk: no count walk, one host read.  If a
-        // walk overflows its room or the stack, the counted build below runs
-        // instead (and later builds get twice the room), and so it does where
-        // the rooms do not fit in memory.
+        // walk overflows its room, the counted build below runs instead (and
+        // later builds get twice the room), and so it does where the rooms do
+        // not fit in memory.
         int64_t &room = t->room[MODE];
         const int at = (int64_t)ng * room <= kRoomMaxEntries
                            ? t->rooms.take(MODE, (size_t)ng * (size_t)room, 0, t->st, pack, rc_rooms)
                            : -1;
         if (rc_rooms) return rc_rooms;
         if (at >= 0) {
-            hipLaunchKernelGGL((room_list_kernel<MODE>), dim3(ng), dim3(64), n_si * sizeof(double4), t->st, ng, v, wb,
-                               r, 0., t->i64b.p, t->rooms.of[at].p, room, nullptr, nullptr, 0, n_si, t->err);
-            SPHK_TRY(hipGetLastError());
-            if (int rc = walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr)) return rc;
+            auto walks = [&](auto deep) {
+                hipLaunchKernelGGL((room_list_kernel<MODE, decltype(deep)::value>), dim3(ng), dim3(64),
+                                   n_si * sizeof(double4), t->st, ng, v, wb, r, 0., t->i64b.p, t->rooms.of[at].p, room,
+                                   nullptr, nullptr, 0, n_si, t->err);
+            };
+            auto offsets = [&]() { return walk_offsets(t, ng, t->i64b.p, t->i64d.p, L.j_off.p, nullptr, nullptr, nullptr); };
             int64_t tot1[2] = {0, 0};
             int flags = 0;
-            if (int rc = read_totals(t, tot1, flags)) return rc;
+            if (int rc = room_walks(t, MODE, walks, offsets, tot1, flags)) return rc;
             if (flags == 0) {
                 if (tot1[0] > std::numeric_limits<int32_t>::max())
                     return set_error(SPHK_E_CAPACITY, "dtree: list longer than 2^31 entries");
@@ -1537,28 +1595,31 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
                 L.built = true;
                 return SPHK_OK;
             }
-            if (flags & 2) room = std::min<int64_t>(room * 2, kRoomMax);
+            if (flags & kFlagRoom) room = std::min<int64_t>(room * 2, kRoomMax);
         }
     }
     if constexpr (MODE == 2) {
         // one walk into rooms per walk (EPJ and SPJ), then the entries packed
         // to the walk offsets: no count walk, one host read.  The counted
-        // build below if a walk overflows a room or the small stack (and later
-        // builds get twice the room that overflowed).
+        // build below if a walk overflows a room (and later builds get twice
+        // the room that overflowed).
         int64_t &rj = t->room_long[0], &rsp = t->room_long[1];
         const int at = (int64_t)ng * rj <= kRoomMaxEntries && (int64_t)ng * rsp <= kRoomMaxEntries
                            ? t->rooms.take(MODE, (size_t)ng * (size_t)rj, (size_t)ng * (size_t)rsp, t->st, pack, rc_rooms)
                            : -1;
         if (rc_rooms) return rc_rooms;
         if (at >= 0) {
-            hipLaunchKernelGGL((room_list_kernel<2>), dim3(ng), dim3(64), 0, t->st, ng, v, wb, r, inv_t2, t->i64a.p,
-                               t->rooms.of[at].p, rj, t->i64b.p, t->rooms.nodes.p, rsp, 0, t->err);
-            SPHK_TRY(hipGetLastError());
-            if (int rc = walk_offsets(t, ng, t->i64a.p, t->i64c.p, L.j_off.p, t->i64b.p, t->i64d.p, L.s_off.p))
-                return rc;
+            auto walks = [&](auto deep) {
+                hipLaunchKernelGGL((room_list_kernel<2, decltype(deep)::value>), dim3(ng), dim3(64), 0, t->st, ng, v, wb,
+                                   r, inv_t2, t->i64a.p, t->rooms.of[at].p, rj, t->i64b.p, t->rooms.nodes.p, rsp, 0,
+                                   t->err);
+            };
+            auto offsets = [&]() {
+                return walk_offsets(t, ng, t->i64a.p, t->i64c.p, L.j_off.p, t->i64b.p, t->i64d.p, L.s_off.p);
+            };
             int64_t tot1[2] = {0, 0};
             int flags = 0;
-            if (int rc = read_totals(t, tot1, flags)) return rc;
+            if (int rc = room_walks(t, MODE, walks, offsets, tot1, flags)) return rc;
             if (flags == 0) {
                 if (tot1[0] > std::numeric_limits<int32_t>::max() || tot1[1] > std::numeric_limits<int32_t>::max())
                     return set_error(SPHK_E_CAPACITY, "dtree: list longer than 2^31 entries");
@@ -1571,8 +1632,8 @@ int build_list(sphk_dtree *t, const double *r, double inv_t2)
                 L.built = true;
                 return SPHK_OK;
             }
-            if (flags & 2) rj = std::min<int64_t>(rj * 2, kRoomMax);
-            if (flags & 4) rsp = std::min<int64_t>(rsp * 2, kRoomMax);
+            if (flags & kFlagRoom) rj = std::min<int64_t>(rj * 2, kRoomMax);
+            if (flags & kFlagNodes) rsp = std::min<int64_t>(rsp * 2, kRoomMax);
         }
     }
     // count walk with the small stack, and with the worst-case one if a walk overflowed it

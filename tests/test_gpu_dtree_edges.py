@@ -80,3 +80,32 @@ def test_offsets_of_one_particle_walks(n):
 def test_large_leaves_equal_host(kind, n, n_leaf, n_group):
     """Leaves beyond the windows held in LDS, up to more than there are particles."""
     test_tree_equals_host(kind, n, n_leaf, n_group)
+
+
+@pytest.mark.parametrize("n,n_leaf,n_group,theta", [(30000, 8, 16, 0.5), (30000, 8, 64, 1.0), (6000, 1, 8, 0.3)])
+def test_steep_profile_equals_host(n, n_leaf, n_group, theta):
+    """Particles spread evenly over four decades of radius: walks at the edge
+    hold the whole centre in their search boxes and keep more entries pending
+    than the first stack holds.  Built three times: such walks are met, known
+    and (with a list that has none between) forgotten again."""
+    rng = np.random.default_rng(n + n_group)
+    x, y, z = rng.standard_normal((3, n)) * 10.0 ** rng.uniform(-4.0, 0.0, n)
+    perm = morton_order(x, y, z)
+    x, y, z = (np.ascontiguousarray(a[perm]) for a in (x, y, z))
+    m, eps2 = rng.uniform(0.5, 1.5, n), np.full(n, 1e-8)
+    h = 0.2 * np.sqrt(x * x + y * y + z * z)
+    d = lambda a: torch.from_numpy(a).cuda()   # noqa: E731
+    ht = HostTree(x, y, z, m, eps2, n_leaf, n_group)
+    dt = DeviceTree(*map(d, (x, y, z, m, eps2)), n_leaf, n_group)
+    try:
+        want = (ht.gather(h), ht.symmetry(h), ht.long(theta))
+        for again in range(3):
+            for name, hl, dl in zip(("gather", "symmetry", "long"), want,
+                                    (dt.gather(d(h)), dt.symmetry(d(h)), dt.long(theta))):
+                for a, b in zip(hl, dl):
+                    assert np.array_equal(a, b.cpu().numpy()), (name, again)
+            for a, b in zip(ht.long(3.0), dt.long(3.0)):
+                assert np.array_equal(a, b.cpu().numpy()), again
+    finally:
+        ht.close()
+        dt.close()
